@@ -190,6 +190,11 @@ void launch_resample(const Filters& fs, int mode, bool have_prefix, hipStream_t 
 // out[4i .. 4i+3] = mean of filter i
 void launch_gather_means(const Filters& fs, float* out, hipStream_t s);
 void launch_zero_u32(uint32_t* p, uint32_t n, hipStream_t s);
+// Whether a single filter of n particles gains from a visiting order: the
+// smallest filters' workgroups hold four particles each, which gather few
+// common lines in any order (2,000 particles: 2 to 7 us of the weight kernel,
+// less than the sort).
+bool order_pays(uint32_t n);
 // Visiting order of f's particles for the cloud weight, into o.order.
 void launch_order(const FilterDev& f, const OrderDev& o, hipStream_t s);
 // The same for count filters at once (device arrays fs[i], os[i]; max_n the

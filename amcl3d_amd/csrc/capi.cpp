@@ -797,7 +797,7 @@ int a3d_pf_update_dev(a3d_pf* p, const a3d_grid* g, const float* d_x, const floa
   f.roll = (float)roll;  // double -> float parameter of computeCloudWeight
   f.pitch = (float)pitch;
   f.rp0 = (f.roll == 0.0f && f.pitch == 0.0f) ? 1u : 0u;
-  if (g_order == A3D_ORDER_SPATIAL) {
+  if (g_order == A3D_ORDER_SPATIAL && order_pays(p->n)) {
     const OrderDev o = order_view(p->ord, p->n);
     launch_order(f, o, p->stream);
     f.order = o.order;

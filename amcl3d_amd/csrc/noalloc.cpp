@@ -94,7 +94,7 @@ extern "C" int a3d_pf_update_noalloc(const a3d_grid* g, float* d_particles, size
   f.roll = (float)roll;  // double -> float parameter of computeCloudWeight
   f.pitch = (float)pitch;
   f.rp0 = (f.roll == 0.0f && f.pitch == 0.0f) ? 1u : 0u;
-  if (current_order() == A3D_ORDER_SPATIAL) {
+  if (current_order() == A3D_ORDER_SPATIAL && order_pays(N)) {
     const OrderDev o = order_view(base + kSumsBytes + kInmapBytes, N);
     launch_order(f, o, s);
     f.order = o.order;

@@ -829,6 +829,231 @@ __global__ __launch_bounds__(kBlockThreads) void lanes_poses_kernel(GridDev g, F
   weight_lanes<Q, IK, false, CLEAN, true>(g, f, p0, count, out, cloud, chunk);
 }
 
+// ---------------------------------------------------------------------------
+// The split form of mapping 0, for launches with too few particles to fill
+// the chip with whole-cloud wavefronts.  A workgroup holds P particles; its W
+// evaluating wavefronts share the cloud out between them (P particles x Q =
+// 64/P points per step, U steps per tile and wavefront) and leave the gathered
+// values in an LDS tile, one row per particle; one more wavefront adds every
+// row in point order, lane = particle, so a sum is the reference's sequential
+// float sum.  Tiles are double buffered and everything runs ahead of the sum:
+// in iteration t the evaluating wavefronts compute tile t's cells, write tile
+// t-1's values and issue tile t's gathers, while the adding wavefront adds
+// tile t-2.  Points past the cloud's end are NaN (rejected: +0, which leaves a
+// sum unchanged), so no remainder loop is needed.
+template <int P, int W>
+struct Split {
+  static constexpr int Q = 64 / P;       // points per wavefront step
+  static constexpr int U = 4;            // steps per wavefront and tile
+  static constexpr int T = U * W * Q;    // points per tile
+  static constexpr int kRow = T + 4;     // floats per row of a value tile
+  static constexpr int kThreads = 64 * (W + 1);
+};
+
+template <int P, int W, bool RP0, int IK, int MODE>
+__device__ __forceinline__ void split_eval(const GridDev& g, const FilterDev& f, const LanePose& lp, int& cnt,
+                                           float* tiles, uint32_t segk) {
+  using S = Split<P, W>;
+  using Idx = typename ProbSrc<IK>::Idx;
+  constexpr int Q = S::Q, U = S::U, T = S::T;
+  const ProbSrc<IK> src(g, segk);
+  const int lane = lane_id();
+  const uint32_t w = threadIdx.x >> 6;
+  const uint32_t m = f.m, ntiles = (m + T - 1) / T;
+  const uint32_t first = w * Q + (uint32_t)(lane % Q);  // this lane's point of step 0
+  float* const row = tiles + (lane / Q) * S::kRow + first;
+  float pend[U];
+  struct Pts {
+    float x[U], y[U], z[U];
+  };
+  auto load = [&](uint32_t t, Pts& p) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t j = t * T + (uint32_t)u * (W * Q) + first;
+      const bool in = j < m;
+      const uint32_t js = in ? j : m - 1;
+      p.x[u] = in ? f.cx[js] : __builtin_nanf("");
+      p.y[u] = f.cy[js];
+      p.z[u] = f.cz[js];
+    }
+  };
+  auto put = [&](uint32_t t) {
+    float* const r = row + (t & 1u) * (P * S::kRow);
+#pragma unroll
+    for (int u = 0; u < U; ++u) r[u * (W * Q)] = pend[u];
+  };
+  auto tile = [&](uint32_t t, const Pts& cur, Pts& nxt) {
+    if (t + 1 < ntiles) load(t + 1, nxt);
+    Idx idx[U];
+    bool nr[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      uint64_t vm;
+      idx[u] = cell_fast<RP0, IK, MODE>(g, src, lp, stage_point<RP0>(cur.x[u], cur.y[u], cur.z[u]), vm, nr[u]);
+      cnt = add_mask_bit(cnt, vm);
+    }
+    if constexpr (MODE == kWindow) {
+      bool any = false;
+#pragma unroll
+      for (int u = 0; u < U; ++u) any |= nr[u];
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(any) != 0, 0)) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (nr[u]) {
+            bool ve;
+            const Idx ie = cell_exact<RP0, IK>(g, src, lp, stage_point<RP0>(cur.x[u], cur.y[u], cur.z[u]), ve);
+            cnt += (ve ? 1 : 0) - (idx[u] != src.zero ? 1 : 0);
+            idx[u] = ie;
+          }
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);  // the cells come before the wait on the previous gathers
+    if (t > 0) put(t - 1);
+#pragma unroll
+    for (int u = 0; u < U; ++u) pend[u] = src(idx[u]);
+    __syncthreads();
+  };
+  Pts a, b;
+  load(0, a);
+  for (uint32_t t = 0; t < ntiles; t += 2) {
+    tile(t, a, b);
+    if (t + 1 < ntiles) tile(t + 1, b, a);
+  }
+  put(ntiles - 1);
+}
+
+// Adds one tile's first `len` values (rounded up to the block of 32) of this
+// lane's row, in order.
+template <int T>
+__device__ __forceinline__ void split_add(const float* row, uint32_t len, float& wsum) {
+  constexpr int B = 8;  // float4 per block
+  const float4* r = reinterpret_cast<const float4*>(row);
+  const int blocks = (int)((len + 4 * B - 1) / (4 * B));
+  float4 a[B], b[B];
+  auto rd = [&](int k, float4 (&v)[B]) {
+#pragma unroll
+    for (int i = 0; i < B; ++i) v[i] = r[k * B + i];
+  };
+  auto add = [&](const float4 (&v)[B]) {
+#pragma unroll
+    for (int i = 0; i < B; ++i) {
+      wsum += v[i].x;
+      wsum += v[i].y;
+      wsum += v[i].z;
+      wsum += v[i].w;
+    }
+  };
+  rd(0, a);
+  for (int k = 0; k < blocks; k += 2) {
+    if (k + 1 < blocks) rd(k + 1, b);
+    add(a);
+    if (k + 1 < blocks) {
+      if (k + 2 < blocks) rd(k + 2, a);
+      add(b);
+    }
+  }
+}
+
+template <int P, int W, int IK, bool CLEAN>
+__device__ __forceinline__ void split_variant(const GridDev& g, const FilterDev& f, const LanePose& lp, int& cnt,
+                                              float* tiles, uint32_t segk) {
+  if constexpr (CLEAN) {
+    const bool zero = __builtin_amdgcn_ballot_w64(lp.slow) != 0;
+    if (f.rp0) {
+      if (zero)
+        split_eval<P, W, true, IK, kCleanZero>(g, f, lp, cnt, tiles, segk);
+      else
+        split_eval<P, W, true, IK, kClean>(g, f, lp, cnt, tiles, segk);
+    } else {
+      if (zero)
+        split_eval<P, W, false, IK, kCleanZero>(g, f, lp, cnt, tiles, segk);
+      else
+        split_eval<P, W, false, IK, kClean>(g, f, lp, cnt, tiles, segk);
+    }
+  } else {
+    if (f.rp0)
+      split_eval<P, W, true, IK, kWindow>(g, f, lp, cnt, tiles, segk);
+    else
+      split_eval<P, W, false, IK, kWindow>(g, f, lp, cnt, tiles, segk);
+  }
+}
+
+template <int P, int W, int IK, bool KFILTER, bool CLEAN>
+__global__ __launch_bounds__((Split<P, W>::kThreads)) void lanes_split_kernel(GridDev g, FilterDev f, float* out) {
+  using S = Split<P, W>;
+  constexpr int Q = S::Q;
+  __shared__ float4 tiles4[2 * P * S::kRow / 4];
+  __shared__ int counts[W * P];
+  float* const tiles = reinterpret_cast<float*>(tiles4);
+  const uint32_t wave = threadIdx.x >> 6;
+  const int lane = lane_id();
+  const bool adds = wave == W;  // the adding wavefront
+  const uint32_t p0 = xcd_block(blockIdx.x, gridDim.x) * P;
+  const uint32_t count = min((uint32_t)P, f.n - p0);  // the grid has ceil(n / P) workgroups
+  const int ps = adds ? lane % P : lane / Q;
+  const bool has = (uint32_t)ps < count;
+  const uint32_t pk = p0 + (has ? (uint32_t)ps : 0u);
+  const uint32_t pi = f.order ? f.order[pk] : pk;
+  const float tx = f.x[pi], ty = f.y[pi], tz = f.z[pi];
+  const bool act = KFILTER ? (has && into_map(g, tx, ty, tz)) : has;
+  if (__ballot(act) == 0) return;  // the same particles in every wavefront: uniform over the workgroup
+  const uint32_t m = f.m, ntiles = (m + S::T - 1) / S::T;
+  if (adds) {
+    float wr = 0.f;
+    if (KFILTER && act && lane < P) wr = range_weight(tx, ty, tz, f.ranges, f.nb, f.sigma);
+    float wsum = 0.f;
+    const float* const row = tiles + ps * S::kRow;
+    auto add = [&](uint32_t t) {
+      split_add<S::T>(row + (t & 1u) * (P * S::kRow), min((uint32_t)S::T, m - t * S::T), wsum);
+    };
+    for (uint32_t t = 0; t < ntiles; ++t) {
+      if (t >= 2) add(t - 2);
+      __syncthreads();
+    }
+    if (ntiles >= 2) add(ntiles - 2);
+    __syncthreads();
+    if (ntiles >= 1) add(ntiles - 1);
+    if (act && lane < P) {
+      int c = 0;
+#pragma unroll
+      for (int w = 0; w < W; ++w) c += counts[w * P + lane];
+      const float wp = (c <= 10) ? 0.f : wsum / (float)c;
+      if (KFILTER) {
+        f.wp[pi] = wp;
+        f.wr[pi] = wr;
+      } else {
+        out[pi] = wp;
+      }
+    }
+    return;
+  }
+  LanePose lp;
+  rotation9(f.roll, f.pitch, f.a[pi], lp.r);
+  const double nan = __builtin_nan("");
+  lp.ox = act ? (double)tx - g.min[0] : nan;
+  lp.oy = act ? (double)ty - g.min[1] : nan;
+  lp.oz = act ? (double)tz - g.min[2] : nan;
+  constexpr double kTiny = 0x1p-96;
+  lp.slow = fabs(lp.ox) < kTiny || fabs(lp.oy) < kTiny || fabs(lp.oz) < kTiny;
+  int cnt = 0;
+  if (ntiles > 0) {
+    if constexpr (IK != kIdxBuf) {
+      uint32_t segk = 0;
+      if (g.seg_bits && f.zr && wave_segment(g, f, act, lp.oz, &segk))
+        split_variant<P, W, kIdxSeg, CLEAN>(g, f, lp, cnt, tiles, segk);
+      else
+        split_variant<P, W, IK, CLEAN>(g, f, lp, cnt, tiles, 0u);
+    } else {
+      split_variant<P, W, IK, CLEAN>(g, f, lp, cnt, tiles, 0u);
+    }
+  }
+#pragma unroll
+  for (int q = 1; q < Q; q <<= 1) cnt += __shfl_xor(cnt, q);
+  if (lane % Q == 0) counts[wave * P + ps] = cnt;
+  __syncthreads();
+}
+
 // One work item of up to kBlockWaves * P particles of one filter, taken by
 // a whole workgroup: wavefront w holds particles p0 + w*P .. and the
 // wavefronts walk the filter's cloud together.  A filter that names its own
@@ -1034,6 +1259,43 @@ void lanes_poses_q(const GridDev& g, const FilterDev& f, float* out, uint32_t ch
 #undef A3D_LAUNCH
 }
 
+// The grids wider than a buffer share the 64-bit kernel (it reads every grid,
+// and takes segment loads like the 32-bit kind).
+template <int P, int W, bool KFILTER>
+void split_pw(const GridDev& g, const FilterDev& f, float* out, hipStream_t s) {
+  const dim3 b((f.n + P - 1) / P), t(Split<P, W>::kThreads);
+  if (index_kind(g) == kIdxBuf) {
+    if (g.clean) lanes_split_kernel<P, W, kIdxBuf, KFILTER, true><<<b, t, 0, s>>>(g, f, out);
+    else lanes_split_kernel<P, W, kIdxBuf, KFILTER, false><<<b, t, 0, s>>>(g, f, out);
+  } else {
+    if (g.clean) lanes_split_kernel<P, W, kIdx64, KFILTER, true><<<b, t, 0, s>>>(g, f, out);
+    else lanes_split_kernel<P, W, kIdx64, KFILTER, false><<<b, t, 0, s>>>(g, f, out);
+  }
+}
+
+// Launches of up to kSplitMax particles take the split form.  Weight kernel
+// alone, whole-cloud wavefronts of 16 against the split form at the chosen P
+// (us; particles x points, map, spread):
+//   600 x 2,000 room, 0.1 m                   62 -> 17 (P = 4; 18 at 8, 24 at 16)
+//   300 x 20,000 floor, 0.1 m                632 -> 92 (P = 4; 110, 196)
+//   2,000 x 4,000 floor, tilted, 0.5 m       171 -> 41 (P = 4; 45, 70)
+//   5,000 x 6,000 floor, tilted, 0.1 m       213 -> 76 (P = 8; 95 at 4, 94 at 16)
+//   20,011 x 7,993 floor, tilted, 0.5 m      385 -> 350 (P = 16)
+//   40,000 x 8,000 floor, 0.5 m              516, split 711: enough whole-cloud
+//   wavefronts, which share more lines per workgroup (64 particles)
+// Small P is bound by the adding wavefront (one dependent add per point, 4.6
+// ns), larger P by the gathers.
+constexpr uint32_t kSplit4Max = 2048, kSplit8Max = 8192, kSplitMax = 28672;
+
+template <bool KFILTER>
+bool launch_split(const GridDev& g, const FilterDev& f, float* out, hipStream_t s) {
+  if (f.n > kSplitMax) return false;
+  if (f.n <= kSplit4Max) split_pw<4, 4, KFILTER>(g, f, out, s);
+  else if (f.n <= kSplit8Max) split_pw<8, 4, KFILTER>(g, f, out, s);
+  else split_pw<16, 4, KFILTER>(g, f, out, s);
+  return true;
+}
+
 template <int Q>
 int fleet_blocks_per_cu(int v) {
   int per_cu = 1;
@@ -1107,6 +1369,8 @@ int clamp_chunk(int points) {
   return kMaxChunk;
 }
 
+bool order_pays(uint32_t n) { return current_mapping() != 0 || n > kSplit4Max; }
+
 void launch_weight(const GridDev& g, const Filters& fs, const WorkItem* d_items, uint32_t nitems,
                    uint32_t* d_counter, int ppw, int persistent, hipStream_t s) {
   ppw = clamp_ppw(ppw);
@@ -1119,6 +1383,7 @@ void launch_weight(const GridDev& g, const Filters& fs, const WorkItem* d_items,
         cloud_zrange_kernel<<<dim3(kZrParts, std::min(fs.count - base, 65535u)), kZrThreads, 0, s>>>(fs, base);
     if (!fs.arr) {
       if (fs.one.n == 0) return;
+      if (launch_split<true>(g, fs.one, nullptr, s)) return;
       if (ppw == 64) lanes_single_q<1>(g, fs.one, chunk, s);
       else if (ppw == 32) lanes_single_q<2>(g, fs.one, chunk, s);
       else lanes_single_q<4>(g, fs.one, chunk, s);
@@ -1165,6 +1430,7 @@ void launch_weight_poses(const GridDev& g, const float* cx, const float* cy, con
   if (current_mapping() == 0) {
     const uint32_t chunk = (uint32_t)clamp_chunk(current_chunk());
     if (index_kind(g) != kIdxBuf && g.seg_bits) cloud_zrange_kernel<<<dim3(kZrParts, 1), kZrThreads, 0, s>>>(single(f), 0u);
+    if (launch_split<false>(g, f, out, s)) return;
     if (ppw == 64) lanes_poses_q<1>(g, f, out, chunk, s);
     else if (ppw == 32) lanes_poses_q<2>(g, f, out, chunk, s);
     else lanes_poses_q<4>(g, f, out, chunk, s);

@@ -1,0 +1,69 @@
+"""The split form of the cloud weight (a workgroup's wavefronts share the cloud,
+one more adds the values in order) at the sizes
+where its tiles, workgroups and dispatch limits end: bit-exact against
+the oracle."""
+import numpy as np
+import pytest
+
+import oracle
+from amcl3d_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def room():
+    c = W.room_case(1)
+    bm = c["map"]
+    pts = bm.points()
+    _, prob = oracle.compute_grid(pts, bm.min, bm.max, bm.res, c["sensor_dev"], exp_mode=1)
+    c.update(points=pts, ogrid=oracle.GridMeta(bm.min, bm.max, bm.res, prob))
+    return c
+
+
+def _open(gpu, room):
+    g = gpu.Grid3d()
+    bm = room["map"]
+    g.open(room["points"], bm.min, bm.max, bm.res, room["sensor_dev"])
+    return g
+
+
+def _poses(room, n, seed=5):
+    rng = np.random.default_rng(seed)
+    base = room["particles"][rng.integers(0, len(room["particles"]), n)]
+    t = base[:, :4] + rng.normal(0, 0.2, (n, 4)).astype(np.float32)
+    if n > 8:
+        t[n // 3, :3] = 1e4  # outside the map
+        t[n // 2, :3] = room["map"].min  # zero offsets
+    return np.ascontiguousarray(t, np.float32)
+
+
+# workgroups of 4, 8 and 16 poses, their last one ragged, and one past the split form
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 2048, 2049, 8192, 8195, 28672, 28673])
+def test_poses_at_dispatch_limits(gpu, room, n):
+    g, t = _open(gpu, room), _poses(room, n)
+    cloud = room["step"].cloud[:300]
+    for roll, pitch in ((0.0, 0.0), (0.05, -0.03)):
+        w = g.cloud_weights(cloud, t[:, 0], t[:, 1], t[:, 2], t[:, 3], roll, pitch)
+        ow = oracle.cloud_weight_batch(room["ogrid"], cloud, t[:, 0], t[:, 1], t[:, 2], t[:, 3], roll, pitch)
+        assert np.array_equal(w.view(np.int32), ow.view(np.int32)), (n, roll)
+
+
+# kernels of every index kind and cell mode; clouds of 0 points, below and
+# around one tile (256, 128 and 64 points), two and several tiles
+@pytest.mark.parametrize("env", [None, ("A3D_FORCE_IDX64", "1"), ("A3D_FORCE_IDX64", "2"), ("A3D_FORCE_IDX32", "2"),
+                                 ("A3D_FORCE_NEAR_TEST", "1")], ids=str)
+@pytest.mark.parametrize("n", [37, 2083, 8205])
+def test_poses_at_tile_edges(gpu, room, env, n, monkeypatch):
+    if env:
+        monkeypatch.setenv(*env)
+    g, t = _open(gpu, room), _poses(room, n)
+    for m in (0, 1, 10, 11, 31, 33, 63, 64, 65, 127, 129, 255, 256, 257, 513, 800):
+        cloud = np.ascontiguousarray(room["step"].cloud[:m])
+        if m > 20:
+            cloud = cloud.copy()
+            cloud[m - 3] = np.nan
+            cloud[m // 2, 1] = np.inf
+        w = g.cloud_weights(cloud, t[:, 0], t[:, 1], t[:, 2], t[:, 3])
+        ow = oracle.cloud_weight_batch(room["ogrid"], cloud, t[:, 0], t[:, 1], t[:, 2], t[:, 3])
+        assert np.array_equal(w.view(np.int32), ow.view(np.int32)), (n, m)
