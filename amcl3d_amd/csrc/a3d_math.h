@@ -162,6 +162,23 @@ __device__ inline void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Inclusive float sums over the lanes of a wavefront (lane 63: the whole sum),
+// in the order of the DPP moves.
+__device__ __forceinline__ float wave_inclusive_sum(float v) {
+#define A3D_DPP_ADD(ctrl, rows) \
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, rows, 0xf, true))
+  A3D_DPP_ADD(0x111, 0xf);  // row_shr 1, 2, 4, 8: lane l of a row holds the row's first l + 1 lanes
+  A3D_DPP_ADD(0x112, 0xf);
+  A3D_DPP_ADD(0x114, 0xf);
+  A3D_DPP_ADD(0x118, 0xf);
+  A3D_DPP_ADD(0x142, 0xa);  // row_bcast 15 into rows 1 and 3, 31 into rows 2 and 3
+  A3D_DPP_ADD(0x143, 0xc);
+#undef A3D_DPP_ADD
+  return v;
+}
+// Sum over the wavefront, in every lane.
+__device__ __forceinline__ float wave_sum(float v) { return readlane_f(wave_inclusive_sum(v), 63); }
+
 template <class F>
 __device__ inline const FilterDev& filter_at(const Filters& fs, uint32_t i) {
   return fs.arr ? fs.arr[i] : fs.one;

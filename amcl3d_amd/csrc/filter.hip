@@ -6,16 +6,17 @@
 //
 // The reference's sums over particles are sequential float sums in index
 // order (wtp, wtr, wt, the mean, resample's running sum c); resampling
-// depends on every bit of them, so they are computed as sequential chains:
-// chain_kernel runs one workgroup per filter in which lane k of wavefront 0
-// adds chain k while the other fifteen wavefronts stage the next block of
-// inputs through LDS.  Everything that does not depend on a chain runs in
-// grid-wide elementwise kernels (grid y = filter).
+// depends on every bit of them, so they are computed exactly, by one workgroup
+// per sum (exact_sum) or, for a large single filter, across the chip (the
+// tiled sums).  Everything else runs in grid-wide elementwise kernels (grid y
+// = filter), or, for filters of up to kTailOneMax particles, beside the sums
+// in one workgroup per filter.
 //
-// update:   tail_a  -> chain(wtp, wtr) -> tail_c -> chain(wt) -> tail_e
-//           -> chain(mean x, y, z, a) beside chain(resample's c)
-// resample: [chain(c) unless update just produced it] -> select -> commit
-// init:     init_a -> chain(wt) -> init_c -> chain(mean)
+// update:   tail_a  -> wtp, wtr -> tail_c -> wt -> tail_e
+//           -> mean x, y, z, a beside resample's c;  small: tail_one
+// resample: [c unless update just produced it] -> select -> commit;  small:
+//           resample_one
+// init:     init_a -> wt -> init_c -> chain(mean)
 #include "a3d_math.h"
 
 namespace a3d {
@@ -503,72 +504,6 @@ __device__ __forceinline__ float exact_sum_range(float s, uint32_t pos, uint32_t
   return s;
 }
 
-__device__ __forceinline__ float exact_sum(uint32_t n, const float* __restrict__ x, float* prefix, ExactLds& L) {
-  return exact_sum_range(0.0f, 0, n, n, x, prefix, L);
-}
-
-// Whether any of w[0..n) is negative or not finite: the running sum c is
-// then not monotone, and resample selects serially (the flag goes to
-// sums[4]).  Called by every thread of the workgroup.
-__device__ __forceinline__ float weights_irregular(uint32_t n, const float* w, ExactLds& L) {
-  uint32_t bad = 0;
-  for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) bad |= (w[i] < 0.0f || !isfinite(w[i])) ? 1u : 0u;
-  return block_min(bad ? 0u : 1u, L) == 0u ? 1.0f : 0.0f;
-}
-
-// wtp and wtr (grid row y = 0, 1), wt, or resample's c with its checkpoints,
-// by exact_sum: one workgroup per filter and sum.
-__global__ __launch_bounds__(kChainThreads) void exact_chain_kernel(Filters fs, int which) {
-  __shared__ ExactLds lds;
-  const FilterDev& f = fsel(fs, blockIdx.x);
-  if (which == kPrefixOnly && f.no_resample) return;
-  const uint32_t n = f.n;
-  float* sc = f.scratch;
-  const float* src;
-  float* dst;
-  float* prefix = nullptr;
-  if (which == kTailTotals) {
-    src = sc + (size_t)blockIdx.y * n;
-    dst = sums_of(f) + blockIdx.y;
-  } else if (which == kWeightTotal) {
-    src = f.w;
-    dst = sums_of(f) + 2;
-  } else {  // kPrefixOnly
-    src = f.w;
-    dst = sums_of(f) + 3;
-    prefix = sc + sc_c32(n);
-  }
-  const float v = exact_sum(n, src, prefix, lds);
-  const float irregular = prefix ? weights_irregular(n, src, lds) : 0.0f;
-  if (threadIdx.x == 0) {
-    *dst = v;
-    if (prefix) sums_of(f)[4] = irregular;
-  }
-}
-
-// The last sums of update, side by side: the four mean terms (grid rows
-// y = 0..3) and resample's running sum c over the new weights with its
-// checkpoints and the monotonicity flag (row 4).  The mean terms may have
-// either sign: exact_sum handles them exactly, restarting at every binade
-// crossing, and finishes serially if they cross too often.
-__global__ __launch_bounds__(kChainThreads) void mean_prefix_kernel(Filters fs) {
-  __shared__ ExactLds lds;
-  const FilterDev& f = fsel(fs, blockIdx.x);
-  const uint32_t n = f.n;
-  float* sc = f.scratch;
-  if (blockIdx.y < 4) {
-    const float v = exact_sum(n, sc + (size_t)blockIdx.y * n, nullptr, lds);
-    if (threadIdx.x == 0) f.mean[blockIdx.y] = v;
-  } else {
-    const float v = exact_sum(n, f.w, sc + sc_c32(n), lds);
-    const float irregular = weights_irregular(n, f.w, lds);
-    if (threadIdx.x == 0) {
-      sums_of(f)[3] = v;
-      sums_of(f)[4] = irregular;
-    }
-  }
-}
-
 // ------------------------------------------------------- tiled exact sums
 // A single large filter's sums, spread over the chip instead of one CU.  The
 // terms are cut into tiles of kTiledTile, each of 16 sub-tiles of 64 (one
@@ -596,7 +531,10 @@ __global__ __launch_bounds__(kChainThreads) void mean_prefix_kernel(Filters fs) 
 //         recorded at their start (the walk writes the others').
 // The guesses only decide which path a run of terms takes, never a bit of
 // the result: every sum is the sequential float sum exactly.
-constexpr uint32_t kTiledMin = 16384;  // particles from which a single filter's sums run tiled
+// Particles from which a single filter's sums run tiled: 20,011 particles take
+// 27 us per phase in one workgroup (three chunks), 36 us and one or two more
+// launches tiled; each further chunk of 8,192 adds about 8 us.
+constexpr uint32_t kTiledMin = 24576;
 constexpr uint32_t kWalkTiles = 1024;  // tile records the walk holds in LDS at a time
 constexpr uint32_t kSubTiles = kTiledTile / 64;
 static_assert(kSubTiles == 16, "a tile's sub-tiles fit one row of 16 lanes");
@@ -1047,6 +985,276 @@ __global__ __launch_bounds__(kChainThreads) void tiled_ckpt_kernel(Filters fs, i
   if (i < n && is_checkpoint(i, n)) prefix[i / kGroup] = (float)(s_in < 0.0f ? -v : v);
 }
 
+// ----------------------------------------- exact sums of a workgroup's chunk
+// The sums of smaller filters, in one workgroup, by the same maps with
+// sub-tiles of 64 terms only.  A chunk of up to kChainThreads * K terms of NS
+// sums: each wavefront guesses the binade each of its sub-tiles starts in from
+// float sums of the earlier terms and composes the sub-tile's maps under the
+// guess and the binade above (without exact ties, the usual case, a map is one
+// integer sum); then wavefront k walks sum k: runs of up to 64 sub-tiles whose
+// maps apply in one scan, any other sub-tile (a binade crossing, both signs,
+// an infinite sum) as 64 float adds in order from LDS.  Bound by the latency
+// of the walk: a scan and 64 dependent adds per binade crossing.  One sum of
+// 5,000 terms takes 12.6 us and of 20,000 terms 26 us, where tiles of 10,240
+// terms scanned again after each crossing (exact_sum_range) took 25 and 40 us.
+template <int NS, int K>
+struct ChunkLds {
+  static constexpr int kTerms = kChainThreads * K;
+  static constexpr int kSubs = kTerms / 64;
+  float x[NS][kTerms];
+  float part[NS][kSubs];
+  // a sub-tile's maps (SubRec's fields; fe = flags | pp << 8 | (e + 256) << 12)
+  uint32_t d0a[NS][kSubs], d1a[NS][kSubs], d0b[NS][kSubs], d1b[NS][kSubs], fe[NS][kSubs];
+  float s[NS];
+};
+
+// The map of one sub-tile (a wavefront's terms) from the scaled magnitudes r =
+// |x| / u: (d0, d1, pp) in every lane.
+__device__ __forceinline__ void subtile_map(float r, uint32_t& d0, uint32_t& d1, uint32_t& pp, bool& hard) {
+  const bool h = !(r < 0x1p24f);
+  hard = __ballot(h) != 0;
+  if (hard) {
+    d0 = d1 = pp = 0u;
+    return;
+  }
+  const float fr = __builtin_amdgcn_fractf(r);
+  if (__ballot(fr == 0.5f) == 0) {
+    uint32_t t = (uint32_t)rintf(r);
+#define A3D_DPP_ADD(ctrl, rows) t += dpp_u32<ctrl, rows>(0u, t)
+    A3D_DPP_ADD(0x111, 0xf);
+    A3D_DPP_ADD(0x112, 0xf);
+    A3D_DPP_ADD(0x114, 0xf);
+    A3D_DPP_ADD(0x118, 0xf);
+    A3D_DPP_ADD(0x142, 0xa);
+    A3D_DPP_ADD(0x143, 0xc);
+#undef A3D_DPP_ADD
+    d0 = d1 = (uint32_t)__builtin_amdgcn_readlane((int)t, 63);
+    pp = (d0 & 1u) | ((~d0 & 1u) << 1);
+    return;
+  }
+  const uint32_t q = (uint32_t)r;  // truncates: floor
+  ParityFn f;
+  if (fr == 0.5f) {
+    f = ParityFn{q + (q & 1u), q + ((q + 1u) & 1u), 0u, 0u};
+  } else {
+    const uint32_t t = q + (fr > 0.5f ? 1u : 0u);
+    f = ParityFn{t, t, t & 1u, (t + 1u) & 1u};
+  }
+  f = wave_inclusive_fn(f);
+  d0 = (uint32_t)__builtin_amdgcn_readlane((int)f.d0, 63);
+  d1 = (uint32_t)__builtin_amdgcn_readlane((int)f.d1, 63);
+  pp = (uint32_t)__builtin_amdgcn_readlane((int)(f.p0 | (f.p1 << 1)), 63);
+}
+
+// One wavefront adds the nq sub-tiles of a chunk to s in order; the running
+// sum after each goes to prefix[0 .. nq) (when given).
+template <class Lds>
+__device__ float chunk_walk(float s, uint32_t nq, int k, float* prefix, const Lds& L) {
+  const uint32_t lane = lane_id();
+  for (uint32_t q = 0; q < nq;) {
+    const uint32_t Q = q + lane;
+    const bool have = Q < nq;
+    const uint32_t fe = have ? L.fe[k][Q] : 0u, fl = fe & 0xffu;
+    if (s == 0.0f) {  // +0 plus sub-tiles of zeros stays +0
+      const uint32_t Z = first_false(have && !(fl & (kPos | kNeg | kIrregularTerm)));
+      if (prefix && lane < Z) prefix[Q] = 0.0f;
+      q += Z;
+      if (q == nq) break;
+    } else if (normal_finite(s)) {
+      const int E = float_exponent(fabsf(s)), e = (int)(fe >> 12) - 256;
+      const bool use_a = e == E && !(fl & kNoMapA), use_b = e + 1 == E && !(fl & kNoMapB);
+      const bool sign_ok = (s > 0.0f) ? !(fl & kNeg) : !(fl & kPos);
+      const uint32_t d0 = have ? (use_a ? L.d0a[k][Q] : L.d0b[k][Q]) : 0u;
+      const uint32_t d1 = have ? (use_a ? L.d1a[k][Q] : L.d1b[k][Q]) : 0u;
+      const uint32_t pp = use_a ? fe >> 8 : fe >> 10;
+      const bool valid = have && (use_a || use_b) && sign_ok && d0 < (1u << 24) && d1 < (1u << 24);
+      if (__ballot(valid) & 1ull) {
+        uint32_t kb, ka;
+        const uint32_t C = run_maps(s, E, ParityFn{d0, d1, pp & 1u, (pp >> 1) & 1u}, valid, kb, ka);
+        if (C > 0) {
+          const bool neg = s < 0.0f;
+          if (prefix && lane < C) prefix[Q] = from_k(ka, E, neg);
+          s = from_k((uint32_t)__builtin_amdgcn_readlane((int)ka, C - 1), E, neg);
+          q += C;
+          if (q == nq) break;
+          if (C == 64) continue;
+        }
+      }
+    }
+    // sub-tile q, which no map covers, by the reference's float adds: every
+    // lane reads the same terms (broadcasts); the zeros past the end leave
+    // the sum, never -0.0, unchanged
+    const float4* x = reinterpret_cast<const float4*>(L.x[k] + q * 64);
+    float4 v[16];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) v[c] = x[c];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+      s += v[c].x;
+      s += v[c].y;
+      s += v[c].z;
+      s += v[c].w;
+    }
+    if (prefix && lane == 0) prefix[q] = s;
+    ++q;
+  }
+  return s;
+}
+
+// s[k] + the chunk's len terms of sum k in order, for every k, in every thread.
+// xv[k][u]: this thread's term u * kChainThreads + tid of sum k (0 past len).
+// prefix (or null): the checkpoints of sum NS - 1 from the chunk's first on.
+template <int NS, int K>
+__device__ __forceinline__ void chunk_sums(float (&s)[NS], const float (&xv)[NS][K], uint32_t len, float* prefix,
+                                           ChunkLds<NS, K>& L) {
+  const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
+  constexpr uint32_t kW = kChainThreads / 64, kSubs = ChunkLds<NS, K>::kSubs;
+  const uint32_t nq = (len + 63) / 64;
+#pragma unroll
+  for (int k = 0; k < NS; ++k) {
+#pragma unroll
+    for (int u = 0; u < K; ++u) {
+      const uint32_t q = u * kW + wave;
+      if (q >= nq) continue;  // uniform over the wavefront
+      L.x[k][u * kChainThreads + tid] = xv[k][u];
+      const float w = wave_sum(xv[k][u]);
+      if (lane == 0) L.part[k][q] = w;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NS; ++k) {
+    // the guesses: s plus the float sums of the sub-tiles before this one
+    constexpr int kParts = (kSubs + 63) / 64;
+    float before[kParts];
+    float run = s[k];
+#pragma unroll
+    for (int h = 0; h < kParts; ++h) {
+      const uint32_t q = h * 64 + lane;
+      const float p = q < nq ? L.part[k][q] : 0.0f;
+      const float inc = wave_inclusive_sum(p);
+      before[h] = run + (inc - p);
+      run += readlane_f(inc, 63);
+    }
+#pragma unroll
+    for (int u = 0; u < K; ++u) {
+      const uint32_t q = u * kW + wave;
+      if (q >= nq) continue;
+      const float x = xv[k][u];
+      const float g = fabsf(readlane_f(before[(u * kW) / 64], q & 63));
+      const bool guess = g >= 0x1p-126f && g <= 0x1p126f;
+      const int e = guess ? float_exponent(g) : 0;
+      uint32_t d0a = 0, d1a = 0, ppa = 0, d0b = 0, d1b = 0, ppb = 0;
+      bool ha = true, hb = true;
+      if (guess) {
+        subtile_map(ldexpf(fabsf(x), 23 - e), d0a, d1a, ppa, ha);
+        subtile_map(ldexpf(fabsf(x), 22 - e), d0b, d1b, ppb, hb);
+      }
+      const uint32_t fl = (ha ? kNoMapA : 0u) | (hb ? kNoMapB : 0u) | (__ballot(x > 0.0f) ? kPos : 0u) |
+                          (__ballot(x < 0.0f) ? kNeg : 0u) | (__ballot(x != x) ? kIrregularTerm : 0u);
+      if (lane == 0) {
+        L.d0a[k][q] = d0a;
+        L.d1a[k][q] = d1a;
+        L.d0b[k][q] = d0b;
+        L.d1b[k][q] = d1b;
+        L.fe[k][q] = fl | (ppa << 8) | (ppb << 10) | ((uint32_t)(e + 256) << 12);
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NS; ++k) {
+    if (wave == (uint32_t)k) {
+      const float v = chunk_walk(s[k], nq, k, k == NS - 1 ? prefix : nullptr, L);
+      if (lane == 0) L.s[k] = v;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NS; ++k) s[k] = L.s[k];
+}
+
+// One sum of n terms, chunk by chunk.
+constexpr int kChunkPer = 8;
+using SumLds = ChunkLds<1, kChunkPer>;
+__device__ __forceinline__ float exact_sum(uint32_t n, const float* __restrict__ x, float* prefix, SumLds& L) {
+  float s[1] = {0.0f};
+  constexpr uint32_t kTerms = SumLds::kTerms;
+  for (uint32_t base = 0; base < n; base += kTerms) {
+    const uint32_t len = min(kTerms, n - base);
+    float xv[1][kChunkPer];
+#pragma unroll
+    for (int u = 0; u < kChunkPer; ++u) {
+      const uint32_t i = u * kChainThreads + threadIdx.x;
+      xv[0][u] = i < len ? x[base + i] : 0.0f;
+    }
+    if (base) __syncthreads();  // every thread has read the previous chunk's sum
+    chunk_sums<1, kChunkPer>(s, xv, len, prefix ? prefix + base / kGroup : nullptr, L);
+  }
+  return s[0];
+}
+
+// Whether any of w[0..n) is negative or not finite: the running sum c is
+// then not monotone, and resample selects serially (the flag goes to
+// sums[4]).  Called by every thread of the workgroup.
+__device__ __forceinline__ float weights_irregular(uint32_t n, const float* w) {
+  int bad = 0;
+  for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) bad |= (w[i] < 0.0f || !isfinite(w[i])) ? 1 : 0;
+  return __syncthreads_or(bad) ? 1.0f : 0.0f;
+}
+
+// wtp and wtr (grid row y = 0, 1), wt, or resample's c with its checkpoints,
+// by exact_sum: one workgroup per filter and sum.
+__global__ __launch_bounds__(kChainThreads) void exact_chain_kernel(Filters fs, int which) {
+  __shared__ SumLds lds;
+  const FilterDev& f = fsel(fs, blockIdx.x);
+  if (which == kPrefixOnly && f.no_resample) return;
+  const uint32_t n = f.n;
+  float* sc = f.scratch;
+  const float* src;
+  float* dst;
+  float* prefix = nullptr;
+  if (which == kTailTotals) {
+    src = sc + (size_t)blockIdx.y * n;
+    dst = sums_of(f) + blockIdx.y;
+  } else if (which == kWeightTotal) {
+    src = f.w;
+    dst = sums_of(f) + 2;
+  } else {  // kPrefixOnly
+    src = f.w;
+    dst = sums_of(f) + 3;
+    prefix = sc + sc_c32(n);
+  }
+  const float v = exact_sum(n, src, prefix, lds);
+  const float irregular = prefix ? weights_irregular(n, src) : 0.0f;
+  if (threadIdx.x == 0) {
+    *dst = v;
+    if (prefix) sums_of(f)[4] = irregular;
+  }
+}
+
+// The last sums of update, side by side: the four mean terms (grid rows
+// y = 0..3) and resample's running sum c over the new weights with its
+// checkpoints and the monotonicity flag (row 4).  The mean terms may have
+// either sign: sub-tiles with both are added term by term.
+__global__ __launch_bounds__(kChainThreads) void mean_prefix_kernel(Filters fs) {
+  __shared__ SumLds lds;
+  const FilterDev& f = fsel(fs, blockIdx.x);
+  const uint32_t n = f.n;
+  float* sc = f.scratch;
+  if (blockIdx.y < 4) {
+    const float v = exact_sum(n, sc + (size_t)blockIdx.y * n, nullptr, lds);
+    if (threadIdx.x == 0) f.mean[blockIdx.y] = v;
+  } else {
+    const float v = exact_sum(n, f.w, sc + sc_c32(n), lds);
+    const float irregular = weights_irregular(n, f.w);
+    if (threadIdx.x == 0) {
+      sums_of(f)[3] = v;
+      sums_of(f)[4] = irregular;
+    }
+  }
+}
+
 inline bool tiled_filter(const Filters& fs) { return !fs.arr && fs.one.n >= kTiledMin; }
 
 // with_dsum false: the kernel that wrote the terms wrote the tile records too.
@@ -1208,36 +1416,142 @@ __global__ __launch_bounds__(kChainThreads) void tail_c_tiled_kernel(Filters fs)
   tile_dsum(f, 0, t, i, w, red);
 }
 
+// The whole tail by one workgroup per filter, for filters of at most
+// kChainThreads * K particles: a particle's fields and weights stay in its
+// thread's registers between the sums, so the six launches and their passes
+// over memory become one (600 particles: 41 -> 34 us for the whole update).
+template <int K>
+__global__ __launch_bounds__(kChainThreads) void tail_one_kernel(GridDev g, Filters fs) {
+  __shared__ __align__(16) unsigned char lds[sizeof(ChunkLds<5, K>)];
+  const FilterDev& f = fsel(fs, blockIdx.x);
+  const uint32_t n = f.n, tid = threadIdx.x;
+  const GridDev& gr = f.gdev ? *f.gdev : g;
+  float p[4][K], wp[K], wr[K], w[K];
+  bool in[K];
+  float t2[2][K];
+#pragma unroll
+  for (int u = 0; u < K; ++u) {
+    const uint32_t i = u * kChainThreads + tid;
+    const bool have = i < n;
+    p[0][u] = have ? f.x[i] : 0.f;
+    p[1][u] = have ? f.y[i] : 0.f;
+    p[2][u] = have ? f.z[i] : 0.f;
+    p[3][u] = have ? f.a[i] : 0.f;
+    wp[u] = have ? f.wp[i] : 0.f;
+    wr[u] = have ? f.wr[i] : 0.f;
+    in[u] = have && into_map(gr, p[0][u], p[1][u], p[2][u]);
+    t2[0][u] = in[u] ? wp[u] : 0.f;  // ParticleFilter.cpp:129-153
+    t2[1][u] = in[u] ? wr[u] : 0.f;
+  }
+  float s2[2] = {0.f, 0.f};
+  chunk_sums<2, K>(s2, t2, n, nullptr, *reinterpret_cast<ChunkLds<2, K>*>(lds));
+  const float wtp = s2[0], wtr = s2[1];
+  float t1[1][K];
+#pragma unroll
+  for (int u = 0; u < K; ++u) {  // ParticleFilter.cpp:158-180
+    const uint32_t i = u * kChainThreads + tid;
+    wp[u] = (wtp > 0) ? wp[u] / wtp : 0.f;
+    wr[u] = (wtr > 0) ? wr[u] / wtr : 0.f;
+    if (i < n) {
+      f.wp[i] = wp[u];
+      f.wr[i] = wr[u];
+    }
+    w[u] = in[u] ? (float)(wp[u] * f.alpha + wr[u] * (1 - f.alpha)) : 0.f;
+    t1[0][u] = w[u];
+  }
+  __syncthreads();  // the sums have been read
+  float s1[1] = {0.f};
+  chunk_sums<1, K>(s1, t1, n, nullptr, *reinterpret_cast<ChunkLds<1, K>*>(lds));
+  const float wt = s1[0];
+  float t5[5][K];
+  int irregular = 0;
+#pragma unroll
+  for (int u = 0; u < K; ++u) {  // ParticleFilter.cpp:182-193
+    const uint32_t i = u * kChainThreads + tid;
+    const float v = (wt > 0) ? w[u] / wt : 0.f;
+    const bool have = i < n;
+    if (have) f.w[i] = v;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) t5[k][u] = have ? v * p[k][u] : 0.f;
+    t5[4][u] = have ? v : 0.f;
+    irregular |= (have && (v < 0.0f || !isfinite(v))) ? 1 : 0;
+  }
+  irregular = __syncthreads_or(irregular);
+  float s5[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+  chunk_sums<5, K>(s5, t5, n, f.scratch + sc_c32(n), *reinterpret_cast<ChunkLds<5, K>*>(lds));
+  if (tid == 0) {
+    float* const sums = sums_of(f);
+    sums[0] = wtp;
+    sums[1] = wtr;
+    sums[2] = wt;
+    sums[3] = s5[4];
+    sums[4] = irregular ? 1.0f : 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) f.mean[k] = s5[k];
+  }
+}
+constexpr uint32_t kTailOneMax = 2 * kChainThreads;  // K = 2: 44 KB of LDS
+
 // ---------------------------------------------------------------- resample
 // FP64 prefix: sequential double sums in blocks of 1024, block totals summed
-// in order (one workgroup per filter).
-__global__ __launch_bounds__(1024) void prefix64_kernel(Filters fs) {
-  const FilterDev& f = fsel(fs, blockIdx.x);
-  if (f.no_resample) return;
-  const uint32_t n = f.n;
-  double* c64 = reinterpret_cast<double*>(f.scratch + sc_c64(n));
-  double* tot = reinterpret_cast<double*>(f.scratch + sc_tot(n));
-  const uint32_t nb = (n + 1023) / 1024;
-  for (uint32_t b = threadIdx.x; b < nb; b += blockDim.x) {
-    double s = 0.0;
-    const uint32_t e = min(n, (b + 1) * 1024);
-    for (uint32_t i = b * 1024; i < e; ++i) {
-      s += (double)f.w[i];
-      c64[i] = s;
-    }
-    tot[b] = s;
-  }
+// in order.  One workgroup per block adds it from LDS (grid y = filter): bound
+// by its 1,024 dependent adds, 8 us for 60,000 particles, where one workgroup
+// per filter with a strided thread per block took 230 us.
+constexpr uint32_t kBlock64 = 1024;
+__global__ __launch_bounds__(256) void prefix64_block_kernel(Filters fs) {
+  const FilterDev& f = fsel(fs, blockIdx.y);
+  const uint32_t n = f.n, b = blockIdx.x, base = b * kBlock64;
+  if (f.no_resample || base >= n) return;
+  __shared__ float w[kBlock64];
+  __shared__ double c[kBlock64];
+  const uint32_t len = min(kBlock64, n - base);
+  for (uint32_t i = threadIdx.x; i < kBlock64; i += blockDim.x) w[i] = i < len ? f.w[base + i] : 0.0f;
   __syncthreads();
   if (threadIdx.x == 0) {
-    double carry = 0.0;
-    for (uint32_t b = 0; b < nb; ++b) {
-      const double t = tot[b];
-      tot[b] = carry;
-      carry = carry + t;
+    double s = 0.0;
+    const float4* const w4 = reinterpret_cast<const float4*>(w);
+    for (uint32_t q = 0; q < kBlock64 / 4; q += 8) {
+      float4 v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = w4[q + k];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const uint32_t i = 4 * (q + k);
+        c[i] = s += (double)v[k].x;
+        c[i + 1] = s += (double)v[k].y;
+        c[i + 2] = s += (double)v[k].z;
+        c[i + 3] = s += (double)v[k].w;
+      }
     }
   }
   __syncthreads();
-  for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) c64[i] = tot[i / 1024] + c64[i];
+  double* const c64 = reinterpret_cast<double*>(f.scratch + sc_c64(n));
+  for (uint32_t i = threadIdx.x; i < len; i += blockDim.x) c64[base + i] = c[i];
+  if (threadIdx.x == 0) reinterpret_cast<double*>(f.scratch + sc_tot(n))[b] = c[len - 1];
+}
+
+// Adds the totals of the earlier blocks, in order, to every block.
+__global__ __launch_bounds__(256) void prefix64_carry_kernel(Filters fs) {
+  const FilterDev& f = fsel(fs, blockIdx.y);
+  const uint32_t n = f.n, b = blockIdx.x, base = b * kBlock64;
+  if (f.no_resample || base >= n) return;
+  __shared__ double t[kBlock64];
+  __shared__ double sum;
+  const double* const tot = reinterpret_cast<const double*>(f.scratch + sc_tot(n));
+  double carry = 0.0;
+  for (uint32_t b0 = 0; b0 < b; b0 += kBlock64) {
+    const uint32_t k = min(kBlock64, b - b0);
+    for (uint32_t i = threadIdx.x; i < k; i += blockDim.x) t[i] = tot[b0 + i];
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (uint32_t i = 0; i < k; ++i) carry = carry + t[i];
+      sum = carry;
+    }
+    __syncthreads();
+  }
+  if (b) carry = sum;
+  double* const c64 = reinterpret_cast<double*>(f.scratch + sc_c64(n));
+  for (uint32_t i = base + threadIdx.x; i < min(n, base + kBlock64); i += blockDim.x) c64[i] = carry + c64[i];
 }
 
 // First i with !(u > c[i]) (the reference's while loop stops there); the
@@ -1272,11 +1586,10 @@ __device__ inline void resample_gather(const FilterDev& f, uint32_t m, uint32_t 
 // thread per filter, for weights whose running sum is not monotone (a
 // negative or non-finite weight, flagged in sums[4] with the running sum):
 // index i only moves forward, which the parallel search cannot express.
-__global__ void resample_select_serial_kernel(Filters fs) {
-  const FilterDev& f = fsel(fs, blockIdx.x);
+// take(m, i) receives particle m's ancestor.
+template <class Take>
+__device__ void select_serial(const FilterDev& f, float u01, Take&& take) {
   const uint32_t n = f.n;
-  if (threadIdx.x != 0 || f.no_resample || sums_of(f)[4] == 0.0f) return;
-  const float u01 = fs.u01 ? fs.u01[blockIdx.x] : f.u01;
   const float factor = 1.f / (float)n;
   const float r = factor * u01;
   float c = f.w[0];
@@ -1287,8 +1600,50 @@ __global__ void resample_select_serial_kernel(Filters fs) {
       if (++i >= n) break;  // the reference reads past the end here: clamped below
       c += f.w[i];
     }
-    resample_gather(f, m, min(i, n - 1));
+    take(m, min(i, n - 1));
   }
+}
+
+// Particle m's ancestor by the reference's running sum: the group holding the
+// first c_i with !(u > c_i), from the checkpoints cp, then c_i itself, re-added
+// in the reference's order from the weights w.
+__device__ __forceinline__ uint32_t select_reference(uint32_t n, uint32_t m, float u01, const float* cp,
+                                                     const float* w) {
+  const float factor = 1.f / (float)n;  // 1.f / p_.size() (size_t -> float)
+  const float r = factor * u01;
+  const float u = r + factor * (float)m;
+  const uint32_t ng = (n + kGroup - 1) / kGroup;
+  uint32_t gi = 0, hi = ng;
+  while (gi < hi) {
+    const uint32_t mid = gi + ((hi - gi) >> 1);
+    if (!(u > cp[mid]))
+      hi = mid;
+    else
+      gi = mid + 1;
+  }
+  if (gi == ng) return n - 1;  // the float total ends below u: clamped (the reference reads p_[n])
+  float c = gi ? cp[gi - 1] : 0.0f;  // 0 + w_0 is w_0 exactly
+  const uint32_t e = min(n, (gi + 1) * kGroup);
+  uint32_t i = e - 1;
+  // 16 weights loaded at a time (independent loads, one wait), then added in
+  // order until the first c that u does not exceed
+  bool found = false;
+  for (uint32_t k0 = gi * kGroup; k0 < e && !found; k0 += 16) {
+    float wv[16];
+#pragma unroll
+    for (uint32_t j = 0; j < 16; ++j) wv[j] = k0 + j < e ? w[k0 + j] : 0.0f;
+#pragma unroll
+    for (uint32_t j = 0; j < 16; ++j) {
+      if (!found && k0 + j < e) {
+        c += wv[j];
+        if (!(u > c)) {
+          i = k0 + j;
+          found = true;
+        }
+      }
+    }
+  }
+  return i;
 }
 
 __global__ void resample_select_kernel(Filters fs, int mode) {
@@ -1296,57 +1651,71 @@ __global__ void resample_select_kernel(Filters fs, int mode) {
   const uint32_t m = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t n = f.n;
   if (m >= n || f.no_resample) return;
-  if (mode == A3D_RESAMPLE_REFERENCE && sums_of(f)[4] != 0.0f) return;  // the serial kernel selects
   float* sc = f.scratch;
   const float u01 = fs.u01 ? fs.u01[blockIdx.y] : f.u01;
   uint32_t i;
   if (mode == A3D_RESAMPLE_REFERENCE) {
-    const float factor = 1.f / (float)n;  // 1.f / p_.size() (size_t -> float)
-    const float r = factor * u01;
-    const float u = r + factor * (float)m;
-    // the group holding the first running sum c_i with !(u > c_i), from the
-    // checkpoints; then c_i itself, re-added in the reference's order
-    const float* cp = sc + sc_c32(n);
-    const uint32_t ng = (n + kGroup - 1) / kGroup;
-    uint32_t gi = 0, hi = ng;
-    while (gi < hi) {
-      const uint32_t mid = gi + ((hi - gi) >> 1);
-      if (!(u > cp[mid]))
-        hi = mid;
-      else
-        gi = mid + 1;
+    if (sums_of(f)[4] != 0.0f) {
+      if (m == 0) select_serial(f, u01, [&](uint32_t j, uint32_t a) { resample_gather(f, j, a); });
+      return;
     }
-    if (gi == ng) {
-      i = n - 1;  // the float total ends below u: clamped (the reference reads p_[n])
-    } else {
-      float c = gi ? cp[gi - 1] : 0.0f;  // 0 + w_0 is w_0 exactly
-      const uint32_t e = min(n, (gi + 1) * kGroup);
-      i = e - 1;
-      // 16 weights loaded at a time (independent loads, one wait), then
-      // added in order until the first c that u does not exceed
-      bool found = false;
-      for (uint32_t k0 = gi * kGroup; k0 < e && !found; k0 += 16) {
-        float wv[16];
-#pragma unroll
-        for (uint32_t j = 0; j < 16; ++j) wv[j] = k0 + j < e ? f.w[k0 + j] : 0.0f;
-#pragma unroll
-        for (uint32_t j = 0; j < 16; ++j) {
-          if (!found && k0 + j < e) {
-            c += wv[j];
-            if (!(u > c)) {
-              i = k0 + j;
-              found = true;
-            }
-          }
-        }
-      }
-    }
+    i = select_reference(n, m, u01, sc + sc_c32(n), f.w);
   } else {
     const double* c64 = reinterpret_cast<const double*>(sc + sc_c64(n));
     const double u = ((double)u01 + (double)m) * (1.0 / (double)n);
     i = first_not_below(c64, n, u);
   }
   resample_gather(f, m, i);
+}
+
+// Selection and commit by one workgroup per filter, for filters of at most
+// kResampleOneMax particles (reference mode): the weights and checkpoints are
+// read from LDS, the gathered particles stay in registers until every thread
+// has read its ancestors.  Two launches and the staging fewer.
+constexpr uint32_t kResampleOneMax = 2 * kChainThreads;
+__global__ __launch_bounds__(kChainThreads) void resample_one_kernel(Filters fs) {
+  constexpr int K = kResampleOneMax / kChainThreads;
+  const FilterDev& f = fsel(fs, blockIdx.x);
+  if (f.no_resample) return;
+  __shared__ float w[kResampleOneMax], cp[kResampleOneMax / kGroup];
+  __shared__ uint32_t anc[kResampleOneMax];
+  const uint32_t n = f.n, tid = threadIdx.x;
+  const float u01 = fs.u01 ? fs.u01[blockIdx.x] : f.u01;
+  for (uint32_t i = tid; i < n; i += kChainThreads) w[i] = f.w[i];
+  if (tid < (n + kGroup - 1) / kGroup) cp[tid] = f.scratch[sc_c32(n) + tid];
+  const bool serial = sums_of(f)[4] != 0.0f;
+  __syncthreads();
+  if (serial) {
+    if (tid == 0 && n) select_serial(f, u01, [&](uint32_t j, uint32_t a) { anc[j] = a; });
+    __syncthreads();
+  }
+  float v[K][6];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const uint32_t m = k * kChainThreads + tid;
+    if (m >= n) break;
+    const uint32_t i = serial ? anc[m] : select_reference(n, m, u01, cp, w);
+    if (f.idx_out) f.idx_out[m] = i;
+    v[k][0] = f.x[i];
+    v[k][1] = f.y[i];
+    v[k][2] = f.z[i];
+    v[k][3] = f.a[i];
+    v[k][4] = f.wp[i];
+    v[k][5] = f.wr[i];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const uint32_t m = k * kChainThreads + tid;
+    if (m >= n) break;
+    f.x[m] = v[k][0];
+    f.y[m] = v[k][1];
+    f.z[m] = v[k][2];
+    f.a[m] = v[k][3];
+    f.wp[m] = v[k][4];
+    f.wr[m] = v[k][5];
+    f.w[m] = 1.f / (float)n;
+  }
 }
 
 __global__ void resample_commit_kernel(Filters fs) {
@@ -1406,6 +1775,11 @@ void launch_update_tail(const GridDev& g, const Filters& fs, hipStream_t s) {
     launch_tiled(fs, kMeanPrefix, 5, s);
     return;
   }
+  if (fs.max_n <= kTailOneMax) {
+    if (fs.max_n <= kChainThreads) tail_one_kernel<1><<<fs.count, kChainThreads, 0, s>>>(g, fs);
+    else tail_one_kernel<2><<<fs.count, kChainThreads, 0, s>>>(g, fs);
+    return;
+  }
   tail_a_kernel<<<ew_grid(fs), kEw, 0, s>>>(g, fs);
   exact_chain_kernel<<<dim3(fs.count, 2), kChainThreads, 0, s>>>(fs, kTailTotals);
   tail_c_kernel<<<ew_grid(fs), kEw, 0, s>>>(fs);
@@ -1425,10 +1799,15 @@ void launch_resample(const Filters& fs, int mode, bool have_prefix, hipStream_t 
         exact_chain_kernel<<<fs.count, kChainThreads, 0, s>>>(fs, kPrefixOnly);
     }
   } else {
-    prefix64_kernel<<<fs.count, 1024, 0, s>>>(fs);
+    const dim3 blocks((fs.max_n + kBlock64 - 1) / kBlock64, fs.count);
+    prefix64_block_kernel<<<blocks, 256, 0, s>>>(fs);
+    prefix64_carry_kernel<<<blocks, 256, 0, s>>>(fs);
+  }
+  if (mode == A3D_RESAMPLE_REFERENCE && fs.max_n <= kResampleOneMax) {
+    resample_one_kernel<<<fs.count, kChainThreads, 0, s>>>(fs);
+    return;
   }
   resample_select_kernel<<<ew_grid(fs), kEw, 0, s>>>(fs, mode);
-  if (mode == A3D_RESAMPLE_REFERENCE) resample_select_serial_kernel<<<fs.count, 64, 0, s>>>(fs);
   resample_commit_kernel<<<ew_grid(fs), kEw, 0, s>>>(fs);
 }
 

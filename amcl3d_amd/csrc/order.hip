@@ -270,20 +270,6 @@ __global__ __launch_bounds__(kKT) void order_scatter_kernel(OrderJob j) {
   if (i < f.n) o.order[cnt[key] + rank] = i;  // < n: the ranges of key k cover exactly its count
 }
 
-// Sum over the wavefront, in every lane.
-__device__ inline float wave_sum(float v) {
-#define A3D_DPP_ADD(ctrl, rows) \
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, rows, 0xf, true))
-  A3D_DPP_ADD(0x111, 0xf);  // row_shr 1, 2, 4, 8: lane 15 of each row holds the row's sum
-  A3D_DPP_ADD(0x112, 0xf);
-  A3D_DPP_ADD(0x114, 0xf);
-  A3D_DPP_ADD(0x118, 0xf);
-  A3D_DPP_ADD(0x142, 0xa);  // row_bcast 15 into rows 1 and 3, 31 into rows 2 and 3
-  A3D_DPP_ADD(0x143, 0xc);
-#undef A3D_DPP_ADD
-  return readlane_f(v, 63);
-}
-
 // The whole sort by one workgroup, for a single filter of at most kBT * K
 // particles: the
 // fields stay in registers between the passes, the histogram in LDS, and a
