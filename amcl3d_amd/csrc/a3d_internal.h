@@ -73,7 +73,17 @@ struct GridDev {
   // 0: never.  The allocation of such a grid of more than 2^30 cells is
   // rounded up to whole segments, so every such load stays inside it.
   uint32_t seg_bits;
-  uint32_t pad2_;
+  // 1 when the cloud weight may form cells in fixed point (fx_*, grid_meta).
+  uint32_t fixed;
+  // The fixed-point form of an axis: the double s * fx_scale + (offset *
+  // fx_scale + fx_shift) is subnormal for cells below 2^20, its high word the
+  // cell and its low word the fraction of the cell, each moved up by delta:
+  // fx_scale = 2^-1042 / res (2^-1042 is one unit of the high word), fx_shift =
+  // delta * 2^-1042.  Fractions below fx_near (2 delta) are within delta of a
+  // cell's face.
+  double fx_scale, fx_shift;
+  uint32_t fx_size[3];  // a point is in the map when its cell is below these (away from the faces)
+  uint32_t fx_near;
 };
 
 // One filter and the parameters of the call being made on it.  Arrays are

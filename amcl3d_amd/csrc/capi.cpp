@@ -64,6 +64,38 @@ static bool axis_clean(double res, double inv_res, uint32_t size) {
   return true;
 }
 
+// The fixed-point cells of the cloud weight, on a clean grid.  For a point at s of a pose at
+// offset o the reference's cell is floor(q / res) with q the float nearest to
+// s + o: its argument differs from (s + o) / res by at most half a float
+// spacing of q over res, at most half that of the axis' largest q.  The fixed
+// form has the same value within 2^-33 for each of its two roundings and q *
+// 2^-33 for the rounding of fx_scale, a subnormal (2^-1074 is its last bit).
+// delta is the sum of these bounds, so the two give the same cell unless the
+// fixed form is within delta of a cell's face.  The bound of the map (lim)
+// must be a face too, within delta's slack, on every axis.  fixed is set while
+// few groups of 256 evaluations hold a point that close (6 delta each: 28% at
+// the limit, 12% on 2,000 cells, 1.5% on 200).
+static void fixed_meta(GridDev& g) {
+  g.fixed = 0u;
+  if (!g.clean) return;
+  const double slack = 0x1p-20;
+  double half = 0.0;
+  for (int a = 0; a < 3; ++a) {
+    float b;
+    std::memcpy(&b, &g.lim[a], 4);
+    const double t = (double)b * g.inv_res, n = std::nearbyint(t);
+    if (!(n >= 1.0 && n < 0x1p19 && std::fabs(t - n) <= slack / 2)) return;
+    g.fx_size[a] = (uint32_t)n;
+    half = std::max(half, std::ldexp(1.0, std::ilogb(b) - 24));
+  }
+  const double delta = half * g.inv_res * 1.0001 + slack;
+  if (!(delta <= 0x1p-12) || !(g.inv_res < 0x1p20) || !(g.inv_res > 0x1p-20)) return;
+  g.fx_scale = std::ldexp(g.inv_res, -1042);
+  g.fx_shift = std::ldexp(delta, -1042);
+  g.fx_near = (uint32_t)std::ceil(std::ldexp(2.0 * delta, 32)) + 2u;
+  g.fixed = 1u;
+}
+
 // Grid metadata exactly as PointCloudTools.cpp:93-101 and Grid3d.cpp:151-153.
 void grid_meta(const double mn[3], const double mx[3], double res, GridDev& g) {
   for (int a = 0; a < 3; ++a) {
@@ -102,6 +134,7 @@ void grid_meta(const double mn[3], const double mx[3], double res, GridDev& g) {
   // Test knob: A3D_FORCE_NEAR_TEST=1 keeps the window test on any map.
   const char* near_test = std::getenv("A3D_FORCE_NEAR_TEST");
   if (near_test && near_test[0] == '1') g.clean = 0u;
+  fixed_meta(g);
   g.step_z = (uint64_t)g.size[0] * g.size[1];
   g.cells = g.step_z * g.size[2];
   // 32-bit cell indices use 24-bit multiply-adds: (iy + sy * iz) * sx + ix

@@ -320,13 +320,14 @@ bool a3d_server::launch(Slot& s) {
   launch_draws(fs, s.d_seedstep, s.d_seedstep + nf, s.d_u01, st);
   launch_predict(fs, st);
   // the launch's grid: the widest index kind any map of the batch needs
-  // (64-bit indices, or 32-bit ones through 64-bit addresses), clean only
-  // if every map is
+  // (64-bit indices, or 32-bit ones through 64-bit addresses), clean and
+  // fixed only if every map is
   GridDev gl = maps[map0]->g;
   for (auto& r : s.reqs) {
     gl.idx64 |= maps[sessions[r.session].map]->g.idx64;
     gl.buf32 &= maps[sessions[r.session].map]->g.buf32;
     gl.clean &= maps[sessions[r.session].map]->g.clean;
+    gl.fixed &= maps[sessions[r.session].map]->g.fixed;
   }
   // No segment loads in served batches: in batches that mix a large map with
   // smaller ones they measured slower than 64-bit addresses (the

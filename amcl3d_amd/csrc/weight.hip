@@ -24,6 +24,10 @@
 // particle's sum is the reference's sequential float sum over the cloud,
 // bit for bit (a rejected point adds -0.0f, which leaves every sum
 // unchanged).  The count of accepted points comes from a ballot.
+//
+// The kernels' instantiations are compiled as three objects side by side
+// (Makefile): A3D_WEIGHT_PART 0 the single-filter and pose launches and the
+// entry points, 1 the split form, 2 the particle-lane fleet kernels.
 #include "a3d_math.h"
 
 // The structured buffer load (buffer_load_dword ... idxen), bound to the
@@ -32,6 +36,11 @@ __device__ float a3d_struct_load_f32(__amdgpu_buffer_rsrc_t r, int vindex, int v
     "llvm.amdgcn.struct.ptr.buffer.load.f32");
 
 namespace a3d {
+
+bool launch_split(const GridDev& g, const FilterDev& f, float* out, hipStream_t s);
+void launch_lanes_fleet(const GridDev& g, const FilterDev* fs, const WorkItem* items, uint32_t nitems,
+                        uint32_t* counter, int ppw, int persistent, uint32_t chunk, hipStream_t s);
+
 namespace {
 
 // Workgroups are dealt to the 8 XCDs round-robin by index.  Single-filter
@@ -314,11 +323,30 @@ struct LanePose {
   float r[9];
   double ox, oy, oz;
   bool slow;
+  // fixed-point cells: offset * fx_scale + fx_shift per axis (a lane without
+  // an active particle: a cell of 2^1042, half way between two faces) and the
+  // pose itself, from which the rare exact path takes the offsets again
+  double fx, fy, fz;
+  float tx, ty, tz;
 };
+
+__device__ __forceinline__ void set_fixed(const GridDev& g, LanePose& lp, bool act, float tx, float ty, float tz) {
+  const double out = __hiloint2double(0x3ff00000, (int)0x80000000u);
+  lp.fx = act ? ((double)tx - g.min[0]) * g.fx_scale + g.fx_shift : out;
+  lp.fy = act ? ((double)ty - g.min[1]) * g.fx_scale + g.fx_shift : out;
+  lp.fz = act ? ((double)tz - g.min[2]) * g.fx_scale + g.fx_shift : out;
+  lp.tx = act ? tx : __builtin_nanf("");
+  lp.ty = ty;
+  lp.tz = tz;
+}
 
 // A cloud point as staged for the particle lanes: x and y as floats and z as
 // a float in .z, or, with roll = pitch = 0 (where z enters the arithmetic
 // only as (double)pz), as that double in (.z, .w).
+// x of a point that is in no map under any pose: its rotation has a coordinate
+// of half its magnitude or more.
+constexpr float kOutside = 1e30f;
+
 template <bool RP0>
 __device__ __forceinline__ float4 stage_point(float px, float py, float pz) {
   if (RP0) {
@@ -379,6 +407,8 @@ __device__ __forceinline__ int add_mask_bit(int c, uint64_t m) {  // c + (this l
   return r;
 }
 
+__device__ __forceinline__ int mask_bit(uint64_t m) { return (int)((m >> lane_id()) & 1ull); }
+
 // How the fast cell index is made exact:
 //   kWindow     window test on every axis, flagged lanes (and slow lanes)
 //               redone with the division;
@@ -387,7 +417,16 @@ __device__ __forceinline__ int add_mask_bit(int c, uint64_t m) {  // c + (this l
 //   kCleanZero  a clean grid and a wavefront with slow lanes: q = -0.0, the
 //               one value the bit-pattern bound rejects wrongly, is accepted
 //               by an explicit compare.
-enum CellMode { kWindow = 0, kClean = 1, kCleanZero = 2 };
+//   kFixed      fixed-point cells (GridDev::fixed): one fused multiply-add and
+//               one compare per axis; lanes within delta of a cell's face
+//               (where the reference's rounding of q could give the other
+//               cell; a zero q and a non-finite point among them) are redone
+//               in kClean's form.
+enum CellMode { kWindow = 0, kClean = 1, kCleanZero = 2, kFixed = 3 };
+
+// The grids of a launch: any (window test), all clean, all with fixed-point
+// cells.
+enum GridMode { kAnyGrid = 0, kCleanGrid = 1, kFixedGrid = 2 };
 
 // Cell of one staged point under the lane's pose, fast form: vm, the lanes
 // whose point is in the map; near (kWindow: some axis needs the exact
@@ -425,6 +464,40 @@ __device__ __forceinline__ typename ProbSrc<IK>::Idx cell_fast(const GridDev& g,
   }
 }
 
+// a * s + c in the three-address form, c kept (the compiler otherwise copies c
+// into a two-address multiply-add, one instruction more per axis).
+__device__ __forceinline__ double fma3(double a, double s, double c) {
+  double r;
+  asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(s), "v"(c));
+  return r;
+}
+
+// kFixed: the index to load, vm, and near, the least fraction of the three axes
+// (below fx_near: cell_redo decides).  24 vector instructions per 64
+// evaluations, its share of the rotation, the sum and the loop included, where
+// kClean takes 34: per axis the offset add, two conversions, the product and
+// the truncation become one multiply-add.
+template <bool RP0, int IK>
+__device__ __forceinline__ typename ProbSrc<IK>::Idx cell_fixed(const GridDev& g, const ProbSrc<IK>& src,
+                                                                   const LanePose& lp, const float4& p, uint64_t& vm,
+                                                                   uint32_t& near) {
+  double dx, dy, dz;
+  rotate<RP0>(lp.r, p, dx, dy, dz);
+  const double x = fma3(dx, g.fx_scale, lp.fx), y = fma3(dy, g.fx_scale, lp.fy), z = fma3(dz, g.fx_scale, lp.fz);
+  const uint32_t ix = (uint32_t)__double2hiint(x), iy = (uint32_t)__double2hiint(y), iz = (uint32_t)__double2hiint(z);
+  near = min(min((uint32_t)__double2loint(x), (uint32_t)__double2loint(y)), (uint32_t)__double2loint(z));
+  const bool inx = ix < g.fx_size[0], iny = iy < g.fx_size[1], inz = iz < g.fx_size[2];
+  const auto lin = linear<IK>(g, ix, iy, iz);
+  if constexpr (IK == kIdx64) {
+    const bool valid = inx & iny & inz;
+    vm = __builtin_amdgcn_ballot_w64(valid);
+    return valid ? lin : src.zero;
+  } else {
+    vm = __builtin_amdgcn_ballot_w64(inx) & __builtin_amdgcn_ballot_w64(iny) & __builtin_amdgcn_ballot_w64(inz);
+    return select_by_mask(vm, lin, src.zero);
+  }
+}
+
 // The same with the correctly rounded division on every axis.
 template <bool RP0, int IK>
 __device__ __forceinline__ typename ProbSrc<IK>::Idx cell_exact(const GridDev& g, const ProbSrc<IK>& src,
@@ -436,6 +509,26 @@ __device__ __forceinline__ typename ProbSrc<IK>::Idx cell_exact(const GridDev& g
   axis_exact(dx, lp.ox, g.ext_hi[0], g.res, g.size[0], okx, ix);
   axis_exact(dy, lp.oy, g.ext_hi[1], g.res, g.size[1], oky, iy);
   axis_exact(dz, lp.oz, g.ext_hi[2], g.res, g.size[2], okz, iz);
+  valid = okx & oky & okz;
+  const auto lin = linear<IK>(g, ix, iy, iz);
+  return valid ? lin : src.zero;
+}
+
+// A near lane of kFixed, by the truncated product (exact on a clean grid; q =
+// -0.0 accepted).  The offsets are taken again from the pose behind an opaque
+// copy: hoisted out of the loop, they would cost the fast path 40 registers.
+template <bool RP0, int IK>
+__device__ __forceinline__ typename ProbSrc<IK>::Idx cell_redo(const GridDev& g, const ProbSrc<IK>& src,
+                                                                  const LanePose& lp, const float4& p, bool& valid) {
+  float tx = lp.tx, ty = lp.ty, tz = lp.tz;
+  asm volatile("" : "+v"(tx), "+v"(ty), "+v"(tz));
+  double dx, dy, dz;
+  rotate<RP0>(lp.r, p, dx, dy, dz);
+  bool okx, oky, okz;
+  uint32_t ix, iy, iz;
+  axis_clean<true>(dx, (double)tx - g.min[0], g.lim[0], g.inv_res, okx, ix);
+  axis_clean<true>(dy, (double)ty - g.min[1], g.lim[1], g.inv_res, oky, iy);
+  axis_clean<true>(dz, (double)tz - g.min[2], g.lim[2], g.inv_res, okz, iz);
   valid = okx & oky & okz;
   const auto lin = linear<IK>(g, ix, iy, iz);
   return valid ? lin : src.zero;
@@ -478,30 +571,41 @@ __device__ __forceinline__ void lanes_chunk(const GridDev& g, const ProbSrc<IK>&
   for (int s0 = 0; s0 < S; s0 += U) {
     Idx idx[U];
     bool nr[U];
+    uint32_t lo[U];
+    uint64_t vm[U];
     float4 pt[U];  // all LDS reads of the group first
 #pragma unroll
     for (int u = 0; u < U; ++u) pt[u] = cl[(s0 + u) * Q + po];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      uint64_t vm;
-      idx[u] = cell_fast<RP0, IK, MODE>(g, src, lp, pt[u], vm, nr[u]);
-      cnt = add_mask_bit(cnt, vm);
+      if constexpr (MODE == kFixed)
+        idx[u] = cell_fixed<RP0, IK>(g, src, lp, pt[u], vm[u], lo[u]);
+      else
+        idx[u] = cell_fast<RP0, IK, MODE>(g, src, lp, pt[u], vm[u], nr[u]);
+      cnt = add_mask_bit(cnt, vm[u]);
     }
     bool any = false;
+    if constexpr (MODE == kFixed) {
+      uint32_t least = lo[0];
 #pragma unroll
-    for (int u = 0; u < U; ++u) any |= nr[u];
-    if (MODE == kWindow && __builtin_expect(__builtin_amdgcn_ballot_w64(any) != 0, 0)) {
-      // rare: redo the flagged lanes with the division, re-reading their
-      // points (nothing of the fast form is kept for this path)
-      const volatile float* vcl = reinterpret_cast<const volatile float*>(cl);
+      for (int u = 1; u < U; ++u) least = min(least, lo[u]);
+      any = least < g.fx_near;
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u) any |= nr[u];
+    }
+    if ((MODE == kWindow || MODE == kFixed) && __builtin_expect(__builtin_amdgcn_ballot_w64(any) != 0, 0)) {
+      // rare: redo the flagged lanes, re-reading their points (the index is
+      // opaque, so nothing of the fast form is kept for this path)
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        if (nr[u]) {
-          const int k = 4 * ((s0 + u) * Q + po);
-          const float4 p = make_float4(vcl[k], vcl[k + 1], vcl[k + 2], vcl[k + 3]);
+        if (MODE == kFixed ? lo[u] < g.fx_near : nr[u]) {
+          int k = (s0 + u) * Q + po;
+          asm volatile("" : "+v"(k));
+          const float4 p = cl[k];
           bool ve;
-          const Idx ie = cell_exact<RP0, IK>(g, src, lp, p, ve);
-          cnt += (ve ? 1 : 0) - (idx[u] != src.zero ? 1 : 0);
+          const Idx ie = MODE == kFixed ? cell_redo<RP0, IK>(g, src, lp, p, ve) : cell_exact<RP0, IK>(g, src, lp, p, ve);
+          cnt += (ve ? 1 : 0) - mask_bit(vm[u]);
           idx[u] = ie;
         }
       }
@@ -518,9 +622,13 @@ __device__ __forceinline__ void lanes_chunk(const GridDev& g, const ProbSrc<IK>&
   }
 }
 
+// A non-finite point, which is in no map, is staged as the outside point
+// (finite: kFixed would redo a non-finite one at every step).
 template <bool RP0>
 __device__ inline float4 cloud_point(const FilterDev& f, uint32_t j) {
-  return stage_point<RP0>(f.cx[j], f.cy[j], f.cz[j]);
+  const float x = f.cx[j], y = f.cy[j], z = f.cz[j];
+  const bool ok = isfinite(x) && isfinite(y) && isfinite(z);
+  return stage_point<RP0>(ok ? x : kOutside, ok ? y : 0.0f, ok ? z : 0.0f);
 }
 
 // One lane's particle over the whole cloud.  BLOCK: the workgroup's
@@ -601,17 +709,24 @@ __device__ __forceinline__ void lanes_loop(const GridDev& g, const FilterDev& f,
     const uint32_t j = c0 + po;
     const bool pin = j < m;
     const uint32_t js = pin ? j : 0u;
-    // a lane past the cloud's end takes a NaN point, which every test rejects
-    const float4 p = stage_point<RP0>(pin ? f.cx[js] : __builtin_nanf(""), f.cy[js], f.cz[js]);
+    // a lane past the cloud's end takes a point outside every map
+    const float4 p = stage_point<RP0>(pin ? f.cx[js] : kOutside, f.cy[js], f.cz[js]);
     uint64_t vm;
     bool nr;
-    Idx idx = cell_fast<RP0, IK, MODE>(g, src, lp, p, vm, nr);
+    Idx idx;
+    if constexpr (MODE == kFixed) {
+      uint32_t lo;
+      idx = cell_fixed<RP0, IK>(g, src, lp, p, vm, lo);
+      nr = lo < g.fx_near;
+    } else {
+      idx = cell_fast<RP0, IK, MODE>(g, src, lp, p, vm, nr);
+    }
     cnt = add_mask_bit(cnt, vm);
-    if (MODE == kWindow && __builtin_expect(__builtin_amdgcn_ballot_w64(nr) != 0, 0)) {
+    if ((MODE == kWindow || MODE == kFixed) && __builtin_expect(__builtin_amdgcn_ballot_w64(nr) != 0, 0)) {
       if (nr) {
         bool ve;
-        const Idx ie = cell_exact<RP0, IK>(g, src, lp, p, ve);
-        cnt += (ve ? 1 : 0) - (idx != src.zero ? 1 : 0);
+        const Idx ie = MODE == kFixed ? cell_redo<RP0, IK>(g, src, lp, p, ve) : cell_exact<RP0, IK>(g, src, lp, p, ve);
+        cnt += (ve ? 1 : 0) - mask_bit(vm);
         idx = ie;
       }
     }
@@ -622,11 +737,16 @@ __device__ __forceinline__ void lanes_loop(const GridDev& g, const FilterDev& f,
 // The loop variant of a wavefront: uniform per wavefront; in BLOCK form
 // wavefronts of one workgroup may take different ones, each passing the same
 // barriers.
-template <int Q, int IK, bool CLEAN, bool BLOCK>
+template <int Q, int IK, int GM, bool BLOCK>
 __device__ __forceinline__ void lanes_variant_loop(const GridDev& g, const FilterDev& f, const LanePose& lp,
                                                    float& wsum, int& cnt, float4* cl, bool run, uint32_t chunk,
                                                    uint32_t segk) {
-  if constexpr (CLEAN) {
+  if constexpr (GM == kFixedGrid) {
+    if (f.rp0)
+      lanes_loop<Q, true, IK, kFixed, BLOCK>(g, f, lp, wsum, cnt, cl, run, chunk, segk);
+    else
+      lanes_loop<Q, false, IK, kFixed, BLOCK>(g, f, lp, wsum, cnt, cl, run, chunk, segk);
+  } else if constexpr (GM == kCleanGrid) {
     const bool zero = __builtin_amdgcn_ballot_w64(lp.slow) != 0;
     if (f.rp0) {
       if (zero)
@@ -747,10 +867,10 @@ __device__ __forceinline__ bool wave_segment(const GridDev& g, const FilterDev& 
   return __builtin_amdgcn_readfirstlane((int)seg) != 0;
 }
 
-// CLEAN: the launch's grids are all clean (GridDev::clean).  BLOCK: the
+// GM: what holds of all the launch's grids (GridMode).  BLOCK: the
 // workgroup walks the cloud together (every wavefront calls this, count may
 // be 0); cl then holds two chunks per workgroup, else one per wavefront.
-template <int Q, int IK, bool KFILTER, bool CLEAN, bool BLOCK>
+template <int Q, int IK, bool KFILTER, int GM, bool BLOCK>
 __device__ void weight_lanes(const GridDev& g, const FilterDev& f, uint32_t p0, uint32_t count, float* out,
                              float4* cl, uint32_t chunk) {
   const int lane = lane_id();
@@ -776,6 +896,7 @@ __device__ void weight_lanes(const GridDev& g, const FilterDev& f, uint32_t p0, 
   lp.oz = act ? (double)tz - g.min[2] : nan;
   constexpr double kTiny = 0x1p-96;
   lp.slow = fabs(lp.ox) < kTiny || fabs(lp.oy) < kTiny || fabs(lp.oz) < kTiny;
+  if constexpr (GM == kFixedGrid) set_fixed(g, lp, act, tx, ty, tz);
   float wr = 0.f;
   if (KFILTER && act && po == 0) wr = range_weight(tx, ty, tz, f.ranges, f.nb, f.sigma);
   float wsum = 0.f;
@@ -783,11 +904,11 @@ __device__ void weight_lanes(const GridDev& g, const FilterDev& f, uint32_t p0, 
   if constexpr (IK != kIdxBuf) {
     uint32_t segk = 0;
     if (g.seg_bits && f.zr && wave_segment(g, f, act, lp.oz, &segk))
-      lanes_variant_loop<Q, kIdxSeg, CLEAN, BLOCK>(g, f, lp, wsum, cnt, cl, run, chunk, segk);
+      lanes_variant_loop<Q, kIdxSeg, GM, BLOCK>(g, f, lp, wsum, cnt, cl, run, chunk, segk);
     else
-      lanes_variant_loop<Q, IK, CLEAN, BLOCK>(g, f, lp, wsum, cnt, cl, run, chunk, 0u);
+      lanes_variant_loop<Q, IK, GM, BLOCK>(g, f, lp, wsum, cnt, cl, run, chunk, 0u);
   } else {
-    lanes_variant_loop<Q, IK, CLEAN, BLOCK>(g, f, lp, wsum, cnt, cl, run, chunk, 0u);
+    lanes_variant_loop<Q, IK, GM, BLOCK>(g, f, lp, wsum, cnt, cl, run, chunk, 0u);
   }
   if (Q > 1) {
     int c = cnt;
@@ -808,17 +929,17 @@ __device__ void weight_lanes(const GridDev& g, const FilterDev& f, uint32_t p0, 
 
 // One filter: the workgroup's wavefronts hold consecutive particles (of the
 // visiting order) and walk the cloud together.
-template <int Q, int IK, bool CLEAN>
+template <int Q, int IK, int GM>
 __global__ __launch_bounds__(kBlockThreads) void lanes_single_kernel(GridDev g, FilterDev f, uint32_t chunk) {
   constexpr uint32_t P = 64 / Q;
   __shared__ float4 cloud[2 * kMaxChunk];
   const uint32_t wave = xcd_block(blockIdx.x, gridDim.x) * kBlockWaves + (threadIdx.x >> 6);
   const uint32_t p0 = wave * P;
   const uint32_t count = p0 < f.n ? min(P, f.n - p0) : 0u;
-  weight_lanes<Q, IK, true, CLEAN, true>(g, f, p0, count, nullptr, cloud, chunk);
+  weight_lanes<Q, IK, true, GM, true>(g, f, p0, count, nullptr, cloud, chunk);
 }
 
-template <int Q, int IK, bool CLEAN>
+template <int Q, int IK, int GM>
 __global__ __launch_bounds__(kBlockThreads) void lanes_poses_kernel(GridDev g, FilterDev f, float* out,
                                                                     uint32_t chunk) {
   constexpr uint32_t P = 64 / Q;
@@ -826,7 +947,7 @@ __global__ __launch_bounds__(kBlockThreads) void lanes_poses_kernel(GridDev g, F
   const uint32_t wave = blockIdx.x * kBlockWaves + (threadIdx.x >> 6);
   const uint32_t p0 = wave * P;
   const uint32_t count = p0 < f.n ? min(P, f.n - p0) : 0u;
-  weight_lanes<Q, IK, false, CLEAN, true>(g, f, p0, count, out, cloud, chunk);
+  weight_lanes<Q, IK, false, GM, true>(g, f, p0, count, out, cloud, chunk);
 }
 
 // ---------------------------------------------------------------------------
@@ -839,7 +960,7 @@ __global__ __launch_bounds__(kBlockThreads) void lanes_poses_kernel(GridDev g, F
 // float sum.  Tiles are double buffered and everything runs ahead of the sum:
 // in iteration t the evaluating wavefronts compute tile t's cells, write tile
 // t-1's values and issue tile t's gathers, while the adding wavefront adds
-// tile t-2.  Points past the cloud's end are NaN (rejected: +0, which leaves a
+// tile t-2.  Points past the cloud's end are outside the map (+0, which leaves a
 // sum unchanged), so no remainder loop is needed.
 template <int P, int W>
 struct Split {
@@ -872,7 +993,7 @@ __device__ __forceinline__ void split_eval(const GridDev& g, const FilterDev& f,
       const uint32_t j = t * T + (uint32_t)u * (W * Q) + first;
       const bool in = j < m;
       const uint32_t js = in ? j : m - 1;
-      p.x[u] = in ? f.cx[js] : __builtin_nanf("");
+      p.x[u] = in ? f.cx[js] : kOutside;
       p.y[u] = f.cy[js];
       p.z[u] = f.cz[js];
     }
@@ -886,23 +1007,32 @@ __device__ __forceinline__ void split_eval(const GridDev& g, const FilterDev& f,
     if (t + 1 < ntiles) load(t + 1, nxt);
     Idx idx[U];
     bool nr[U];
+    uint32_t lo[U];
+    uint64_t vm[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      uint64_t vm;
-      idx[u] = cell_fast<RP0, IK, MODE>(g, src, lp, stage_point<RP0>(cur.x[u], cur.y[u], cur.z[u]), vm, nr[u]);
-      cnt = add_mask_bit(cnt, vm);
+      const float4 p = stage_point<RP0>(cur.x[u], cur.y[u], cur.z[u]);
+      if constexpr (MODE == kFixed)
+        idx[u] = cell_fixed<RP0, IK>(g, src, lp, p, vm[u], lo[u]);
+      else
+        idx[u] = cell_fast<RP0, IK, MODE>(g, src, lp, p, vm[u], nr[u]);
+      cnt = add_mask_bit(cnt, vm[u]);
     }
-    if constexpr (MODE == kWindow) {
+    if constexpr (MODE == kWindow || MODE == kFixed) {
       bool any = false;
 #pragma unroll
-      for (int u = 0; u < U; ++u) any |= nr[u];
+      for (int u = 0; u < U; ++u) {
+        if (MODE == kFixed) nr[u] = lo[u] < g.fx_near;
+        any |= nr[u];
+      }
       if (__builtin_expect(__builtin_amdgcn_ballot_w64(any) != 0, 0)) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           if (nr[u]) {
             bool ve;
-            const Idx ie = cell_exact<RP0, IK>(g, src, lp, stage_point<RP0>(cur.x[u], cur.y[u], cur.z[u]), ve);
-            cnt += (ve ? 1 : 0) - (idx[u] != src.zero ? 1 : 0);
+            const float4 p = stage_point<RP0>(cur.x[u], cur.y[u], cur.z[u]);
+            const Idx ie = MODE == kFixed ? cell_redo<RP0, IK>(g, src, lp, p, ve) : cell_exact<RP0, IK>(g, src, lp, p, ve);
+            cnt += (ve ? 1 : 0) - mask_bit(vm[u]);
             idx[u] = ie;
           }
         }
@@ -955,10 +1085,15 @@ __device__ __forceinline__ void split_add(const float* row, uint32_t len, float&
   }
 }
 
-template <int P, int W, int IK, bool CLEAN>
+template <int P, int W, int IK, int GM>
 __device__ __forceinline__ void split_variant(const GridDev& g, const FilterDev& f, const LanePose& lp, int& cnt,
                                               float* tiles, uint32_t segk) {
-  if constexpr (CLEAN) {
+  if constexpr (GM == kFixedGrid) {
+    if (f.rp0)
+      split_eval<P, W, true, IK, kFixed>(g, f, lp, cnt, tiles, segk);
+    else
+      split_eval<P, W, false, IK, kFixed>(g, f, lp, cnt, tiles, segk);
+  } else if constexpr (GM == kCleanGrid) {
     const bool zero = __builtin_amdgcn_ballot_w64(lp.slow) != 0;
     if (f.rp0) {
       if (zero)
@@ -979,7 +1114,7 @@ __device__ __forceinline__ void split_variant(const GridDev& g, const FilterDev&
   }
 }
 
-template <int P, int W, int IK, bool KFILTER, bool CLEAN>
+template <int P, int W, int IK, bool KFILTER, int GM>
 __global__ __launch_bounds__((Split<P, W>::kThreads)) void lanes_split_kernel(GridDev g, FilterDev f, float* out) {
   using S = Split<P, W>;
   constexpr int Q = S::Q;
@@ -1036,16 +1171,17 @@ __global__ __launch_bounds__((Split<P, W>::kThreads)) void lanes_split_kernel(Gr
   lp.oz = act ? (double)tz - g.min[2] : nan;
   constexpr double kTiny = 0x1p-96;
   lp.slow = fabs(lp.ox) < kTiny || fabs(lp.oy) < kTiny || fabs(lp.oz) < kTiny;
+  if constexpr (GM == kFixedGrid) set_fixed(g, lp, act, tx, ty, tz);
   int cnt = 0;
   if (ntiles > 0) {
     if constexpr (IK != kIdxBuf) {
       uint32_t segk = 0;
       if (g.seg_bits && f.zr && wave_segment(g, f, act, lp.oz, &segk))
-        split_variant<P, W, kIdxSeg, CLEAN>(g, f, lp, cnt, tiles, segk);
+        split_variant<P, W, kIdxSeg, GM>(g, f, lp, cnt, tiles, segk);
       else
-        split_variant<P, W, IK, CLEAN>(g, f, lp, cnt, tiles, 0u);
+        split_variant<P, W, IK, GM>(g, f, lp, cnt, tiles, 0u);
     } else {
-      split_variant<P, W, IK, CLEAN>(g, f, lp, cnt, tiles, 0u);
+      split_variant<P, W, IK, GM>(g, f, lp, cnt, tiles, 0u);
     }
   }
 #pragma unroll
@@ -1060,7 +1196,7 @@ __global__ __launch_bounds__((Split<P, W>::kThreads)) void lanes_split_kernel(Gr
 // grid (a batch over several maps) is weighted on that grid, else on the
 // launch's; the launch grid's seg_bits = 0 keeps every filter off segment
 // loads.
-template <int Q, int IK, bool CLEAN>
+template <int Q, int IK, int GM>
 __device__ __forceinline__ void lanes_item(const GridDev& g, const FilterDev& f, const WorkItem& it, float4* cl,
                                            uint32_t chunk) {
   constexpr uint32_t P = 64 / Q;
@@ -1069,16 +1205,16 @@ __device__ __forceinline__ void lanes_item(const GridDev& g, const FilterDev& f,
   if (f.gdev) {
     GridDev gf = *f.gdev;
     if (!g.seg_bits) gf.seg_bits = 0u;  // the launch holds off segment loads
-    weight_lanes<Q, IK, true, CLEAN, true>(gf, f, p0, count, nullptr, cl, chunk);
+    weight_lanes<Q, IK, true, GM, true>(gf, f, p0, count, nullptr, cl, chunk);
   } else {
-    weight_lanes<Q, IK, true, CLEAN, true>(g, f, p0, count, nullptr, cl, chunk);
+    weight_lanes<Q, IK, true, GM, true>(g, f, p0, count, nullptr, cl, chunk);
   }
 }
 
 // Clean grids: at most 128 registers, four wavefronts per SIMD (the loads
 // of spread particle sets need the wavefronts to hide their latency).
-template <int Q, int IK, bool CLEAN>
-__global__ __launch_bounds__(kBlockThreads, CLEAN ? 4 : 1) void lanes_fleet_kernel(GridDev g, const FilterDev* fs,
+template <int Q, int IK, int GM>
+__global__ __launch_bounds__(kBlockThreads, GM != kAnyGrid ? 4 : 1) void lanes_fleet_kernel(GridDev g, const FilterDev* fs,
                                                                     const WorkItem* items, uint32_t nitems,
                                                                     uint32_t* counter, int persistent,
                                                                     uint32_t chunk, uint32_t deal) {
@@ -1087,7 +1223,7 @@ __global__ __launch_bounds__(kBlockThreads, CLEAN ? 4 : 1) void lanes_fleet_kern
   if (!persistent) {
     if (blockIdx.x >= nitems) return;
     const WorkItem it = items[blockIdx.x];
-    lanes_item<Q, IK, CLEAN>(g, fs[it.filter], it, cloud, chunk);
+    lanes_item<Q, IK, GM>(g, fs[it.filter], it, cloud, chunk);
     return;
   }
   for (uint32_t r = 0; r < kXcds; ++r) {
@@ -1099,7 +1235,7 @@ __global__ __launch_bounds__(kBlockThreads, CLEAN ? 4 : 1) void lanes_fleet_kern
       __syncthreads();  // every wavefront has read it before the next take
       if (t >= len) break;  // uniform over the workgroup
       const WorkItem it = items[deal_item(nitems, x, deal, t)];
-      lanes_item<Q, IK, CLEAN>(g, fs[it.filter], it, cloud, chunk);
+      lanes_item<Q, IK, GM>(g, fs[it.filter], it, cloud, chunk);
     }
   }
 }
@@ -1173,6 +1309,29 @@ __global__ void zero_u32_kernel(uint32_t* p, uint32_t n) {
   if (i < n) p[i] = 0u;
 }
 
+// The index kind a launch reads its grids with: the widest its maps need.
+inline int index_kind(const GridDev& g) { return g.idx64 ? kIdx64 : (g.buf32 ? kIdxBuf : kIdx32); }
+
+// Launches pick the kernel of the grid's index kind and grid mode: variant 3 *
+// kind + mode.
+inline int grid_mode(const GridDev& g) { return g.fixed ? kFixedGrid : (g.clean ? kCleanGrid : kAnyGrid); }
+inline int lanes_variant(const GridDev& g) { return 3 * index_kind(g) + grid_mode(g); }
+[[maybe_unused]] constexpr int kVariants = 9;
+
+#define A3D_LANES_VARIANT(v, KERNEL, Q, LAUNCH, ...) \
+  switch (v) { \
+    case 0: KERNEL<Q, kIdxBuf, kAnyGrid><<<LAUNCH>>>(__VA_ARGS__); break; \
+    case 1: KERNEL<Q, kIdxBuf, kCleanGrid><<<LAUNCH>>>(__VA_ARGS__); break; \
+    case 2: KERNEL<Q, kIdxBuf, kFixedGrid><<<LAUNCH>>>(__VA_ARGS__); break; \
+    case 3: KERNEL<Q, kIdx32, kAnyGrid><<<LAUNCH>>>(__VA_ARGS__); break; \
+    case 4: KERNEL<Q, kIdx32, kCleanGrid><<<LAUNCH>>>(__VA_ARGS__); break; \
+    case 5: KERNEL<Q, kIdx32, kFixedGrid><<<LAUNCH>>>(__VA_ARGS__); break; \
+    case 6: KERNEL<Q, kIdx64, kAnyGrid><<<LAUNCH>>>(__VA_ARGS__); break; \
+    case 7: KERNEL<Q, kIdx64, kCleanGrid><<<LAUNCH>>>(__VA_ARGS__); break; \
+    default: KERNEL<Q, kIdx64, kFixedGrid><<<LAUNCH>>>(__VA_ARGS__); break; \
+  }
+
+#if A3D_WEIGHT_PART == 0
 template <int PB>
 void launch_single_pb(const GridDev& g, const FilterDev& f, hipStream_t s) {
   const uint32_t waves = (f.n + PB - 1) / PB;
@@ -1222,23 +1381,6 @@ void launch_fleet_pb(const GridDev& g, const FilterDev* fs, const WorkItem* item
     weight_fleet_kernel<PB, false><<<blocks, kThreads, 0, s>>>(g, fs, items, nitems, counter, persistent, deal);
 }
 
-// The index kind a launch reads its grids with: the widest its maps need.
-inline int index_kind(const GridDev& g) { return g.idx64 ? kIdx64 : (g.buf32 ? kIdxBuf : kIdx32); }
-
-// Launches pick the kernel of the grid's index kind and, for a clean grid,
-// the one without the window test: variant 2 * kind + clean.
-#define A3D_LANES_VARIANT(v, KERNEL, Q, LAUNCH, ...)                                   \
-  switch (v) {                                                                          \
-    case 0: KERNEL<Q, kIdxBuf, false><<<LAUNCH>>>(__VA_ARGS__); break;                  \
-    case 1: KERNEL<Q, kIdxBuf, true><<<LAUNCH>>>(__VA_ARGS__); break;                   \
-    case 2: KERNEL<Q, kIdx32, false><<<LAUNCH>>>(__VA_ARGS__); break;                   \
-    case 3: KERNEL<Q, kIdx32, true><<<LAUNCH>>>(__VA_ARGS__); break;                    \
-    case 4: KERNEL<Q, kIdx64, false><<<LAUNCH>>>(__VA_ARGS__); break;                   \
-    default: KERNEL<Q, kIdx64, true><<<LAUNCH>>>(__VA_ARGS__); break;                   \
-  }
-
-inline int lanes_variant(const GridDev& g) { return 2 * index_kind(g) + (g.clean ? 1 : 0); }
-
 template <int Q>
 void lanes_single_q(const GridDev& g, const FilterDev& f, uint32_t chunk, hipStream_t s) {
   constexpr uint32_t P = 64 / Q;
@@ -1259,96 +1401,7 @@ void lanes_poses_q(const GridDev& g, const FilterDev& f, float* out, uint32_t ch
 #undef A3D_LAUNCH
 }
 
-// The grids wider than a buffer share the 64-bit kernel (it reads every grid,
-// and takes segment loads like the 32-bit kind).
-template <int P, int W, bool KFILTER>
-void split_pw(const GridDev& g, const FilterDev& f, float* out, hipStream_t s) {
-  const dim3 b((f.n + P - 1) / P), t(Split<P, W>::kThreads);
-  if (index_kind(g) == kIdxBuf) {
-    if (g.clean) lanes_split_kernel<P, W, kIdxBuf, KFILTER, true><<<b, t, 0, s>>>(g, f, out);
-    else lanes_split_kernel<P, W, kIdxBuf, KFILTER, false><<<b, t, 0, s>>>(g, f, out);
-  } else {
-    if (g.clean) lanes_split_kernel<P, W, kIdx64, KFILTER, true><<<b, t, 0, s>>>(g, f, out);
-    else lanes_split_kernel<P, W, kIdx64, KFILTER, false><<<b, t, 0, s>>>(g, f, out);
-  }
-}
-
-// Launches of up to kSplitMax particles take the split form.  Weight kernel
-// alone, whole-cloud wavefronts of 16 against the split form at the chosen P
-// (us; particles x points, map, spread):
-//   600 x 2,000 room, 0.1 m                   62 -> 17 (P = 4; 18 at 8, 24 at 16)
-//   300 x 20,000 floor, 0.1 m                632 -> 92 (P = 4; 110, 196)
-//   2,000 x 4,000 floor, tilted, 0.5 m       171 -> 41 (P = 4; 45, 70)
-//   5,000 x 6,000 floor, tilted, 0.1 m       213 -> 76 (P = 8; 95 at 4, 94 at 16)
-//   20,011 x 7,993 floor, tilted, 0.5 m      385 -> 350 (P = 16)
-//   40,000 x 8,000 floor, 0.5 m              516, split 711: enough whole-cloud
-//   wavefronts, which share more lines per workgroup (64 particles)
-// Small P is bound by the adding wavefront (one dependent add per point, 4.6
-// ns), larger P by the gathers.
-constexpr uint32_t kSplit4Max = 2048, kSplit8Max = 8192, kSplitMax = 28672;
-
-template <bool KFILTER>
-bool launch_split(const GridDev& g, const FilterDev& f, float* out, hipStream_t s) {
-  if (f.n > kSplitMax) return false;
-  if (f.n <= kSplit4Max) split_pw<4, 4, KFILTER>(g, f, out, s);
-  else if (f.n <= kSplit8Max) split_pw<8, 4, KFILTER>(g, f, out, s);
-  else split_pw<16, 4, KFILTER>(g, f, out, s);
-  return true;
-}
-
-template <int Q>
-int fleet_blocks_per_cu(int v) {
-  int per_cu = 1;
-  switch (v) {
-    case 0: (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lanes_fleet_kernel<Q, kIdxBuf, false>,
-                                                               kBlockThreads, 0); break;
-    case 1: (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lanes_fleet_kernel<Q, kIdxBuf, true>,
-                                                               kBlockThreads, 0); break;
-    case 2: (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lanes_fleet_kernel<Q, kIdx32, false>,
-                                                               kBlockThreads, 0); break;
-    case 3: (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lanes_fleet_kernel<Q, kIdx32, true>,
-                                                               kBlockThreads, 0); break;
-    case 4: (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lanes_fleet_kernel<Q, kIdx64, false>,
-                                                               kBlockThreads, 0); break;
-    default: (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lanes_fleet_kernel<Q, kIdx64, true>,
-                                                                kBlockThreads, 0); break;
-  }
-  return per_cu;
-}
-
-// g.clean must hold for every grid the filters name (the caller clears it
-// otherwise), and g's index kind must be at least as wide as each grid's.
-template <int Q>
-void lanes_fleet_q(const GridDev& g, const FilterDev* fs, const WorkItem* items, uint32_t nitems, uint32_t* counter,
-                   int persistent, uint32_t chunk, hipStream_t s) {
-  const int v = lanes_variant(g);
-  uint32_t blocks;
-  if (persistent) {
-    static int cus = 0, per_cu[6] = {0, 0, 0, 0, 0, 0};
-    if (!cus) {
-      int dev = 0;
-      (void)hipGetDevice(&dev);
-      (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-      for (int k = 0; k < 6; ++k) per_cu[k] = fleet_blocks_per_cu<Q>(k);
-      if (cus < 1) cus = 256;
-    }
-    blocks = (uint32_t)(cus * std::max(1, per_cu[v]));
-    if (blocks > nitems) blocks = nitems;  // one item per workgroup
-    if (blocks == 0) blocks = 1;
-    zero_u32_kernel<<<1, 64, 0, s>>>(counter, kXcds);
-  } else {
-    blocks = nitems;
-  }
-  if (blocks == 0) return;
-  const dim3 b(blocks), t(kBlockThreads);
-  const uint32_t deal = (uint32_t)current_deal();
-#define A3D_LAUNCH b, t, 0, s
-  A3D_LANES_VARIANT(v, lanes_fleet_kernel, Q, A3D_LAUNCH, g, fs, items, nitems, counter, persistent, chunk, deal)
-#undef A3D_LAUNCH
-}
-
 #undef A3D_LANES_VARIANT
-
 }  // namespace
 
 int item_particles(int mapping, int ppw) {
@@ -1369,8 +1422,6 @@ int clamp_chunk(int points) {
   return kMaxChunk;
 }
 
-bool order_pays(uint32_t n) { return current_mapping() != 0 || n > kSplit4Max; }
-
 void launch_weight(const GridDev& g, const Filters& fs, const WorkItem* d_items, uint32_t nitems,
                    uint32_t* d_counter, int ppw, int persistent, hipStream_t s) {
   ppw = clamp_ppw(ppw);
@@ -1383,16 +1434,14 @@ void launch_weight(const GridDev& g, const Filters& fs, const WorkItem* d_items,
         cloud_zrange_kernel<<<dim3(kZrParts, std::min(fs.count - base, 65535u)), kZrThreads, 0, s>>>(fs, base);
     if (!fs.arr) {
       if (fs.one.n == 0) return;
-      if (launch_split<true>(g, fs.one, nullptr, s)) return;
+      if (launch_split(g, fs.one, nullptr, s)) return;
       if (ppw == 64) lanes_single_q<1>(g, fs.one, chunk, s);
       else if (ppw == 32) lanes_single_q<2>(g, fs.one, chunk, s);
       else lanes_single_q<4>(g, fs.one, chunk, s);
       return;
     }
     if (nitems == 0) return;
-    if (ppw == 64) lanes_fleet_q<1>(g, fs.arr, d_items, nitems, d_counter, persistent, chunk, s);
-    else if (ppw == 32) lanes_fleet_q<2>(g, fs.arr, d_items, nitems, d_counter, persistent, chunk, s);
-    else lanes_fleet_q<4>(g, fs.arr, d_items, nitems, d_counter, persistent, chunk, s);
+    launch_lanes_fleet(g, fs.arr, d_items, nitems, d_counter, ppw, persistent, chunk, s);
     return;
   }
   if (!fs.arr) {
@@ -1430,7 +1479,7 @@ void launch_weight_poses(const GridDev& g, const float* cx, const float* cy, con
   if (current_mapping() == 0) {
     const uint32_t chunk = (uint32_t)clamp_chunk(current_chunk());
     if (index_kind(g) != kIdxBuf && g.seg_bits) cloud_zrange_kernel<<<dim3(kZrParts, 1), kZrThreads, 0, s>>>(single(f), 0u);
-    if (launch_split<false>(g, f, out, s)) return;
+    if (launch_split(g, f, out, s)) return;
     if (ppw == 64) lanes_poses_q<1>(g, f, out, chunk, s);
     else if (ppw == 32) lanes_poses_q<2>(g, f, out, chunk, s);
     else lanes_poses_q<4>(g, f, out, chunk, s);
@@ -1446,4 +1495,127 @@ void launch_zero_u32(uint32_t* p, uint32_t n, hipStream_t s) {
   zero_u32_kernel<<<(n + 255) / 256, 256, 0, s>>>(p, n);
 }
 
+#elif A3D_WEIGHT_PART == 1
+// The grids wider than a buffer share the 64-bit kernel (it reads every grid,
+// and takes segment loads like the 32-bit kind).
+template <int P, int W, bool KFILTER>
+void split_pw(const GridDev& g, const FilterDev& f, float* out, hipStream_t s) {
+  const dim3 b((f.n + P - 1) / P), t(Split<P, W>::kThreads);
+  if (index_kind(g) == kIdxBuf) {
+    switch (grid_mode(g)) {
+      case kFixedGrid: lanes_split_kernel<P, W, kIdxBuf, KFILTER, kFixedGrid><<<b, t, 0, s>>>(g, f, out); break;
+      case kCleanGrid: lanes_split_kernel<P, W, kIdxBuf, KFILTER, kCleanGrid><<<b, t, 0, s>>>(g, f, out); break;
+      default: lanes_split_kernel<P, W, kIdxBuf, KFILTER, kAnyGrid><<<b, t, 0, s>>>(g, f, out); break;
+    }
+  } else {
+    switch (grid_mode(g)) {
+      case kFixedGrid: lanes_split_kernel<P, W, kIdx64, KFILTER, kFixedGrid><<<b, t, 0, s>>>(g, f, out); break;
+      case kCleanGrid: lanes_split_kernel<P, W, kIdx64, KFILTER, kCleanGrid><<<b, t, 0, s>>>(g, f, out); break;
+      default: lanes_split_kernel<P, W, kIdx64, KFILTER, kAnyGrid><<<b, t, 0, s>>>(g, f, out); break;
+    }
+  }
+}
+
+// Launches of up to kSplitMax particles take the split form.  Weight kernel
+// alone, whole-cloud wavefronts of 16 against the split form at P = 4, 8, 16
+// (us, fixed-point cells; particles x points, map, spread):
+//   1,000 x 4,000 floor, tilted, 0.1 m      157    26   38   61
+//   2,000 x 4,000 floor, tilted, 0.5 m      192    47   45   73
+//   5,000 x 6,000 floor, tilted, 0.1 m      205    98   77   82
+//   5,000 x 6,000 floor, tilted, 1 m        268   130  133  154
+//   6,500 x 6,000 floor, tilted, 0.5 m      214   152  151  115
+//   12,000 x 6,000 floor, tilted, 0.1 m     208   231  153  132
+//   20,011 x 7,993 floor, tilted, 0.5 m     343   490  390  323
+//   28,000 x 5,000 floor, level, 0.1 m      177   413  262  249
+// Small P is bound by the adding wavefront (one dependent add per point, 4.6
+// ns), larger P by the gathers; from 20,000 particles on there are enough
+// whole-cloud wavefronts, which share more lines per workgroup (64 particles).
+constexpr uint32_t kSplit4Max = 2048, kSplit8Max = 5632, kSplitMax = 20480;
+
+template <bool KFILTER>
+void split_kf(const GridDev& g, const FilterDev& f, float* out, hipStream_t s) {
+  if (f.n <= kSplit4Max) split_pw<4, 4, KFILTER>(g, f, out, s);
+  else if (f.n <= kSplit8Max) split_pw<8, 4, KFILTER>(g, f, out, s);
+  else split_pw<16, 4, KFILTER>(g, f, out, s);
+}
+
+#undef A3D_LANES_VARIANT
+}  // namespace
+
+bool order_pays(uint32_t n) { return current_mapping() != 0 || n > kSplit4Max; }
+
+// A single filter's launch, or (out) explicit poses; false: too many for the
+// split form.
+bool launch_split(const GridDev& g, const FilterDev& f, float* out, hipStream_t s) {
+  if (f.n > kSplitMax) return false;
+  if (out) split_kf<false>(g, f, out, s);
+  else split_kf<true>(g, f, nullptr, s);
+  return true;
+}
+
+#else
+template <int Q>
+int fleet_blocks_per_cu(int v) {
+  int per_cu = 1;
+#define A3D_OCCUPANCY(ik, gm)                                                                                          \
+  case 3 * ik + gm:                                                                                                    \
+    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lanes_fleet_kernel<Q, ik, gm>, kBlockThreads, 0);      \
+    break;
+  switch (v) {
+    A3D_OCCUPANCY(kIdxBuf, kAnyGrid)
+    A3D_OCCUPANCY(kIdxBuf, kCleanGrid)
+    A3D_OCCUPANCY(kIdxBuf, kFixedGrid)
+    A3D_OCCUPANCY(kIdx32, kAnyGrid)
+    A3D_OCCUPANCY(kIdx32, kCleanGrid)
+    A3D_OCCUPANCY(kIdx32, kFixedGrid)
+    A3D_OCCUPANCY(kIdx64, kAnyGrid)
+    A3D_OCCUPANCY(kIdx64, kCleanGrid)
+    A3D_OCCUPANCY(kIdx64, kFixedGrid)
+  }
+#undef A3D_OCCUPANCY
+  return per_cu;
+}
+
+// g.clean and g.fixed must hold for every grid the filters name (the caller
+// clears them otherwise), and g's index kind must be at least as wide as each grid's.
+template <int Q>
+void lanes_fleet_q(const GridDev& g, const FilterDev* fs, const WorkItem* items, uint32_t nitems, uint32_t* counter,
+                   int persistent, uint32_t chunk, hipStream_t s) {
+  const int v = lanes_variant(g);
+  uint32_t blocks;
+  if (persistent) {
+    static int cus = 0, per_cu[kVariants] = {};
+    if (!cus) {
+      int dev = 0;
+      (void)hipGetDevice(&dev);
+      (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+      for (int k = 0; k < kVariants; ++k) per_cu[k] = fleet_blocks_per_cu<Q>(k);
+      if (cus < 1) cus = 256;
+    }
+    blocks = (uint32_t)(cus * std::max(1, per_cu[v]));
+    if (blocks > nitems) blocks = nitems;  // one item per workgroup
+    if (blocks == 0) blocks = 1;
+    zero_u32_kernel<<<1, 64, 0, s>>>(counter, kXcds);
+  } else {
+    blocks = nitems;
+  }
+  if (blocks == 0) return;
+  const dim3 b(blocks), t(kBlockThreads);
+  const uint32_t deal = (uint32_t)current_deal();
+#define A3D_LAUNCH b, t, 0, s
+  A3D_LANES_VARIANT(v, lanes_fleet_kernel, Q, A3D_LAUNCH, g, fs, items, nitems, counter, persistent, chunk, deal)
+#undef A3D_LAUNCH
+}
+
+#undef A3D_LANES_VARIANT
+}  // namespace
+
+void launch_lanes_fleet(const GridDev& g, const FilterDev* fs, const WorkItem* items, uint32_t nitems,
+                        uint32_t* counter, int ppw, int persistent, uint32_t chunk, hipStream_t s) {
+  if (ppw == 64) lanes_fleet_q<1>(g, fs, items, nitems, counter, persistent, chunk, s);
+  else if (ppw == 32) lanes_fleet_q<2>(g, fs, items, nitems, counter, persistent, chunk, s);
+  else lanes_fleet_q<4>(g, fs, items, nitems, counter, persistent, chunk, s);
+}
+
+#endif
 }  // namespace a3d

@@ -1,7 +1,6 @@
 """The split form of the cloud weight (a workgroup's wavefronts share the cloud,
-one more adds the values in order) at the sizes
-where its tiles, workgroups and dispatch limits end: bit-exact against
-the oracle."""
+one more adds the values in order) at the sizes where its tiles, workgroups
+and dispatch limits end: bit-exact against the oracle."""
 import numpy as np
 import pytest
 
@@ -39,7 +38,7 @@ def _poses(room, n, seed=5):
 
 
 # workgroups of 4, 8 and 16 poses, their last one ragged, and one past the split form
-@pytest.mark.parametrize("n", [1, 3, 4, 5, 2048, 2049, 8192, 8195, 28672, 28673])
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 2048, 2049, 5632, 5635, 20480, 20481])
 def test_poses_at_dispatch_limits(gpu, room, n):
     g, t = _open(gpu, room), _poses(room, n)
     cloud = room["step"].cloud[:300]
@@ -53,7 +52,7 @@ def test_poses_at_dispatch_limits(gpu, room, n):
 # around one tile (256, 128 and 64 points), two and several tiles
 @pytest.mark.parametrize("env", [None, ("A3D_FORCE_IDX64", "1"), ("A3D_FORCE_IDX64", "2"), ("A3D_FORCE_IDX32", "2"),
                                  ("A3D_FORCE_NEAR_TEST", "1")], ids=str)
-@pytest.mark.parametrize("n", [37, 2083, 8205])
+@pytest.mark.parametrize("n", [37, 2083, 5645])
 def test_poses_at_tile_edges(gpu, room, env, n, monkeypatch):
     if env:
         monkeypatch.setenv(*env)
