@@ -12,12 +12,19 @@
 //   ijk = (int)(floor(p * inv) - (float)min_b), all in float;
 //   one output point per distinct idx, in increasing idx, at the float
 //   centroid (sum of x, y, z in order, divided by the count as float).
-// Here the (idx, point) pairs are radix sorted, which is stable: the points of
-// one voxel are summed in point-index order.  PCL's std::sort leaves them in
-// an order of its own, so a centroid of three or more points can differ from
-// PCL's in the last bits; the voxel set and its order are the same.
+// Here the points of one voxel are summed in point-index order.  PCL's
+// std::sort leaves them in an order of its own, so a centroid of three or more
+// points can differ from PCL's in the last bits; the voxel set and its order
+// are the same.
+//
+// Lattices of up to kMaxLattice voxels (a 0.1 m leaf over 50 x 50 x 26 m) are
+// ranked through a bitmap, one bit per voxel: the number of marked voxels
+// below a point's is its output position, and the points are placed in their
+// voxel's list without a sort.  Larger ones (and clouds of more than
+// kMaxBitmapPoints) radix sort the (idx, point) pairs, which is stable.
 #include <hipcub/hipcub.hpp>
 
+#include <algorithm>
 #include <cfloat>
 #include <vector>
 
@@ -34,6 +41,7 @@ struct VoxelMeta {
   uint32_t nfin;
   int overflow;
   int min_b[3];
+  int div[3];
   int mul[3];
 };
 
@@ -43,71 +51,90 @@ __device__ inline const float* point_at(const uint8_t* base, size_t stride, uint
   return reinterpret_cast<const float*>(base + (size_t)i * stride);
 }
 
-// One workgroup: bounds of the finite points and the voxel lattice.
-__global__ __launch_bounds__(kVT) void voxel_meta_kernel(const uint8_t* pts, uint32_t n, size_t stride, float leaf,
-                                                         VoxelMeta* meta) {
-  __shared__ float red[6][kVT / 64];
-  __shared__ uint32_t cnt[kVT / 64];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  float mn[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, mx[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
-  uint32_t c = 0;
-  for (uint32_t i = tid; i < n; i += kVT) {
+struct VoxelBounds {
+  float lo[3], hi[3];
+  uint32_t n;
+  uint32_t pad_;
+};
+constexpr uint32_t kBoundsBlocks = 64;
+
+// Bounds and number of the finite points, per workgroup (one workgroup over all
+// of 100,000 points took 66 us, this and the lattice kernel 8 us).
+__global__ __launch_bounds__(kVT) void voxel_bounds_kernel(const uint8_t* pts, uint32_t n, size_t stride,
+                                                           VoxelBounds* out) {
+  __shared__ VoxelBounds red[kVT / 64];
+  const int lane = lane_id(), wave = threadIdx.x >> 6;
+  VoxelBounds b{{FLT_MAX, FLT_MAX, FLT_MAX}, {-FLT_MAX, -FLT_MAX, -FLT_MAX}, 0u, 0u};
+  for (uint32_t i = blockIdx.x * kVT + threadIdx.x; i < n; i += kBoundsBlocks * kVT) {
     const float* p = point_at(pts, stride, i);
     if (!finite3(p)) continue;
-    ++c;
+    ++b.n;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      mn[k] = fminf(mn[k], p[k]);
-      mx[k] = fmaxf(mx[k], p[k]);
+      b.lo[k] = fminf(b.lo[k], p[k]);
+      b.hi[k] = fmaxf(b.hi[k], p[k]);
     }
   }
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
+  auto across = [&]() {
     for (int d = 32; d >= 1; d >>= 1) {
-      mn[k] = fminf(mn[k], __shfl_xor(mn[k], d));
-      mx[k] = fmaxf(mx[k], __shfl_xor(mx[k], d));
-    }
-  }
-  for (int d = 32; d >= 1; d >>= 1) c += __shfl_xor(c, d);
-  if (lane == 0) {
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      red[k][wave] = mn[k];
-      red[3 + k][wave] = mx[k];
+      for (int k = 0; k < 3; ++k) {
+        b.lo[k] = fminf(b.lo[k], __shfl_xor(b.lo[k], d));
+        b.hi[k] = fmaxf(b.hi[k], __shfl_xor(b.hi[k], d));
+      }
+      b.n += __shfl_xor(b.n, d);
     }
-    cnt[wave] = c;
-  }
+  };
+  across();
+  if (lane == 0) red[wave] = b;
   __syncthreads();
-  if (tid != 0) return;
-  float lo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, hi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
-  uint32_t total = 0;
-  for (int w = 0; w < kVT / 64; ++w) {
+  if (wave != 0) return;
+  b = VoxelBounds{{FLT_MAX, FLT_MAX, FLT_MAX}, {-FLT_MAX, -FLT_MAX, -FLT_MAX}, 0u, 0u};
+  if (lane < kVT / 64) b = red[lane];
+  across();
+  if (lane == 0) out[blockIdx.x] = b;
+}
+
+// One wavefront: the bounds of all the workgroups, and the voxel lattice.
+__global__ __launch_bounds__(64) void voxel_meta_kernel(const VoxelBounds* part, float leaf, VoxelMeta* meta) {
+  static_assert(kBoundsBlocks == 64, "one workgroup's bounds per lane");
+  VoxelBounds b = part[threadIdx.x];
+  for (int d = 32; d >= 1; d >>= 1) {
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      lo[k] = fminf(lo[k], red[k][w]);
-      hi[k] = fmaxf(hi[k], red[3 + k][w]);
+      b.lo[k] = fminf(b.lo[k], __shfl_xor(b.lo[k], d));
+      b.hi[k] = fmaxf(b.hi[k], __shfl_xor(b.hi[k], d));
     }
-    total += cnt[w];
+    b.n += __shfl_xor(b.n, d);
   }
+  if (threadIdx.x != 0) return;
+  const float* lo = b.lo;
+  const float* hi = b.hi;
   VoxelMeta m{};
   m.inv = 1.0f / leaf;
-  m.nfin = total;
-  if (total > 0) {
+  m.nfin = b.n;
+  if (b.n > 0) {
     int64_t d[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) d[k] = (int64_t)((hi[k] - lo[k]) * m.inv) + 1;
     m.overflow = (d[0] * d[1] * d[2] > (int64_t)INT32_MAX) ? 1 : 0;
-    int div[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
       m.min_b[k] = (int)floorf(lo[k] * m.inv);
-      div[k] = (int)floorf(hi[k] * m.inv) - m.min_b[k] + 1;
+      m.div[k] = (int)floorf(hi[k] * m.inv) - m.min_b[k] + 1;
     }
     m.mul[0] = 1;
-    m.mul[1] = div[0];
-    m.mul[2] = div[0] * div[1];
+    m.mul[1] = m.div[0];
+    m.mul[2] = m.div[0] * m.div[1];
   }
   *meta = m;
+}
+
+__device__ inline uint32_t voxel_key(const VoxelMeta& m, const float* p) {
+  int ijk[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) ijk[a] = (int)(floorf(p[a] * m.inv) - (float)m.min_b[a]);
+  return (uint32_t)(ijk[0] * m.mul[0] + ijk[1] * m.mul[1] + ijk[2] * m.mul[2]);
 }
 
 __global__ void voxel_key_kernel(const uint8_t* pts, uint32_t n, size_t stride, const VoxelMeta* meta,
@@ -117,12 +144,7 @@ __global__ void voxel_key_kernel(const uint8_t* pts, uint32_t n, size_t stride, 
   const VoxelMeta m = *meta;
   const float* p = point_at(pts, stride, i);
   uint32_t k = kNoVoxel;
-  if (finite3(p)) {
-    int ijk[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) ijk[a] = (int)(floorf(p[a] * m.inv) - (float)m.min_b[a]);
-    k = (uint32_t)(ijk[0] * m.mul[0] + ijk[1] * m.mul[1] + ijk[2] * m.mul[2]);
-  }
+  if (finite3(p)) k = voxel_key(m, p);
   key[i] = k;
   val[i] = i;
 }
@@ -163,15 +185,223 @@ __global__ void voxel_copy_kernel(const uint8_t* pts, size_t stride, uint32_t n,
   oz[i] = p[2];
 }
 
+// ------------------------------------------------------------ bitmap ranking
+constexpr uint32_t kMaxLattice = 1u << 26;  // voxels: a bitmap of 8 MB and as much for its prefix
+constexpr uint32_t kRankWords = 1024;       // bitmap words per workgroup of the ranking
+constexpr uint32_t kMaxBitmapPoints = 1u << 20;
+
+__global__ void voxel_clear_kernel(uint4* p, uint32_t n) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = make_uint4(0u, 0u, 0u, 0u);
+}
+
+// Every finite point's voxel, and its bit.  Bound by the atomics (21 us for
+// 100,000 points; testing the bit before setting it measured the same).
+__global__ void voxel_mark_kernel(const uint8_t* pts, uint32_t n, size_t stride, const VoxelMeta* meta, uint32_t* key,
+                                  uint32_t* bits) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const VoxelMeta m = *meta;
+  const float* p = point_at(pts, stride, i);
+  uint32_t k = kNoVoxel;
+  if (finite3(p)) {
+    k = voxel_key(m, p);
+    atomicOr(&bits[k >> 5], 1u << (k & 31));
+  }
+  key[i] = k;
+}
+
+__device__ inline uint32_t block_sum_u(uint32_t v, uint32_t* red) {
+  for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d);
+  if (lane_id() == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  uint32_t t = 0;
+  for (uint32_t w = 0; w < blockDim.x / 64; ++w) t += red[w];
+  __syncthreads();
+  return t;
+}
+
+// Marked voxels per kRankWords words.
+__global__ __launch_bounds__(kRankWords) void voxel_count_kernel(const uint32_t* bits, uint32_t words, uint32_t* sums) {
+  __shared__ uint32_t red[kRankWords / 64];
+  const uint32_t i = blockIdx.x * kRankWords + threadIdx.x;
+  const uint32_t t = block_sum_u(i < words ? (uint32_t)__popc(bits[i]) : 0u, red);
+  if (threadIdx.x == 0) sums[blockIdx.x] = t;
+}
+
+// Marked voxels before each word; the last workgroup leaves their number.
+__global__ __launch_bounds__(kRankWords) void voxel_rank_kernel(const uint32_t* bits, uint32_t words,
+                                                                const uint32_t* sums, uint32_t* before,
+                                                                uint32_t* total) {
+  __shared__ uint32_t red[kRankWords / 64];
+  const uint32_t tid = threadIdx.x, i = blockIdx.x * kRankWords + tid;
+  const int lane = lane_id(), wave = tid >> 6;
+  uint32_t s = 0;
+  for (uint32_t b = tid; b < blockIdx.x; b += kRankWords) s += sums[b];
+  const uint32_t base = block_sum_u(s, red);
+  const uint32_t c = i < words ? (uint32_t)__popc(bits[i]) : 0u;
+  uint32_t inc = c;
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t v = __shfl_up(inc, d);
+    if (lane >= d) inc += v;
+  }
+  if (lane == 63) red[wave] = inc;
+  __syncthreads();
+  uint32_t r = base + inc - c;
+  for (int w = 0; w < wave; ++w) r += red[w];
+  if (i < words) before[i] = r;
+  if (blockIdx.x == gridDim.x - 1 && tid == kRankWords - 1) *total = r + c;
+}
+
+// Every point's output voxel (over its key) and its arrival number there.
+__global__ void voxel_tally_kernel(uint32_t* key, uint32_t n, const uint32_t* bits, const uint32_t* before,
+                                   uint32_t* count, uint32_t* slot) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t k = key[i];
+  if (k == kNoVoxel) return;
+  const uint32_t w = k >> 5, o = before[w] + (uint32_t)__popc(bits[w] & ((1u << (k & 31)) - 1u));  // < n
+  key[i] = o;
+  slot[i] = atomicAdd(&count[o], 1u);
+}
+
+// Where each voxel's list starts: a workgroup takes one range for its voxels
+// (the lists' order does not matter).
+__global__ __launch_bounds__(kVT) void voxel_alloc_kernel(const uint32_t* count, const uint32_t* total, uint32_t* start,
+                                                          uint32_t* used) {
+  __shared__ uint32_t red[kVT / 64];
+  __shared__ uint32_t base;
+  const uint32_t tid = threadIdx.x, o = blockIdx.x * kVT + tid, nv = *total;
+  const int lane = lane_id(), wave = tid >> 6;
+  if (blockIdx.x * kVT >= nv) return;  // uniform
+  const uint32_t c = o < nv ? count[o] : 0u;
+  uint32_t inc = c;
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t v = __shfl_up(inc, d);
+    if (lane >= d) inc += v;
+  }
+  if (lane == 63) red[wave] = inc;
+  __syncthreads();
+  uint32_t r = inc - c;
+  for (int w = 0; w < wave; ++w) r += red[w];
+  if (tid == kVT - 1) base = atomicAdd(used, r + c);
+  __syncthreads();
+  if (o < nv) start[o] = base + r;
+}
+
+__global__ void voxel_place_kernel(const uint32_t* voxel, uint32_t n, const uint32_t* start, const uint32_t* slot,
+                                   uint32_t* list) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const uint32_t o = voxel[i];
+  if (o != kNoVoxel) list[start[o] + slot[i]] = i;  // < n: a voxel's slots cover exactly its count
+}
+
+// The centroids.  Half a wavefront takes a voxel of up to 32 points: it orders
+// them by index (a lane's rank is the number of smaller ones) and sums them in
+// that order.  A voxel of more points is taken by the whole wavefront, which
+// ranks them the same way (c^2 / 64 steps), or, past kRankMax points or where
+// that is shorter, searches all the cloud's points for them (n / 64 steps).
+constexpr uint32_t kRankMax = 1024;
+__global__ __launch_bounds__(256) void voxel_average_kernel(const uint8_t* pts, uint32_t n, size_t stride,
+                                                            const uint32_t* voxel, const uint32_t* count,
+                                                            const uint32_t* start, const uint32_t* list,
+                                                            const uint32_t* total, float* ox, float* oy, float* oz) {
+  constexpr uint32_t kWaves = 4;
+  __shared__ float xyz[kWaves][3][kRankMax];
+  const int lane = lane_id(), l = lane & 31, half = lane >> 5;
+  const uint32_t wave = threadIdx.x >> 6, nv = *total;
+  float(&xs)[3][kRankMax] = xyz[wave];
+  auto put = [&](uint32_t at, uint32_t i) {
+    const float* p = point_at(pts, stride, i);
+    xs[0][at] = p[0];
+    xs[1][at] = p[1];
+    xs[2][at] = p[2];
+  };
+  auto sum = [&](int axis, uint32_t first, uint32_t c, uint32_t o) {
+    float s = 0.f;
+#pragma unroll 8
+    for (uint32_t j = 0; j < c; ++j) s += xs[axis][first + j];
+    float* const out = axis == 0 ? ox : axis == 1 ? oy : oz;
+    out[o] = s / (float)c;
+  };
+  for (uint32_t o2 = (blockIdx.x * kWaves + wave) * 2; o2 < nv; o2 += gridDim.x * kWaves * 2) {  // uniform
+    const uint32_t o = o2 + half;
+    const uint32_t c = o < nv ? count[o] : 0u;
+    const bool few = c <= 32;
+    const bool have = few && (uint32_t)l < c;
+    const uint32_t i = have ? list[start[o] + l] : 0xffffffffu;
+    uint32_t rank = 0;
+#pragma unroll
+    for (int j = 0; j < 32; ++j) rank += (uint32_t)__shfl((int)i, (lane & 32) + j) < i ? 1u : 0u;
+    wave_lds_sync();  // the previous voxels' reads precede these writes
+    if (have) put(half * 32 + rank, i);
+    wave_lds_sync();
+    if (few && l < 3 && o < nv) sum(l, half * 32, c, o);  // lanes 0, 1, 2: x, y, z
+    uint64_t crowded = __ballot(!few && l == 0);
+    while (crowded) {  // uniform
+      const int src = (int)__builtin_ctzll(crowded);
+      crowded &= crowded - 1;
+      const uint32_t v = (uint32_t)__builtin_amdgcn_readlane((int)o, src);
+      const uint32_t cv = (uint32_t)__builtin_amdgcn_readlane((int)c, src);
+      if (cv <= kRankMax && (uint64_t)cv * cv <= 2 * (uint64_t)n) {
+        const uint32_t* const lv = list + start[v];
+        wave_lds_sync();
+        for (uint32_t j0 = 0; j0 < cv; j0 += 64) {
+          const uint32_t mine = j0 + lane < cv ? lv[j0 + lane] : 0xffffffffu;
+          uint32_t r = 0;
+          for (uint32_t j1 = 0; j1 < cv; j1 += 64) {
+            const uint32_t other = j1 + lane < cv ? lv[j1 + lane] : 0xffffffffu;
+#pragma unroll
+            for (int j = 0; j < 64; ++j) r += (uint32_t)__builtin_amdgcn_readlane((int)other, j) < mine ? 1u : 0u;
+          }
+          if (j0 + lane < cv) put(r, mine);
+        }
+        wave_lds_sync();
+        if (lane < 3) sum(lane, 0, cv, v);
+        continue;
+      }
+      float sx = 0.f, sy = 0.f, sz = 0.f;
+      for (uint32_t j0 = 0; j0 < n; j0 += 64) {
+        const uint32_t j = j0 + lane;
+        const bool in = j < n && voxel[j] == v;
+        uint64_t m = __ballot(in);
+        if (!m) continue;
+        float x = 0.f, y = 0.f, z = 0.f;
+        if (in) {
+          const float* p = point_at(pts, stride, j);
+          x = p[0];
+          y = p[1];
+          z = p[2];
+        }
+        while (m) {
+          const int q = (int)__builtin_ctzll(m);
+          m &= m - 1;
+          sx += readlane_f(x, q);
+          sy += readlane_f(y, q);
+          sz += readlane_f(z, q);
+        }
+      }
+      if (lane == 0) {
+        ox[v] = sx / (float)cv;
+        oy[v] = sy / (float)cv;
+        oz[v] = sz / (float)cv;
+      }
+    }
+  }
+}
+
 }  // namespace
 
 // Device buffers of voxel_grid_device, kept by a caller that filters many
-// clouds: the meta record, six arrays of `cap` words (keys, values, their
-// sorted copies, voxel heads and positions) and the sort / scan temporary.
+// clouds: the meta record (with the workgroups' bounds and the voxel count
+// after it), an array of words for the path taken (bitmap ranking, or the
+// sort's keys, values, their sorted copies, voxel heads and positions) and the
+// sort / scan temporary.
 struct VoxelWorkspace {
   VoxelMeta* meta = nullptr;
   uint32_t* buf = nullptr;
-  size_t cap = 0;
+  size_t cap = 0;  // words
   void* tmp = nullptr;
   size_t tmp_cap = 0;
 };
@@ -211,9 +441,14 @@ int voxel_grid_device(const void* d_pts, size_t n, size_t stride, float leaf, fl
     cleanup();                  \
     return A3D_ERR_HIP;         \
   }
-  if (!w.meta) A3D_TRY(hipMalloc(&w.meta, sizeof(VoxelMeta)));
+  constexpr size_t kPartAt = (sizeof(VoxelMeta) + 63) & ~(size_t)63;
+  constexpr size_t kTotalAt = kPartAt + kBoundsBlocks * sizeof(VoxelBounds);
+  if (!w.meta) A3D_TRY(hipMalloc(&w.meta, kTotalAt + 64));
   VoxelMeta* const meta = w.meta;
-  voxel_meta_kernel<<<1, kVT, 0, s>>>(pts, nn, stride, leaf, meta);
+  VoxelBounds* const part = reinterpret_cast<VoxelBounds*>(reinterpret_cast<uint8_t*>(meta) + kPartAt);
+  uint32_t* const total = reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(meta) + kTotalAt);
+  voxel_bounds_kernel<<<kBoundsBlocks, kVT, 0, s>>>(pts, nn, stride, part);
+  voxel_meta_kernel<<<1, 64, 0, s>>>(part, leaf, meta);
   A3D_TRY(hipGetLastError());
   VoxelMeta hm{};
   A3D_TRY(hipMemcpyAsync(&hm, meta, sizeof(VoxelMeta), hipMemcpyDeviceToHost, s));
@@ -230,19 +465,61 @@ int voxel_grid_device(const void* d_pts, size_t n, size_t stride, float leaf, fl
     *out_n = n;
     return A3D_OK;
   }
-  if (w.cap < n) {
+  auto grow = [&](size_t words) {
+    if (w.cap >= words) return hipSuccess;
     (void)hipFree(w.buf);
     w.buf = nullptr;
     w.cap = 0;
-    A3D_TRY(hipMalloc(&w.buf, 6 * n * 4));
-    w.cap = n;
+    const hipError_t e = hipMalloc(&w.buf, words * 4);
+    if (e == hipSuccess) w.cap = words;
+    return e;
+  };
+  // The bitmap serves a lattice of at most kMaxLattice voxels whose cells are
+  // exact floats (a key is then below the lattice's size); clearing and ranking
+  // a bitmap much larger than the cloud would cost more than the sort (7.5M
+  // voxels take 5 us, 67M 20 us, the sort's extra launches 60 us).
+  const double lattice = (double)hm.div[0] * hm.div[1] * hm.div[2];
+  bool bitmap = lattice <= (double)kMaxLattice && nn <= kMaxBitmapPoints;
+  for (int k = 0; k < 3; ++k)
+    bitmap = bitmap && hm.div[k] > 0 && hm.div[k] < (1 << 24) && hm.min_b[k] > -(1 << 30) && hm.min_b[k] < (1 << 30);
+  if (bitmap) {
+    const uint32_t words = (uint32_t)(((uint64_t)lattice + 31) / 32), wp = (words + 3) & ~3u, np = (nn + 3) & ~3u;
+    const uint32_t rank_blocks = (words + kRankWords - 1) / kRankWords;
+    A3D_TRY(grow(2 * (size_t)wp + 5 * (size_t)np + 4 + rank_blocks));
+    uint32_t* const bits = w.buf;  // cleared together with used and count
+    uint32_t* const used = bits + wp;
+    uint32_t* const count = used + 4;
+    uint32_t* const before = count + np;
+    uint32_t* const voxel = before + wp;  // each point's key, then its output voxel
+    uint32_t* const slot = voxel + np;
+    uint32_t* const start = slot + np;
+    uint32_t* const list = start + np;
+    uint32_t* const sums = list + np;
+    const uint32_t clear = (wp + 4 + np) / 4;
+    voxel_clear_kernel<<<(clear + 255) / 256, 256, 0, s>>>(reinterpret_cast<uint4*>(bits), clear);
+    voxel_mark_kernel<<<blocks, 256, 0, s>>>(pts, nn, stride, meta, voxel, bits);
+    voxel_count_kernel<<<rank_blocks, kRankWords, 0, s>>>(bits, words, sums);
+    voxel_rank_kernel<<<rank_blocks, kRankWords, 0, s>>>(bits, words, sums, before, total);
+    voxel_tally_kernel<<<blocks, 256, 0, s>>>(voxel, nn, bits, before, count, slot);
+    voxel_alloc_kernel<<<(nn + kVT - 1) / kVT, kVT, 0, s>>>(count, total, start, used);
+    voxel_place_kernel<<<blocks, 256, 0, s>>>(voxel, nn, start, slot, list);
+    voxel_average_kernel<<<std::min(1024u, (nn + 7) / 8), 256, 0, s>>>(pts, nn, stride, voxel, count, start, list,
+                                                                       total, d_x, d_y, d_z);
+    A3D_TRY(hipGetLastError());
+    uint32_t nv = 0;
+    A3D_TRY(hipMemcpyAsync(&nv, total, 4, hipMemcpyDeviceToHost, s));
+    A3D_TRY(hipStreamSynchronize(s));
+    cleanup();
+    *out_n = nv;
+    return A3D_OK;
   }
+  A3D_TRY(grow(6 * n));
   key = w.buf;
-  val = key + w.cap;
-  key2 = val + w.cap;
-  val2 = key2 + w.cap;
-  head = val2 + w.cap;
-  pos = head + w.cap;
+  val = key + n;
+  key2 = val + n;
+  val2 = key2 + n;
+  head = val2 + n;
+  pos = head + n;
   voxel_key_kernel<<<blocks, 256, 0, s>>>(pts, nn, stride, meta, key, val);
   A3D_TRY(hipGetLastError());
   A3D_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp_bytes, key, key2, val, val2, (int)nn, 0, 32, s));
