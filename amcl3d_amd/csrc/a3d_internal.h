@@ -187,10 +187,11 @@ void grid_meta(const double mn[3], const double mx[3], double res, GridDev& g);
 void launch_weight(const GridDev& g, const Filters& fs, const WorkItem* d_items, uint32_t nitems,
                    uint32_t* d_counter, int ppw, int persistent, hipStream_t s);
 // Poses given explicitly (a3d_grid_cloud_weight): out[i]; zr: 2 * kZrParts
-// floats of device memory for the cloud's z ranges.
+// floats of device memory for the cloud's z ranges; ord: order_bytes(n) of
+// device memory for a visiting order of the poses, or null.
 void launch_weight_poses(const GridDev& g, const float* cx, const float* cy, const float* cz, uint32_t m,
                          const float* tx, const float* ty, const float* tz, const float* yaw, uint32_t n, float roll,
-                         float pitch, float* out, float* zr, int ppw, hipStream_t s);
+                         float pitch, float* out, float* zr, void* ord, int ppw, hipStream_t s);
 // Normalisation, blend and mean of ParticleFilter::update (ParticleFilter.cpp:150-195).
 void launch_update_tail(const GridDev& g, const Filters& fs, hipStream_t s);
 void launch_predict(const Filters& fs, hipStream_t s);
@@ -274,6 +275,35 @@ static_assert(kSumZr + 2 * kZrParts <= 32, "the z ranges must fit the 32 per-fil
 __host__ __device__ constexpr size_t scratch_floats(uint32_t n) {
   return sc_tiles(n) + (16 + 16 * 8) * kTiledSums * tiled_tiles(n);
 }
+
+// A buffer for the length of one call (pool.cpp): device memory, or pinned host
+// memory that kernels may read and write.  Give it back only when no stream
+// uses it.
+struct PoolBuf {
+  void* p = nullptr;
+  size_t bytes = 0;
+  int dev = 0;
+  bool host = false;
+};
+bool pool_take(PoolBuf& out, bool host, size_t bytes);
+void pool_give(PoolBuf& b);
+struct Pooled : PoolBuf {  // given back at the end of its scope
+  Pooled() = default;
+  Pooled(const Pooled&) = delete;
+  Pooled& operator=(const Pooled&) = delete;
+  ~Pooled() { pool_give(*this); }
+  bool take(bool on_host, size_t n) { return pool_take(*this, on_host, n); }
+  float* f() const { return static_cast<float*>(p); }
+};
+// Largest transfer that goes through a pinned buffer in one piece.
+constexpr size_t kPinnedMax = (size_t)16 << 20;
+
+// Particles between the fields' arrays (7 x n) and rows of seven.
+void launch_pack_particles(const float* soa, uint64_t n, float* rows, hipStream_t s);
+void launch_unpack_particles(const float* rows, uint64_t n, float* soa, hipStream_t s);
+// The same to and from the caller's memory, synchronously (capi.cpp).
+int read_particles(const float* soa, uint64_t n, float* rows, hipStream_t s);
+int write_particles(const float* rows, uint64_t n, float* soa, hipStream_t s);
 
 // Event pairs around the cloud-weight launches.  Completed pairs are folded
 // into acc_ms and reused as later launches take pairs, so a caller that never

@@ -184,6 +184,41 @@ inline size_t prob_alloc_bytes(const GridDev& g) {
   return (size_t)b;
 }
 
+int read_particles(const float* soa, uint64_t n, float* rows, hipStream_t s) {
+  if (!n) return A3D_OK;
+  Pooled h;
+  if (28 * n <= kPinnedMax && h.take(true, 28 * n)) {  // the kernel transposes into pinned host memory
+    launch_pack_particles(soa, n, h.f(), s);
+    const bool ok = hip_ok(hipGetLastError(), "particles");
+    if (!hip_ok(hipStreamSynchronize(s), "particles") || !ok) return A3D_ERR_HIP;
+    std::memcpy(rows, h.p, 28 * n);
+    return A3D_OK;
+  }
+  std::vector<float> v(7 * n);
+  A3D_HIP(hipMemcpyAsync(v.data(), soa, 28 * n, hipMemcpyDeviceToHost, s));
+  A3D_HIP(hipStreamSynchronize(s));
+  for (uint64_t i = 0; i < n; ++i)
+    for (int k = 0; k < 7; ++k) rows[7 * i + k] = v[k * n + i];
+  return A3D_OK;
+}
+
+int write_particles(const float* rows, uint64_t n, float* soa, hipStream_t s) {
+  if (!n) return A3D_OK;
+  Pooled h;
+  if (28 * n <= kPinnedMax && h.take(true, 28 * n)) {
+    std::memcpy(h.p, rows, 28 * n);
+    launch_unpack_particles(h.f(), n, soa, s);
+    const bool ok = hip_ok(hipGetLastError(), "particles");
+    return hip_ok(hipStreamSynchronize(s), "particles") && ok ? A3D_OK : A3D_ERR_HIP;
+  }
+  std::vector<float> v(7 * n);
+  for (uint64_t i = 0; i < n; ++i)
+    for (int k = 0; k < 7; ++k) v[k * n + i] = rows[7 * i + k];
+  A3D_HIP(hipMemcpyAsync(soa, v.data(), 28 * n, hipMemcpyHostToDevice, s));
+  A3D_HIP(hipStreamSynchronize(s));
+  return A3D_OK;
+}
+
 }  // namespace a3d
 
 using namespace a3d;
@@ -195,7 +230,8 @@ struct a3d_pf {
   float* x = nullptr;  // one allocation: x y z a w wp wr
   float* scratch = nullptr;
   uint8_t* inmap = nullptr;
-  float* mean = nullptr;
+  float* mean = nullptr;  // 4 floats of pinned host memory, written by the update's last kernel
+  PoolBuf mean_buf;
   uint32_t* idx = nullptr;
   void* ord = nullptr;     // particle visiting order buffers (order_view)
   float* stage = nullptr;  // host-input staging
@@ -319,24 +355,26 @@ int a3d_voxel_grid(const void* points, size_t n, size_t stride, float leaf, floa
   if (rc) return rc;
   *out_n = 0;
   if (n == 0) return A3D_OK;
-  void* d_in = nullptr;
-  float* d_out = nullptr;
-  if (hipMalloc(&d_in, n * stride) != hipSuccess || hipMalloc(&d_out, 3 * n * 4) != hipSuccess) {
-    (void)hipFree(d_in);
-    return fail(A3D_ERR_NOMEM, "a3d_voxel_grid: device allocation failed");
-  }
+  Pooled d;  // the scan, then the centroids
+  const size_t in = (n * stride + 255) & ~(size_t)255;
+  if (!d.take(false, in + 12 * n)) return fail(A3D_ERR_NOMEM, "a3d_voxel_grid: device allocation failed");
+  float* const d_out = reinterpret_cast<float*>(static_cast<uint8_t*>(d.p) + in);
   size_t k = 0;
-  rc = hip_ok(hipMemcpy(d_in, points, n * stride, hipMemcpyHostToDevice), "a3d_voxel_grid: upload") ? A3D_OK
-                                                                                                    : A3D_ERR_HIP;
-  if (!rc) rc = voxel_grid_device(d_in, n, stride, leaf, d_out, d_out + n, d_out + 2 * n, &k, nullptr);
-  if (!rc && k) {
-    const bool ok = hipMemcpy(out_x, d_out, k * 4, hipMemcpyDeviceToHost) == hipSuccess &&
-                    hipMemcpy(out_y, d_out + n, k * 4, hipMemcpyDeviceToHost) == hipSuccess &&
-                    hipMemcpy(out_z, d_out + 2 * n, k * 4, hipMemcpyDeviceToHost) == hipSuccess;
+  rc = hip_ok(hipMemcpy(d.p, points, n * stride, hipMemcpyHostToDevice), "a3d_voxel_grid: upload") ? A3D_OK
+                                                                                                 : A3D_ERR_HIP;
+  if (!rc) rc = voxel_grid_device(d.p, n, stride, leaf, d_out, d_out + n, d_out + 2 * n, &k, nullptr);
+  float* const out[3] = {out_x, out_y, out_z};
+  Pooled h;
+  if (!rc && k && 12 * k <= kPinnedMax && h.take(true, 12 * k)) {
+    bool ok = hipMemcpy2DAsync(h.p, 4 * k, d_out, 4 * n, 4 * k, 3, hipMemcpyDeviceToHost, nullptr) == hipSuccess;
+    ok = hipStreamSynchronize(nullptr) == hipSuccess && ok;
     if (!ok) rc = fail(A3D_ERR_HIP, "a3d_voxel_grid: download failed");
+    for (int a = 0; ok && a < 3; ++a) std::memcpy(out[a], h.f() + (size_t)a * k, 4 * k);
+  } else if (!rc && k) {
+    for (int a = 0; a < 3 && !rc; ++a)
+      if (hipMemcpy(out[a], d_out + (size_t)a * n, k * 4, hipMemcpyDeviceToHost) != hipSuccess)
+        rc = fail(A3D_ERR_HIP, "a3d_voxel_grid: download failed");
   }
-  (void)hipFree(d_in);
-  (void)hipFree(d_out);
   if (!rc) *out_n = k;
   return rc;
 }
@@ -536,6 +574,11 @@ int a3d_grid_is_into_map(const a3d_grid* g, float x, float y, float z, int* insi
   return A3D_OK;
 }
 
+// Poses are visited in a spatial order from this many evaluations on (the sort
+// takes 16 to 25 us and saves a fifth of the weight kernel).
+static constexpr double kPoseOrderMin = 3e7;
+static constexpr size_t kDirectOut = 4096;
+
 int a3d_grid_cloud_weight(const a3d_grid* g, const float* x, const float* y, const float* z, size_t m,
                           const float* tx, const float* ty, const float* tz, const float* yaw, size_t n, float roll,
                           float pitch, float* out) {
@@ -547,42 +590,42 @@ int a3d_grid_cloud_weight(const a3d_grid* g, const float* x, const float* y, con
     return A3D_OK;
   }
   if (m > 0xffffffffull || n > 0xffffffffull) return fail(A3D_ERR_ARG, "a3d_grid_cloud_weight: too large");
-  float* buf = nullptr;
-  const size_t floats = 3 * m + 5 * n + 64;
-  if (hipMalloc(&buf, floats * sizeof(float)) != hipSuccess)
+  // the inputs go over in one copy from a pinned buffer, the weights come back
+  // into it (seven copies of pageable memory cost 70 of a small call's 100 us)
+  const size_t in = 3 * m + 4 * n;
+  const bool ordered = g_order == A3D_ORDER_SPATIAL && order_pays((uint32_t)n) && (double)n * (double)m >= kPoseOrderMin;
+  const size_t dev_floats = (in + n + 64 + 63) & ~(size_t)63;  // 2 * kZrParts of the spare ones for the z ranges
+  const bool pinned = (in + n) * 4 <= kPinnedMax;
+  Pooled d, h;
+  if (!d.take(false, dev_floats * 4 + (ordered ? order_bytes((uint32_t)n) : 0)) || (pinned && !h.take(true, (in + n) * 4)))
     return fail(A3D_ERR_NOMEM, "a3d_grid_cloud_weight: staging");
-  float* cx = buf;
-  float* cy = cx + m;
-  float* cz = cy + m;
-  float* dtx = cz + m;
-  float* dty = dtx + n;
-  float* dtz = dty + n;
-  float* dya = dtz + n;
-  float* dout = dya + n;
-  float* dzr = dout + n;  // 2 * kZrParts of the 64 spare floats
-  int rc = A3D_OK;
+  const float* const src[7] = {x, y, z, tx, ty, tz, yaw};
   hipStream_t s = g->stream;
-  if (m) {
-    if (!hip_ok(hipMemcpyAsync(cx, x, m * 4, hipMemcpyHostToDevice, s), "upload") ||
-        !hip_ok(hipMemcpyAsync(cy, y, m * 4, hipMemcpyHostToDevice, s), "upload") ||
-        !hip_ok(hipMemcpyAsync(cz, z, m * 4, hipMemcpyHostToDevice, s), "upload"))
-      rc = A3D_ERR_HIP;
+  float* at = pinned ? h.f() : d.f();
+  bool ok = true;
+  for (int k = 0; k < 7; ++k) {
+    const size_t len = k < 3 ? m : n;
+    if (len && pinned) std::memcpy(at, src[k], len * 4);
+    if (len && !pinned) ok = ok && hip_ok(hipMemcpyAsync(at, src[k], len * 4, hipMemcpyHostToDevice, s), "upload");
+    at += len;
   }
-  if (!rc && (!hip_ok(hipMemcpyAsync(dtx, tx, n * 4, hipMemcpyHostToDevice, s), "upload") ||
-              !hip_ok(hipMemcpyAsync(dty, ty, n * 4, hipMemcpyHostToDevice, s), "upload") ||
-              !hip_ok(hipMemcpyAsync(dtz, tz, n * 4, hipMemcpyHostToDevice, s), "upload") ||
-              !hip_ok(hipMemcpyAsync(dya, yaw, n * 4, hipMemcpyHostToDevice, s), "upload")))
-    rc = A3D_ERR_HIP;
-  if (!rc) {
-    launch_weight_poses(g->g, cx, cy, cz, (uint32_t)m, dtx, dty, dtz, dya, (uint32_t)n, roll, pitch, dout, dzr, g_ppw,
-                        s);
-    if (!hip_ok(hipGetLastError(), "cloud weight kernel") ||
-        !hip_ok(hipMemcpyAsync(out, dout, n * 4, hipMemcpyDeviceToHost, s), "download") ||
-        !hip_ok(hipStreamSynchronize(s), "cloud weight"))
-      rc = A3D_ERR_HIP;
+  if (pinned) ok = hip_ok(hipMemcpyAsync(d.p, h.p, in * 4, hipMemcpyHostToDevice, s), "upload");
+  float* const cx = d.f();
+  float* const t = cx + 3 * m;
+  float* const dout = t + 4 * n;
+  // few weights are written straight to the host
+  float* const wout = pinned && n <= kDirectOut ? h.f() + in : dout;
+  if (ok) {
+    launch_weight_poses(g->g, cx, cx + m, cx + 2 * m, (uint32_t)m, t, t + n, t + 2 * n, t + 3 * n, (uint32_t)n, roll,
+                        pitch, wout, dout + n, ordered ? d.f() + dev_floats : nullptr, g_ppw, s);
+    ok = hip_ok(hipGetLastError(), "cloud weight kernel") &&
+         (wout != dout || hip_ok(hipMemcpyAsync(pinned ? h.f() + in : out, dout, n * 4, hipMemcpyDeviceToHost, s),
+                                 "download"));
   }
-  (void)hipFree(buf);
-  return rc;
+  // the buffers go back only once the stream is done with them
+  if (!hip_ok(hipStreamSynchronize(s), "cloud weight") || !ok) return A3D_ERR_HIP;
+  if (pinned) std::memcpy(out, h.f() + in, n * 4);
+  return A3D_OK;
 }
 
 // .grid file, Grid3d.cpp:210-275
@@ -673,6 +716,11 @@ int a3d_pf_create(a3d_pf** out) {
     delete p;
     return fail(A3D_ERR_HIP, "a3d_pf_create: cannot create a stream");
   }
+  if (!pool_take(p->mean_buf, true, 16)) {
+    (void)hipStreamDestroy(p->stream);
+    delete p;
+    return fail(A3D_ERR_NOMEM, "a3d_pf_create: cannot allocate the mean");
+  }
   *out = p;
   return A3D_OK;
 }
@@ -681,10 +729,9 @@ static void pf_free_state(a3d_pf* p) {
   (void)hipFree(p->x);
   (void)hipFree(p->scratch);
   (void)hipFree(p->inmap);
-  (void)hipFree(p->mean);
   (void)hipFree(p->idx);
   (void)hipFree(p->ord);
-  p->x = p->scratch = p->mean = nullptr;
+  p->x = p->scratch = nullptr;
   p->inmap = nullptr;
   p->idx = nullptr;
   p->ord = nullptr;
@@ -697,6 +744,7 @@ int a3d_pf_destroy(a3d_pf* p) {
   p->timing.destroy();
   pf_free_state(p);
   (void)hipFree(p->stage);
+  pool_give(p->mean_buf);
   if (p->stream) (void)hipStreamDestroy(p->stream);
   delete p;
   return A3D_OK;
@@ -709,22 +757,18 @@ static int pf_resize(a3d_pf* p, uint32_t n) {
   float* x = nullptr;
   float* sc = nullptr;
   uint8_t* in = nullptr;
-  float* mean = nullptr;
   uint32_t* idx = nullptr;
   void* ord = nullptr;
   if (hipMalloc(&x, 7 * (size_t)n * 4) != hipSuccess || hipMalloc(&sc, scratch_floats(n) * 4) != hipSuccess ||
-      hipMalloc(&in, n) != hipSuccess || hipMalloc(&mean, 4 * 4) != hipSuccess ||
-      hipMalloc(&idx, (size_t)n * 4) != hipSuccess || hipMalloc(&ord, order_bytes(n)) != hipSuccess) {
+      hipMalloc(&in, n) != hipSuccess || hipMalloc(&idx, (size_t)n * 4) != hipSuccess || hipMalloc(&ord, order_bytes(n)) != hipSuccess) {
     (void)hipFree(x);
     (void)hipFree(sc);
     (void)hipFree(in);
-    (void)hipFree(mean);
     (void)hipFree(idx);
     (void)hipFree(ord);
     return fail(A3D_ERR_NOMEM, "particle filter: cannot allocate particle state");
   }
   A3D_HIP(hipMemsetAsync(x, 0, 7 * (size_t)n * 4, p->stream));
-  A3D_HIP(hipMemsetAsync(mean, 0, 16, p->stream));
   const uint32_t keep = std::min(n, p->n);
   for (int k = 0; k < 7 && keep; ++k)
     A3D_HIP(hipMemcpyAsync(x + (size_t)k * n, p->x + (size_t)k * p->n, (size_t)keep * 4, hipMemcpyDeviceToDevice,
@@ -734,7 +778,8 @@ static int pf_resize(a3d_pf* p, uint32_t n) {
   p->x = x;
   p->scratch = sc;
   p->inmap = in;
-  p->mean = mean;
+  p->mean = static_cast<float*>(p->mean_buf.p);  // the stream is idle
+  std::fill(p->mean, p->mean + 4, 0.0f);
   p->idx = idx;
   p->ord = ord;
   p->n = n;
@@ -793,19 +838,33 @@ int a3d_pf_predict_dev(a3d_pf* p, const double mods[4], const double deltas[4], 
   return A3D_OK;
 }
 
+static constexpr uint32_t kDirectDraws = 4096;
+
 int a3d_pf_predict(a3d_pf* p, double odom_x_mod, double odom_y_mod, double odom_z_mod, double odom_a_mod,
                    double delta_x, double delta_y, double delta_z, double delta_a, const float* z4) {
   if (!p || !z4) return fail(A3D_ERR_ARG, "a3d_pf_predict: null argument");
   if (p->capturing) return fail(A3D_ERR_STATE, "a3d_pf_predict: use the _dev form during capture");
   if (!p->n) return fail(A3D_ERR_STATE, "a3d_pf_predict: filter has no particles (call init)");
-  int rc = pf_stage(p, 4 * (size_t)p->n);
-  if (rc) return rc;
-  A3D_HIP(hipMemcpyAsync(p->stage, z4, 4 * (size_t)p->n * 4, hipMemcpyHostToDevice, p->stream));
+  int rc = A3D_OK;
+  const size_t bytes = 16 * (size_t)p->n;
+  // few draws are read by the kernel straight from pinned host memory (its four
+  // loads per particle each cross the bus); more are copied first
+  Pooled h;
+  const bool pinned = bytes <= kPinnedMax && h.take(true, bytes);
+  if (pinned) std::memcpy(h.p, z4, bytes);
+  const float* draws = h.f();
+  if (!pinned || p->n > kDirectDraws) {
+    rc = pf_stage(p, 4 * (size_t)p->n);
+    if (rc) return rc;
+    A3D_HIP(hipMemcpyAsync(p->stage, pinned ? h.p : z4, bytes, hipMemcpyHostToDevice, p->stream));
+    draws = p->stage;
+  }
   const double mods[4] = {odom_x_mod, odom_y_mod, odom_z_mod, odom_a_mod};
   const double deltas[4] = {delta_x, delta_y, delta_z, delta_a};
-  rc = a3d_pf_predict_dev(p, mods, deltas, p->stage);
+  rc = a3d_pf_predict_dev(p, mods, deltas, draws);
+  const bool done = hip_ok(hipStreamSynchronize(p->stream), "a3d_pf_predict");
   if (rc) return rc;
-  A3D_HIP(hipStreamSynchronize(p->stream));
+  if (!done) return A3D_ERR_HIP;
   return A3D_OK;
 }
 
@@ -872,7 +931,7 @@ int a3d_pf_update(a3d_pf* p, const a3d_grid* g, const float* x, const float* y, 
     }
     rc = a3d_pf_set_particles(p, pp.data(), p->n);
     if (rc) return rc;
-    A3D_HIP(hipMemset(p->mean, 0, 16));
+    std::fill(p->mean, p->mean + 4, 0.0f);  // set_particles left the stream idle
     return A3D_OK;
   }
   int rc = pf_stage(p, 3 * m + 4 * nb + 16);
@@ -881,16 +940,27 @@ int a3d_pf_update(a3d_pf* p, const a3d_grid* g, const float* x, const float* y, 
   float* cy = cx + m;
   float* cz = cy + m;
   float* rg = cz + m;
-  if (m) {
-    A3D_HIP(hipMemcpyAsync(cx, x, m * 4, hipMemcpyHostToDevice, p->stream));
-    A3D_HIP(hipMemcpyAsync(cy, y, m * 4, hipMemcpyHostToDevice, p->stream));
-    A3D_HIP(hipMemcpyAsync(cz, z, m * 4, hipMemcpyHostToDevice, p->stream));
+  const size_t bytes = (3 * m + 4 * nb) * 4;
+  Pooled h;  // the cloud and the ranges go over in one copy
+  if (bytes && bytes <= kPinnedMax && h.take(true, bytes)) {
+    const float* const src[4] = {x, y, z, ranges};
+    for (int k = 0; k < 4; ++k) {
+      const size_t len = k < 3 ? m : 4 * nb;
+      if (len) std::memcpy(h.f() + (size_t)k * m, src[k], len * 4);
+    }
+    A3D_HIP(hipMemcpyAsync(cx, h.p, bytes, hipMemcpyHostToDevice, p->stream));
+  } else {
+    if (m) {
+      A3D_HIP(hipMemcpyAsync(cx, x, m * 4, hipMemcpyHostToDevice, p->stream));
+      A3D_HIP(hipMemcpyAsync(cy, y, m * 4, hipMemcpyHostToDevice, p->stream));
+      A3D_HIP(hipMemcpyAsync(cz, z, m * 4, hipMemcpyHostToDevice, p->stream));
+    }
+    if (nb) A3D_HIP(hipMemcpyAsync(rg, ranges, nb * 16, hipMemcpyHostToDevice, p->stream));
   }
-  if (nb) A3D_HIP(hipMemcpyAsync(rg, ranges, nb * 16, hipMemcpyHostToDevice, p->stream));
   rc = a3d_pf_update_dev(p, g, cx, cy, cz, m, nb ? rg : nullptr, nb, alpha, sigma, roll, pitch);
+  const bool done = hip_ok(hipStreamSynchronize(p->stream), "a3d_pf_update");
   if (rc) return rc;
-  A3D_HIP(hipStreamSynchronize(p->stream));
-  return A3D_OK;
+  return done ? A3D_OK : A3D_ERR_HIP;
 }
 
 }  // extern "C"
@@ -915,27 +985,36 @@ int pf_resample_device_u01(a3d_pf* p, const float* d_u01) {
 
 extern "C" {
 
-int a3d_pf_resample_dev(a3d_pf* p, float u01, int mode) {
+static int pf_resample(a3d_pf* p, float u01, int mode, uint32_t* idx) {
   if (!p) return fail(A3D_ERR_ARG, "a3d_pf_resample: null filter");
   if (!p->n) return fail(A3D_ERR_STATE, "a3d_pf_resample: filter has no particles (call init)");
   if (mode != A3D_RESAMPLE_REFERENCE && mode != A3D_RESAMPLE_FP64)
     return fail(A3D_ERR_ARG, "a3d_pf_resample: unknown mode");
   FilterDev f = p->dev();
   f.u01 = u01;
-  f.idx_out = p->idx;
+  f.idx_out = idx ? idx : p->idx;
   launch_resample(single(f), mode, p->prefix_valid, p->stream);
   p->prefix_valid = false;
   A3D_HIP(hipGetLastError());
   return A3D_OK;
 }
 
+int a3d_pf_resample_dev(a3d_pf* p, float u01, int mode) { return pf_resample(p, u01, mode, nullptr); }
+
 int a3d_pf_resample(a3d_pf* p, float u01, int mode, uint32_t* idx_out) {
   if (!p) return fail(A3D_ERR_ARG, "a3d_pf_resample: null filter");
   if (p->capturing) return fail(A3D_ERR_STATE, "a3d_pf_resample: use the _dev form during capture");
-  int rc = a3d_pf_resample_dev(p, u01, mode);
+  const size_t bytes = (size_t)p->n * 4;
+  Pooled h;  // the kernel writes each index once, in order, to pinned host memory
+  const bool direct = idx_out && bytes && bytes <= kPinnedMax && h.take(true, bytes);
+  int rc = pf_resample(p, u01, mode, direct ? static_cast<uint32_t*>(h.p) : nullptr);
+  if (!rc && idx_out && !direct && !hip_ok(hipMemcpyAsync(idx_out, p->idx, bytes, hipMemcpyDeviceToHost, p->stream),
+                                           "a3d_pf_resample: indices"))
+    rc = A3D_ERR_HIP;
+  const bool done = hip_ok(hipStreamSynchronize(p->stream), "a3d_pf_resample");
   if (rc) return rc;
-  if (idx_out) A3D_HIP(hipMemcpyAsync(idx_out, p->idx, (size_t)p->n * 4, hipMemcpyDeviceToHost, p->stream));
-  A3D_HIP(hipStreamSynchronize(p->stream));
+  if (!done) return A3D_ERR_HIP;
+  if (direct) std::memcpy(idx_out, h.p, bytes);
   return A3D_OK;
 }
 
@@ -951,8 +1030,8 @@ int a3d_pf_get_mean(const a3d_pf* p, float mean[4]) {
     std::fill(mean, mean + 4, 0.f);
     return A3D_OK;
   }
-  A3D_HIP(hipMemcpyAsync(mean, p->mean, 16, hipMemcpyDeviceToHost, p->stream));
   A3D_HIP(hipStreamSynchronize(p->stream));
+  std::copy(p->mean, p->mean + 4, mean);
   return A3D_OK;
 }
 
@@ -971,13 +1050,7 @@ int a3d_pf_size(const a3d_pf* p, size_t* n) {
 int a3d_pf_get_particles(const a3d_pf* p, float* p7, size_t n) {
   if (!p || (!p7 && n)) return fail(A3D_ERR_ARG, "a3d_pf_get_particles: null argument");
   if (n != p->n) return fail(A3D_ERR_ARG, "a3d_pf_get_particles: n must equal the particle count");
-  if (!n) return A3D_OK;
-  std::vector<float> soa(7 * n);
-  A3D_HIP(hipMemcpyAsync(soa.data(), p->x, 7 * n * 4, hipMemcpyDeviceToHost, p->stream));
-  A3D_HIP(hipStreamSynchronize(p->stream));
-  for (size_t i = 0; i < n; ++i)
-    for (int k = 0; k < 7; ++k) p7[7 * i + k] = soa[k * n + i];
-  return A3D_OK;
+  return read_particles(p->x, n, p7, p->stream);
 }
 
 int a3d_pf_set_particles(a3d_pf* p, const float* p7, size_t n) {
@@ -986,11 +1059,8 @@ int a3d_pf_set_particles(a3d_pf* p, const float* p7, size_t n) {
   if (n > 0xffffffffull) return fail(A3D_ERR_ARG, "a3d_pf_set_particles: too many particles");
   int rc = pf_resize(p, (uint32_t)n);
   if (rc) return rc;
-  std::vector<float> soa(7 * n);
-  for (size_t i = 0; i < n; ++i)
-    for (int k = 0; k < 7; ++k) soa[k * n + i] = p7[7 * i + k];
-  A3D_HIP(hipMemcpyAsync(p->x, soa.data(), 7 * n * 4, hipMemcpyHostToDevice, p->stream));
-  A3D_HIP(hipStreamSynchronize(p->stream));
+  rc = write_particles(p7, n, p->x, p->stream);
+  if (rc) return rc;
   p->initialized = true;
   p->prefix_valid = false;
   return A3D_OK;

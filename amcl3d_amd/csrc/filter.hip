@@ -1740,9 +1740,27 @@ __global__ void gather_means_kernel(Filters fs, float* out) {
   for (int k = 0; k < 4; ++k) out[4 * (size_t)i + k] = f.mean[k];
 }
 
+// Rows of seven fields, one float per thread: the rows' side, which may be
+// host memory, is read and written in order.
+__global__ void pack_particles_kernel(const float* soa, uint64_t n, float* rows) {
+  const uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e < 7 * n) rows[e] = soa[(e % 7) * n + e / 7];
+}
+__global__ void unpack_particles_kernel(const float* rows, uint64_t n, float* soa) {
+  const uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e < 7 * n) soa[(e % 7) * n + e / 7] = rows[e];
+}
+
 inline dim3 ew_grid(const Filters& fs) { return dim3((fs.max_n + kEw - 1) / kEw, fs.count); }
 
 }  // namespace
+
+void launch_pack_particles(const float* soa, uint64_t n, float* rows, hipStream_t s) {
+  if (n) pack_particles_kernel<<<(uint32_t)((7 * n + kEw - 1) / kEw), kEw, 0, s>>>(soa, n, rows);
+}
+void launch_unpack_particles(const float* rows, uint64_t n, float* soa, hipStream_t s) {
+  if (n) unpack_particles_kernel<<<(uint32_t)((7 * n + kEw - 1) / kEw), kEw, 0, s>>>(rows, n, soa);
+}
 
 void launch_gather_means(const Filters& fs, float* out, hipStream_t s) {
   if (fs.count == 0) return;

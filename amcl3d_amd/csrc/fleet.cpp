@@ -269,11 +269,7 @@ int a3d_fleet_destroy(a3d_fleet* fl) {
 int a3d_fleet_set_particles(a3d_fleet* fl, const float* p7) {
   if (!fl || !p7) return fail(A3D_ERR_ARG, "a3d_fleet_set_particles: null argument");
   if (int rc = refuse_capture(fl, "a3d_fleet_set_particles")) return rc;
-  std::vector<float> soa(7 * fl->total);
-  for (uint64_t i = 0; i < fl->total; ++i)
-    for (int k = 0; k < 7; ++k) soa[k * fl->total + i] = p7[7 * i + k];
-  A3D_HIP(hipMemcpyAsync(fl->state, soa.data(), soa.size() * 4, hipMemcpyHostToDevice, fl->stream));
-  A3D_HIP(hipStreamSynchronize(fl->stream));
+  if (int rc = write_particles(p7, fl->total, fl->state, fl->stream)) return rc;
   fl->prefix_valid = false;
   return A3D_OK;
 }
@@ -281,12 +277,7 @@ int a3d_fleet_set_particles(a3d_fleet* fl, const float* p7) {
 int a3d_fleet_get_particles(const a3d_fleet* fl, float* p7) {
   if (!fl || !p7) return fail(A3D_ERR_ARG, "a3d_fleet_get_particles: null argument");
   if (int rc = refuse_capture(fl, "a3d_fleet_get_particles")) return rc;
-  std::vector<float> soa(7 * fl->total);
-  A3D_HIP(hipMemcpyAsync(soa.data(), fl->state, soa.size() * 4, hipMemcpyDeviceToHost, fl->stream));
-  A3D_HIP(hipStreamSynchronize(fl->stream));
-  for (uint64_t i = 0; i < fl->total; ++i)
-    for (int k = 0; k < 7; ++k) p7[7 * i + k] = soa[k * fl->total + i];
-  return A3D_OK;
+  return read_particles(fl->state, fl->total, p7, fl->stream);
 }
 
 int a3d_fleet_init(a3d_fleet* fl, const float* poses, const float* devs, const float* z4) {

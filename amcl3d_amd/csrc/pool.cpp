@@ -1,0 +1,95 @@
+// Buffers for the length of one call: device memory and pinned host memory that
+// kernels read and write directly.  hipMalloc, hipFree and pinning cost tens of
+// microseconds each, as much as the smallest calls' kernels, so a returned
+// buffer is kept for the next call of any thread, as long as the idle buffers of
+// its kind fit kIdleMax; a buffer is given back only once no stream uses it.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <mutex>
+#include <vector>
+
+#include "a3d_internal.h"
+
+namespace a3d {
+namespace {
+
+constexpr size_t kSmallest = 4096;
+constexpr size_t kStep = (size_t)16 << 20;
+constexpr size_t kIdleMax[2] = {(size_t)256 << 20, (size_t)64 << 20};  // device, host
+
+struct Pool {
+  std::mutex mu;
+  std::vector<PoolBuf> idle;
+  size_t bytes[2] = {0, 0};
+};
+// never destroyed: buffers may come back while the process ends
+Pool& pool() {
+  static Pool* p = new Pool();
+  return *p;
+}
+
+void release(const PoolBuf& b) {
+  if (b.host)
+    (void)hipHostFree(b.p);
+  else
+    (void)hipFree(b.p);
+}
+
+hipError_t fresh(PoolBuf& b) { return b.host ? hipHostMalloc(&b.p, b.bytes, hipHostMallocDefault) : hipMalloc(&b.p, b.bytes); }
+
+}  // namespace
+
+bool pool_take(PoolBuf& out, bool host, size_t bytes) {
+  PoolBuf b{};
+  b.host = host;
+  b.bytes = kSmallest;  // powers of two, then whole steps of kStep
+  while (b.bytes < bytes && b.bytes < kStep) b.bytes *= 2;
+  if (bytes > kStep) b.bytes = (bytes + kStep - 1) / kStep * kStep;
+  if (hipGetDevice(&b.dev) != hipSuccess) return false;
+  Pool& P = pool();
+  {
+    std::lock_guard<std::mutex> lock(P.mu);
+    for (size_t i = P.idle.size(); i-- > 0;) {
+      const PoolBuf& c = P.idle[i];
+      if (c.host == host && c.dev == b.dev && c.bytes == b.bytes) {
+        out = c;
+        P.bytes[host] -= c.bytes;
+        P.idle.erase(P.idle.begin() + (ptrdiff_t)i);
+        return true;
+      }
+    }
+  }
+  if (fresh(b) != hipSuccess) {  // give the idle ones back and try again
+    (void)hipGetLastError();
+    std::vector<PoolBuf> drop;
+    {
+      std::lock_guard<std::mutex> lock(P.mu);
+      drop.swap(P.idle);
+      P.bytes[0] = P.bytes[1] = 0;
+    }
+    for (const PoolBuf& c : drop) release(c);
+    b.p = nullptr;
+    if (fresh(b) != hipSuccess) return false;
+  }
+  out = b;
+  return true;
+}
+
+void pool_give(PoolBuf& b) {
+  if (!b.p) return;
+  Pool& P = pool();
+  {
+    std::lock_guard<std::mutex> lock(P.mu);
+    if (P.bytes[b.host] + b.bytes <= kIdleMax[b.host]) {
+      P.idle.push_back(b);
+      P.bytes[b.host] += b.bytes;
+      b.p = nullptr;
+      return;
+    }
+  }
+  release(b);
+  b.p = nullptr;
+}
+
+}  // namespace a3d

@@ -96,7 +96,8 @@ __global__ __launch_bounds__(kVT) void voxel_bounds_kernel(const uint8_t* pts, u
 }
 
 // One wavefront: the bounds of all the workgroups, and the voxel lattice.
-__global__ __launch_bounds__(64) void voxel_meta_kernel(const VoxelBounds* part, float leaf, VoxelMeta* meta) {
+__global__ __launch_bounds__(64) void voxel_meta_kernel(const VoxelBounds* part, float leaf, VoxelMeta* meta,
+                                                        VoxelMeta* host) {
   static_assert(kBoundsBlocks == 64, "one workgroup's bounds per lane");
   VoxelBounds b = part[threadIdx.x];
   for (int d = 32; d >= 1; d >>= 1) {
@@ -128,6 +129,7 @@ __global__ __launch_bounds__(64) void voxel_meta_kernel(const VoxelBounds* part,
     m.mul[2] = m.div[0] * m.div[1];
   }
   *meta = m;
+  *host = m;
 }
 
 __device__ inline uint32_t voxel_key(const VoxelMeta& m, const float* p) {
@@ -232,7 +234,7 @@ __global__ __launch_bounds__(kRankWords) void voxel_count_kernel(const uint32_t*
 // Marked voxels before each word; the last workgroup leaves their number.
 __global__ __launch_bounds__(kRankWords) void voxel_rank_kernel(const uint32_t* bits, uint32_t words,
                                                                 const uint32_t* sums, uint32_t* before,
-                                                                uint32_t* total) {
+                                                                uint32_t* total, uint32_t* host_total) {
   __shared__ uint32_t red[kRankWords / 64];
   const uint32_t tid = threadIdx.x, i = blockIdx.x * kRankWords + tid;
   const int lane = lane_id(), wave = tid >> 6;
@@ -250,7 +252,7 @@ __global__ __launch_bounds__(kRankWords) void voxel_rank_kernel(const uint32_t* 
   uint32_t r = base + inc - c;
   for (int w = 0; w < wave; ++w) r += red[w];
   if (i < words) before[i] = r;
-  if (blockIdx.x == gridDim.x - 1 && tid == kRankWords - 1) *total = r + c;
+  if (blockIdx.x == gridDim.x - 1 && tid == kRankWords - 1) *total = *host_total = r + c;
 }
 
 // Every point's output voxel (over its key) and its arrival number there.
@@ -393,28 +395,18 @@ __global__ __launch_bounds__(256) void voxel_average_kernel(const uint8_t* pts, 
 
 }  // namespace
 
-// Device buffers of voxel_grid_device, kept by a caller that filters many
-// clouds: the meta record (with the workgroups' bounds and the voxel count
-// after it), an array of words for the path taken (bitmap ranking, or the
-// sort's keys, values, their sorted copies, voxel heads and positions) and the
-// sort / scan temporary.
+// Buffers of voxel_grid_device, kept by a caller that filters many clouds: the
+// meta record (with the workgroups' bounds and the voxel count after it), the
+// host's copy of the record and the count, the words of the path taken (bitmap
+// ranking, or the sort's keys, values, their sorted copies, voxel heads and
+// positions) and the sort / scan temporary.
 struct VoxelWorkspace {
-  VoxelMeta* meta = nullptr;
-  uint32_t* buf = nullptr;
-  size_t cap = 0;  // words
-  void* tmp = nullptr;
-  size_t tmp_cap = 0;
+  Pooled meta, host, buf, tmp;
 };
 
 VoxelWorkspace* voxel_workspace_new() { return new VoxelWorkspace(); }
 
-void voxel_workspace_free(VoxelWorkspace* w) {
-  if (!w) return;
-  (void)hipFree(w->meta);
-  (void)hipFree(w->buf);
-  (void)hipFree(w->tmp);
-  delete w;
-}
+void voxel_workspace_free(VoxelWorkspace* w) { delete w; }
 
 // d_pts: n points, `stride` bytes apart (x, y, z the first three floats).
 // Writes the filtered cloud as d_x, d_y, d_z (capacity n) and its size.
@@ -430,50 +422,44 @@ int voxel_grid_device(const void* d_pts, size_t n, size_t stride, float leaf, fl
   VoxelWorkspace& w = ws ? *ws : local;
   uint32_t *key = nullptr, *val = nullptr, *key2 = nullptr, *val2 = nullptr, *head = nullptr, *pos = nullptr;
   size_t tmp_bytes = 0, tmp2 = 0;
-  auto cleanup = [&]() {
-    if (ws) return;
-    (void)hipFree(local.meta);
-    (void)hipFree(local.buf);
-    (void)hipFree(local.tmp);
-  };
-#define A3D_TRY(call)           \
-  if (!hip_ok((call), #call)) { \
-    cleanup();                  \
-    return A3D_ERR_HIP;         \
+  // Every return leaves the stream idle: a buffer that goes back to the pool
+  // is not in use.
+#define A3D_TRY(call)               \
+  if (!hip_ok((call), #call)) {     \
+    (void)hipStreamSynchronize(s);  \
+    return A3D_ERR_HIP;             \
   }
+  // grown only while the stream is idle
+  auto grow = [](Pooled& b, bool host, size_t bytes) {
+    if (b.p && b.bytes >= bytes) return hipSuccess;
+    pool_give(b);
+    return b.take(host, bytes) ? hipSuccess : hipErrorOutOfMemory;
+  };
+  struct Host {
+    VoxelMeta meta;
+    uint32_t total;
+  };
   constexpr size_t kPartAt = (sizeof(VoxelMeta) + 63) & ~(size_t)63;
   constexpr size_t kTotalAt = kPartAt + kBoundsBlocks * sizeof(VoxelBounds);
-  if (!w.meta) A3D_TRY(hipMalloc(&w.meta, kTotalAt + 64));
-  VoxelMeta* const meta = w.meta;
-  VoxelBounds* const part = reinterpret_cast<VoxelBounds*>(reinterpret_cast<uint8_t*>(meta) + kPartAt);
-  uint32_t* const total = reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(meta) + kTotalAt);
+  A3D_TRY(grow(w.meta, false, kTotalAt + 64));
+  A3D_TRY(grow(w.host, true, sizeof(Host)));
+  VoxelMeta* const meta = static_cast<VoxelMeta*>(w.meta.p);
+  VoxelBounds* const part = reinterpret_cast<VoxelBounds*>(static_cast<uint8_t*>(w.meta.p) + kPartAt);
+  uint32_t* const total = reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(w.meta.p) + kTotalAt);
+  Host* const host = static_cast<Host*>(w.host.p);
   voxel_bounds_kernel<<<kBoundsBlocks, kVT, 0, s>>>(pts, nn, stride, part);
-  voxel_meta_kernel<<<1, 64, 0, s>>>(part, leaf, meta);
+  voxel_meta_kernel<<<1, 64, 0, s>>>(part, leaf, meta, &host->meta);
   A3D_TRY(hipGetLastError());
-  VoxelMeta hm{};
-  A3D_TRY(hipMemcpyAsync(&hm, meta, sizeof(VoxelMeta), hipMemcpyDeviceToHost, s));
   A3D_TRY(hipStreamSynchronize(s));
-  if (hm.nfin == 0) {
-    cleanup();
-    return A3D_OK;
-  }
+  const VoxelMeta hm = host->meta;
+  if (hm.nfin == 0) return A3D_OK;
   if (hm.overflow) {  // PCL: integer indices would overflow, output = input
     voxel_copy_kernel<<<blocks, 256, 0, s>>>(pts, stride, nn, d_x, d_y, d_z);
     A3D_TRY(hipGetLastError());
     A3D_TRY(hipStreamSynchronize(s));
-    cleanup();
     *out_n = n;
     return A3D_OK;
   }
-  auto grow = [&](size_t words) {
-    if (w.cap >= words) return hipSuccess;
-    (void)hipFree(w.buf);
-    w.buf = nullptr;
-    w.cap = 0;
-    const hipError_t e = hipMalloc(&w.buf, words * 4);
-    if (e == hipSuccess) w.cap = words;
-    return e;
-  };
   // The bitmap serves a lattice of at most kMaxLattice voxels whose cells are
   // exact floats (a key is then below the lattice's size); clearing and ranking
   // a bitmap much larger than the cloud would cost more than the sort (7.5M
@@ -485,8 +471,8 @@ int voxel_grid_device(const void* d_pts, size_t n, size_t stride, float leaf, fl
   if (bitmap) {
     const uint32_t words = (uint32_t)(((uint64_t)lattice + 31) / 32), wp = (words + 3) & ~3u, np = (nn + 3) & ~3u;
     const uint32_t rank_blocks = (words + kRankWords - 1) / kRankWords;
-    A3D_TRY(grow(2 * (size_t)wp + 5 * (size_t)np + 4 + rank_blocks));
-    uint32_t* const bits = w.buf;  // cleared together with used and count
+    A3D_TRY(grow(w.buf, false, (2 * (size_t)wp + 5 * (size_t)np + 4 + rank_blocks) * 4));
+    uint32_t* const bits = static_cast<uint32_t*>(w.buf.p);  // cleared together with used and count
     uint32_t* const used = bits + wp;
     uint32_t* const count = used + 4;
     uint32_t* const before = count + np;
@@ -499,22 +485,19 @@ int voxel_grid_device(const void* d_pts, size_t n, size_t stride, float leaf, fl
     voxel_clear_kernel<<<(clear + 255) / 256, 256, 0, s>>>(reinterpret_cast<uint4*>(bits), clear);
     voxel_mark_kernel<<<blocks, 256, 0, s>>>(pts, nn, stride, meta, voxel, bits);
     voxel_count_kernel<<<rank_blocks, kRankWords, 0, s>>>(bits, words, sums);
-    voxel_rank_kernel<<<rank_blocks, kRankWords, 0, s>>>(bits, words, sums, before, total);
+    voxel_rank_kernel<<<rank_blocks, kRankWords, 0, s>>>(bits, words, sums, before, total, &host->total);
     voxel_tally_kernel<<<blocks, 256, 0, s>>>(voxel, nn, bits, before, count, slot);
     voxel_alloc_kernel<<<(nn + kVT - 1) / kVT, kVT, 0, s>>>(count, total, start, used);
     voxel_place_kernel<<<blocks, 256, 0, s>>>(voxel, nn, start, slot, list);
     voxel_average_kernel<<<std::min(1024u, (nn + 7) / 8), 256, 0, s>>>(pts, nn, stride, voxel, count, start, list,
                                                                        total, d_x, d_y, d_z);
     A3D_TRY(hipGetLastError());
-    uint32_t nv = 0;
-    A3D_TRY(hipMemcpyAsync(&nv, total, 4, hipMemcpyDeviceToHost, s));
     A3D_TRY(hipStreamSynchronize(s));
-    cleanup();
-    *out_n = nv;
+    *out_n = host->total;
     return A3D_OK;
   }
-  A3D_TRY(grow(6 * n));
-  key = w.buf;
+  A3D_TRY(grow(w.buf, false, 6 * n * 4));
+  key = static_cast<uint32_t*>(w.buf.p);
   val = key + n;
   key2 = val + n;
   val2 = key2 + n;
@@ -525,14 +508,8 @@ int voxel_grid_device(const void* d_pts, size_t n, size_t stride, float leaf, fl
   A3D_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp_bytes, key, key2, val, val2, (int)nn, 0, 32, s));
   A3D_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp2, head, pos, (int)nn, s));
   tmp_bytes = std::max(tmp_bytes, tmp2);
-  if (w.tmp_cap < tmp_bytes) {
-    (void)hipFree(w.tmp);
-    w.tmp = nullptr;
-    w.tmp_cap = 0;
-    A3D_TRY(hipMalloc(&w.tmp, tmp_bytes));
-    w.tmp_cap = tmp_bytes;
-  }
-  void* const tmp = w.tmp;
+  A3D_TRY(grow(w.tmp, false, std::max(tmp_bytes, (size_t)1)));
+  void* const tmp = w.tmp.p;
   A3D_TRY(hipcub::DeviceRadixSort::SortPairs(tmp, tmp_bytes, key, key2, val, val2, (int)nn, 0, 32, s));
   voxel_head_kernel<<<blocks, 256, 0, s>>>(key2, nn, head);
   A3D_TRY(hipGetLastError());
@@ -544,7 +521,6 @@ int voxel_grid_device(const void* d_pts, size_t n, size_t stride, float leaf, fl
   A3D_TRY(hipMemcpyAsync(&last[1], head + (nn - 1), 4, hipMemcpyDeviceToHost, s));
   A3D_TRY(hipStreamSynchronize(s));
 #undef A3D_TRY
-  cleanup();
   *out_n = (size_t)last[0] + last[1];
   return A3D_OK;
 }

@@ -1459,7 +1459,7 @@ void launch_weight(const GridDev& g, const Filters& fs, const WorkItem* d_items,
 
 void launch_weight_poses(const GridDev& g, const float* cx, const float* cy, const float* cz, uint32_t m,
                          const float* tx, const float* ty, const float* tz, const float* yaw, uint32_t n, float roll,
-                         float pitch, float* out, float* zr, int ppw, hipStream_t s) {
+                         float pitch, float* out, float* zr, void* ord, int ppw, hipStream_t s) {
   if (n == 0) return;
   FilterDev f{};
   f.zr = zr;
@@ -1476,6 +1476,11 @@ void launch_weight_poses(const GridDev& g, const float* cx, const float* cy, con
   f.pitch = pitch;
   f.rp0 = (roll == 0.0f && pitch == 0.0f) ? 1u : 0u;
   ppw = clamp_ppw(ppw);
+  if (ord) {
+    const OrderDev o = order_view(ord, n);
+    launch_order(f, o, s);
+    f.order = o.order;
+  }
   if (current_mapping() == 0) {
     const uint32_t chunk = (uint32_t)clamp_chunk(current_chunk());
     if (index_kind(g) != kIdxBuf && g.seg_bits) cloud_zrange_kernel<<<dim3(kZrParts, 1), kZrThreads, 0, s>>>(single(f), 0u);
