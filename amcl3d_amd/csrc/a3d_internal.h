@@ -144,6 +144,7 @@ struct Filters {
   uint32_t count;        // number of filters
   uint32_t max_n;        // largest particle count
   const float* u01;      // optional device array: resample uniform of filter i
+  uint32_t own_grids;    // some filter of arr names its own grid (FilterDev::gdev)
   FilterDev one;         // used when arr == null
 };
 
@@ -244,6 +245,10 @@ int current_ppw();
 // Points per LDS cloud tile of the particle-lane kernels (32, 64, 128, 256).
 int clamp_chunk(int points);
 int current_chunk();
+// The same for a single filter or explicit poses: 256 unless the caller has set
+// a tile (100,000 x 20,000: 1,446 us against 1,530 at 64; no other shape
+// measured slower with it).
+int single_chunk();
 // Work-list dealing of persistent (fleet, served) launches: 0 contiguous
 // ranges per XCD, k > 0 runs of k items dealt round-robin.
 int current_deal();

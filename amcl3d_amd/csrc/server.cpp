@@ -317,6 +317,7 @@ bool a3d_server::launch(Slot& s) {
   fs.arr = s.d_filters;
   fs.count = (uint32_t)nf;
   fs.max_n = max_n;
+  fs.own_grids = mixed ? 1u : 0u;
   launch_draws(fs, s.d_seedstep, s.d_seedstep + nf, s.d_u01, st);
   launch_predict(fs, st);
   // the launch's grid: the widest index kind any map of the batch needs

@@ -37,8 +37,9 @@ __device__ float a3d_struct_load_f32(__amdgpu_buffer_rsrc_t r, int vindex, int v
 
 namespace a3d {
 
-bool launch_split(const GridDev& g, const FilterDev& f, float* out, hipStream_t s);
-void launch_lanes_fleet(const GridDev& g, const FilterDev* fs, const WorkItem* items, uint32_t nitems,
+uint32_t split_first(uint32_t n, uint32_t m, uint32_t per_block);
+void launch_split(const GridDev& g, const FilterDev& f, uint32_t first, float* out, hipStream_t s);
+void launch_lanes_fleet(const GridDev& g, const FilterDev* fs, bool own_grids, const WorkItem* items, uint32_t nitems,
                         uint32_t* counter, int ppw, int persistent, uint32_t chunk, hipStream_t s);
 
 namespace {
@@ -571,10 +572,8 @@ __device__ __forceinline__ float group_member(float v) {
 // Points per cloud tile staged in LDS (the tile shape's second dimension,
 // chosen at launch: 32, 64, 128 or 256): the workgroup loads a tile with one
 // coalesced load per thread and array, then every step reads its point with
-// one LDS read.  Per-wavefront staging (work items of different filters in
-// one workgroup) uses tiles of 64.
+// one LDS read.
 constexpr int kMaxChunk = 256;
-constexpr int kWaveChunk = 64;
 
 // Steps whose gathers a wavefront issues together (a group).
 template <int Q>
@@ -658,23 +657,25 @@ __device__ inline float4 cloud_point(const FilterDev& f, uint32_t j) {
   return stage_point<RP0>(ok ? x : kOutside, ok ? y : 0.0f, ok ? z : 0.0f);
 }
 
-// One lane's particle over the whole cloud.  BLOCK: the workgroup's
-// wavefronts (all on the same filter) walk the cloud together: tiles of
-// `chunk` points (a multiple of 32, at most kMaxChunk and at most the
-// workgroup's thread count) are staged once per workgroup in LDS (double
-// buffered, one barrier per tile), so the wavefronts' nearby poses gather the
-// same points at the same time and share cache lines; every wavefront of the
-// workgroup must call this (run = false skips the arithmetic of a wavefront
-// with no active particle).  Otherwise each wavefront stages its own tiles of
-// kWaveChunk points (work-queue kernels whose wavefronts hold different
-// filters).
-template <int Q, bool RP0, int IK, int MODE, bool BLOCK>
+// Stages point j of the cloud (past its end: the outside point).
+template <bool RP0>
+__device__ __forceinline__ float4 stage_at(const FilterDev& f, uint32_t j) {
+  return j < f.m ? cloud_point<RP0>(f, j) : stage_point<RP0>(kOutside, 0.0f, 0.0f);
+}
+
+// One lane's particle over the whole cloud.  The workgroup's wavefronts (all
+// on the same filter) walk the cloud together: tiles of `chunk` points (a
+// multiple of 32, at most kMaxChunk and at most the workgroup's thread count)
+// are staged once per workgroup in LDS (double buffered, one barrier per tile),
+// so the wavefronts' nearby poses gather the same points at the same time and
+// share cache lines; every wavefront of the workgroup must call this (run =
+// false skips the arithmetic of a wavefront with no active particle).  The last
+// tile's points end with whole groups of steps, its rest outside the map.
+template <int Q, bool RP0, int IK, int MODE>
 __device__ __forceinline__ void lanes_loop(const GridDev& g, const FilterDev& f, const LanePose& lp, float& wsum,
                                            int& cnt, float4* cl, bool run, uint32_t chunk, uint32_t segk) {
-  using Idx = typename ProbSrc<IK>::Idx;
   const ProbSrc<IK> src(g, segk);
-  const int lane = lane_id();
-  const int po = lane % Q;
+  const int po = lane_id() % Q;
   const uint32_t m = f.m;
   // Each lane counts its own accepted points (an integer count is order-free;
   // the caller adds the Q lanes of a particle at the end).  The float sum is
@@ -696,104 +697,63 @@ __device__ __forceinline__ void lanes_loop(const GridDev& g, const FilterDev& f,
       wsum += group_member<4, 3>(v);
     }
   };
-  if (!BLOCK) chunk = kWaveChunk;
-  const uint32_t mfull = m - m % chunk;
-  const int steps = (int)(chunk / Q);
+  constexpr uint32_t kStepPoints = kGroup<Q> * Q;  // points of a group of steps
   int full = 0;  // uniform: steps whose every lane was in the map, counted at the end
   float pend[kGroup<Q>];
 #pragma unroll
   for (int u = 0; u < kGroup<Q>; ++u) pend[u] = -0.0f;
-  if constexpr (BLOCK) {
-    const uint32_t tid = threadIdx.x;
-    if (mfull > 0) {
-      if (tid < chunk) cl[tid] = cloud_point<RP0>(f, tid);
-      __syncthreads();
-    }
-    uint32_t buf = 0;
-    for (uint32_t c0 = 0; c0 < mfull; c0 += chunk, buf ^= 1u) {
-      const float4* cur = cl + buf * chunk;
-      float4* nxt = cl + (buf ^ 1u) * chunk;
-      const bool more = c0 + chunk < mfull;
-      float4 next = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (more && tid < chunk) next = cloud_point<RP0>(f, c0 + chunk + tid);
-      if (run) lanes_chunk<Q, RP0, IK, MODE>(g, src, lp, cur, po, steps, cnt, full, pend, accumulate);
-      // every wavefront is done with the buffer written next (it read it in
-      // the previous tile, before the last barrier)
-      if (more && tid < chunk) nxt[tid] = next;
-      __syncthreads();
-    }
-  } else {
-    for (uint32_t c0 = 0; c0 < mfull; c0 += chunk) {
-      wave_lds_sync();  // the previous tile's reads precede these writes
-      cl[lane] = cloud_point<RP0>(f, c0 + lane);
-      wave_lds_sync();
-      lanes_chunk<Q, RP0, IK, MODE>(g, src, lp, cl, po, steps, cnt, full, pend, accumulate);
-    }
+  const uint32_t tid = threadIdx.x;
+  if (tid < chunk) cl[tid] = stage_at<RP0>(f, tid);
+  __syncthreads();
+  uint32_t buf = 0;
+  for (uint32_t c0 = 0; c0 < m; c0 += chunk, buf ^= 1u) {
+    const float4* cur = cl + buf * chunk;
+    float4* nxt = cl + (buf ^ 1u) * chunk;
+    const bool more = m - c0 > chunk;
+    const uint32_t len = more ? chunk : (m - c0 + kStepPoints - 1) / kStepPoints * kStepPoints;  // <= chunk
+    float4 next = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (more && tid < chunk) next = stage_at<RP0>(f, c0 + chunk + tid);
+    if (run) lanes_chunk<Q, RP0, IK, MODE>(g, src, lp, cur, po, (int)(len / Q), cnt, full, pend, accumulate);
+    // every wavefront is done with the buffer written next (it read it in
+    // the previous tile, before the last barrier)
+    if (more && tid < chunk) nxt[tid] = next;
+    __syncthreads();
   }
   if (!run) return;
   cnt += full;
 #pragma unroll
-  for (int u = 0; u < kGroup<Q>; ++u) accumulate(pend[u]);  // the last group of the last tile
-  for (uint32_t c0 = mfull; c0 < m; c0 += Q) {  // the last m mod chunk points
-    const uint32_t j = c0 + po;
-    const bool pin = j < m;
-    const uint32_t js = pin ? j : 0u;
-    // a lane past the cloud's end takes a point outside every map
-    const float4 p = stage_point<RP0>(pin ? f.cx[js] : kOutside, f.cy[js], f.cz[js]);
-    uint64_t vm;
-    bool nr;
-    Idx idx;
-    if constexpr (MODE == kFixed) {
-      uint32_t lo;
-      idx = cell_fixed<RP0, IK>(g, lp, p, vm, lo);
-      idx = keep_in_map<IK>(src, vm, idx);
-      nr = lo < g.fx_near;
-    } else {
-      idx = cell_fast<RP0, IK, MODE>(g, src, lp, p, vm, nr);
-    }
-    cnt = add_mask_bit(cnt, vm);
-    if ((MODE == kWindow || MODE == kFixed) && __builtin_expect(__builtin_amdgcn_ballot_w64(nr) != 0, 0)) {
-      if (nr) {
-        bool ve;
-        const Idx ie = MODE == kFixed ? cell_redo<RP0, IK>(g, src, lp, p, ve) : cell_exact<RP0, IK>(g, src, lp, p, ve);
-        cnt += (ve ? 1 : 0) - mask_bit(vm);
-        idx = ie;
-      }
-    }
-    accumulate(src(idx));
-  }
+  for (int u = 0; u < kGroup<Q>; ++u) accumulate(pend[u]);  // the last group
 }
 
-// The loop variant of a wavefront: uniform per wavefront; in BLOCK form
-// wavefronts of one workgroup may take different ones, each passing the same
-// barriers.
-template <int Q, int IK, int GM, bool BLOCK>
+// The loop variant of a wavefront: uniform per wavefront; wavefronts of one
+// workgroup may take different ones, each passing the same barriers.
+template <int Q, int IK, int GM>
 __device__ __forceinline__ void lanes_variant_loop(const GridDev& g, const FilterDev& f, const LanePose& lp,
                                                    float& wsum, int& cnt, float4* cl, bool run, uint32_t chunk,
                                                    uint32_t segk) {
   if constexpr (GM == kFixedGrid) {
     if (f.rp0)
-      lanes_loop<Q, true, IK, kFixed, BLOCK>(g, f, lp, wsum, cnt, cl, run, chunk, segk);
+      lanes_loop<Q, true, IK, kFixed>(g, f, lp, wsum, cnt, cl, run, chunk, segk);
     else
-      lanes_loop<Q, false, IK, kFixed, BLOCK>(g, f, lp, wsum, cnt, cl, run, chunk, segk);
+      lanes_loop<Q, false, IK, kFixed>(g, f, lp, wsum, cnt, cl, run, chunk, segk);
   } else if constexpr (GM == kCleanGrid) {
     const bool zero = __builtin_amdgcn_ballot_w64(lp.slow) != 0;
     if (f.rp0) {
       if (zero)
-        lanes_loop<Q, true, IK, kCleanZero, BLOCK>(g, f, lp, wsum, cnt, cl, run, chunk, segk);
+        lanes_loop<Q, true, IK, kCleanZero>(g, f, lp, wsum, cnt, cl, run, chunk, segk);
       else
-        lanes_loop<Q, true, IK, kClean, BLOCK>(g, f, lp, wsum, cnt, cl, run, chunk, segk);
+        lanes_loop<Q, true, IK, kClean>(g, f, lp, wsum, cnt, cl, run, chunk, segk);
     } else {
       if (zero)
-        lanes_loop<Q, false, IK, kCleanZero, BLOCK>(g, f, lp, wsum, cnt, cl, run, chunk, segk);
+        lanes_loop<Q, false, IK, kCleanZero>(g, f, lp, wsum, cnt, cl, run, chunk, segk);
       else
-        lanes_loop<Q, false, IK, kClean, BLOCK>(g, f, lp, wsum, cnt, cl, run, chunk, segk);
+        lanes_loop<Q, false, IK, kClean>(g, f, lp, wsum, cnt, cl, run, chunk, segk);
     }
   } else {
     if (f.rp0)
-      lanes_loop<Q, true, IK, kWindow, BLOCK>(g, f, lp, wsum, cnt, cl, run, chunk, segk);
+      lanes_loop<Q, true, IK, kWindow>(g, f, lp, wsum, cnt, cl, run, chunk, segk);
     else
-      lanes_loop<Q, false, IK, kWindow, BLOCK>(g, f, lp, wsum, cnt, cl, run, chunk, segk);
+      lanes_loop<Q, false, IK, kWindow>(g, f, lp, wsum, cnt, cl, run, chunk, segk);
   }
 }
 
@@ -897,10 +857,10 @@ __device__ __forceinline__ bool wave_segment(const GridDev& g, const FilterDev& 
   return __builtin_amdgcn_readfirstlane((int)seg) != 0;
 }
 
-// GM: what holds of all the launch's grids (GridMode).  BLOCK: the
-// workgroup walks the cloud together (every wavefront calls this, count may
-// be 0); cl then holds two chunks per workgroup, else one per wavefront.
-template <int Q, int IK, bool KFILTER, int GM, bool BLOCK>
+// GM: what holds of all the launch's grids (GridMode).  The workgroup walks the
+// cloud together (every wavefront calls this, count may be 0); cl holds two
+// chunks.
+template <int Q, int IK, bool KFILTER, int GM>
 __device__ void weight_lanes(const GridDev& g, const FilterDev& f, uint32_t p0, uint32_t count, float* out,
                              float4* cl, uint32_t chunk) {
   const int lane = lane_id();
@@ -917,7 +877,6 @@ __device__ void weight_lanes(const GridDev& g, const FilterDev& f, uint32_t p0, 
   }
   const bool act = KFILTER ? (has && into_map(g, tx, ty, tz)) : has;
   const bool run = __ballot(act) != 0;
-  if (!BLOCK && !run) return;
   LanePose lp;
   rotation9(f.roll, f.pitch, ta, lp.r);
   const double nan = __builtin_nan("");
@@ -934,11 +893,11 @@ __device__ void weight_lanes(const GridDev& g, const FilterDev& f, uint32_t p0, 
   if constexpr (IK != kIdxBuf) {
     uint32_t segk = 0;
     if (g.seg_bits && f.zr && wave_segment(g, f, act, lp.oz, &segk))
-      lanes_variant_loop<Q, kIdxSeg, GM, BLOCK>(g, f, lp, wsum, cnt, cl, run, chunk, segk);
+      lanes_variant_loop<Q, kIdxSeg, GM>(g, f, lp, wsum, cnt, cl, run, chunk, segk);
     else
-      lanes_variant_loop<Q, IK, GM, BLOCK>(g, f, lp, wsum, cnt, cl, run, chunk, 0u);
+      lanes_variant_loop<Q, IK, GM>(g, f, lp, wsum, cnt, cl, run, chunk, 0u);
   } else {
-    lanes_variant_loop<Q, IK, GM, BLOCK>(g, f, lp, wsum, cnt, cl, run, chunk, 0u);
+    lanes_variant_loop<Q, IK, GM>(g, f, lp, wsum, cnt, cl, run, chunk, 0u);
   }
   if (Q > 1) {
     int c = cnt;
@@ -966,7 +925,7 @@ __global__ __launch_bounds__(kBlockThreads) void lanes_single_kernel(GridDev g, 
   const uint32_t wave = xcd_block(blockIdx.x, gridDim.x) * kBlockWaves + (threadIdx.x >> 6);
   const uint32_t p0 = wave * P;
   const uint32_t count = p0 < f.n ? min(P, f.n - p0) : 0u;
-  weight_lanes<Q, IK, true, GM, true>(g, f, p0, count, nullptr, cloud, chunk);
+  weight_lanes<Q, IK, true, GM>(g, f, p0, count, nullptr, cloud, chunk);
 }
 
 template <int Q, int IK, int GM>
@@ -977,7 +936,7 @@ __global__ __launch_bounds__(kBlockThreads) void lanes_poses_kernel(GridDev g, F
   const uint32_t wave = blockIdx.x * kBlockWaves + (threadIdx.x >> 6);
   const uint32_t p0 = wave * P;
   const uint32_t count = p0 < f.n ? min(P, f.n - p0) : 0u;
-  weight_lanes<Q, IK, false, GM, true>(g, f, p0, count, out, cloud, chunk);
+  weight_lanes<Q, IK, false, GM>(g, f, p0, count, out, cloud, chunk);
 }
 
 // ---------------------------------------------------------------------------
@@ -1147,7 +1106,8 @@ __device__ __forceinline__ void split_variant(const GridDev& g, const FilterDev&
 }
 
 template <int P, int W, int IK, bool KFILTER, int GM>
-__global__ __launch_bounds__((Split<P, W>::kThreads)) void lanes_split_kernel(GridDev g, FilterDev f, float* out) {
+__global__ __launch_bounds__((Split<P, W>::kThreads)) void lanes_split_kernel(GridDev g, FilterDev f, uint32_t first,
+                                                                             float* out) {
   using S = Split<P, W>;
   constexpr int Q = S::Q;
   __shared__ float4 tiles4[2 * P * S::kRow / 4];
@@ -1156,8 +1116,8 @@ __global__ __launch_bounds__((Split<P, W>::kThreads)) void lanes_split_kernel(Gr
   const uint32_t wave = threadIdx.x >> 6;
   const int lane = lane_id();
   const bool adds = wave == W;  // the adding wavefront
-  const uint32_t p0 = xcd_block(blockIdx.x, gridDim.x) * P;
-  const uint32_t count = min((uint32_t)P, f.n - p0);  // the grid has ceil(n / P) workgroups
+  const uint32_t p0 = first + xcd_block(blockIdx.x, gridDim.x) * P;
+  const uint32_t count = min((uint32_t)P, f.n - p0);  // the grid has ceil((n - first) / P) workgroups
   const int ps = adds ? lane % P : lane / Q;
   const bool has = (uint32_t)ps < count;
   const uint32_t pk = p0 + (has ? (uint32_t)ps : 0u);
@@ -1222,53 +1182,77 @@ __global__ __launch_bounds__((Split<P, W>::kThreads)) void lanes_split_kernel(Gr
   __syncthreads();
 }
 
+// *p (the same in every lane) in scalar registers: fields read through a
+// descriptor would otherwise sit in vector registers.
+template <class T>
+__device__ __forceinline__ T uniform_copy(const T* p) {
+  static_assert(sizeof(T) % 4 == 0, "whole words");
+  uint32_t w[sizeof(T) / 4];
+  const uint32_t* const q = reinterpret_cast<const uint32_t*>(p);
+#pragma unroll
+  for (size_t k = 0; k < sizeof(T) / 4; ++k) w[k] = (uint32_t)__builtin_amdgcn_readfirstlane((int)q[k]);
+  T t;
+  __builtin_memcpy(&t, w, sizeof(T));
+  return t;
+}
+
 // One work item of up to kBlockWaves * P particles of one filter, taken by
 // a whole workgroup: wavefront w holds particles p0 + w*P .. and the
 // wavefronts walk the filter's cloud together.  A filter that names its own
 // grid (a batch over several maps) is weighted on that grid, else on the
 // launch's; the launch grid's seg_bits = 0 keeps every filter off segment
 // loads.
-template <int Q, int IK, int GM>
+template <int Q, int IK, int GM, bool OWN>
 __device__ __forceinline__ void lanes_item(const GridDev& g, const FilterDev& f, const WorkItem& it, float4* cl,
                                            uint32_t chunk) {
   constexpr uint32_t P = 64 / Q;
   const uint32_t w = threadIdx.x >> 6, p0 = it.p0 + w * P;
   const uint32_t count = (w * P < it.count) ? min(P, it.count - w * P) : 0u;
-  if (f.gdev) {
-    GridDev gf = *f.gdev;
-    if (!g.seg_bits) gf.seg_bits = 0u;  // the launch holds off segment loads
-    weight_lanes<Q, IK, true, GM, true>(gf, f, p0, count, nullptr, cl, chunk);
+  if constexpr (OWN) {
+    GridDev gf = g;
+    if (f.gdev) {
+      gf = uniform_copy(f.gdev);
+      if (!g.seg_bits) gf.seg_bits = 0u;  // the launch holds off segment loads
+    }
+    weight_lanes<Q, IK, true, GM>(gf, f, p0, count, nullptr, cl, chunk);
   } else {
-    weight_lanes<Q, IK, true, GM, true>(g, f, p0, count, nullptr, cl, chunk);
+    weight_lanes<Q, IK, true, GM>(g, f, p0, count, nullptr, cl, chunk);
   }
 }
 
 // Clean grids: at most 128 registers, four wavefronts per SIMD (the loads
 // of spread particle sets need the wavefronts to hide their latency).
-template <int Q, int IK, int GM>
+// OWN: filters may name their own grids.
+template <int Q, int IK, int GM, bool OWN>
 __global__ __launch_bounds__(kBlockThreads, GM != kAnyGrid ? 4 : 1) void lanes_fleet_kernel(GridDev g, const FilterDev* fs,
                                                                     const WorkItem* items, uint32_t nitems,
                                                                     uint32_t* counter, int persistent,
                                                                     uint32_t chunk, uint32_t deal) {
   __shared__ float4 cloud[2 * kMaxChunk];
   __shared__ uint32_t taken;
-  if (!persistent) {
-    if (blockIdx.x >= nitems) return;
-    const WorkItem it = items[blockIdx.x];
-    lanes_item<Q, IK, GM>(g, fs[it.filter], it, cloud, chunk);
-    return;
-  }
-  for (uint32_t r = 0; r < kXcds; ++r) {
-    const uint32_t x = (blockIdx.x + r) % kXcds, len = deal_len(nitems, x, deal);
-    for (;;) {
+  // one call of the item's code for both forms: two copies of it need more
+  // registers than either
+  uint32_t r = 0;
+  for (;;) {
+    uint32_t k = blockIdx.x;
+    if (persistent) {
+      const uint32_t x = (blockIdx.x + r) % kXcds, len = deal_len(nitems, x, deal);
       if (threadIdx.x == 0) taken = atomicAdd(counter + x, 1u);
       __syncthreads();
-      const uint32_t t = taken;
+      const uint32_t t = (uint32_t)__builtin_amdgcn_readfirstlane((int)taken);
       __syncthreads();  // every wavefront has read it before the next take
-      if (t >= len) break;  // uniform over the workgroup
-      const WorkItem it = items[deal_item(nitems, x, deal, t)];
-      lanes_item<Q, IK, GM>(g, fs[it.filter], it, cloud, chunk);
+      if (t >= len) {   // uniform over the workgroup
+        if (++r == kXcds) break;
+        continue;
+      }
+      k = deal_item(nitems, x, deal, t);
+    } else if (k >= nitems) {
+      break;
     }
+    const WorkItem it = items[k];
+    const FilterDev f = uniform_copy(fs + it.filter);
+    lanes_item<Q, IK, GM, OWN>(g, f, it, cloud, chunk);
+    if (!persistent) break;
   }
 }
 
@@ -1458,7 +1442,7 @@ void launch_weight(const GridDev& g, const Filters& fs, const WorkItem* d_items,
                    uint32_t* d_counter, int ppw, int persistent, hipStream_t s) {
   ppw = clamp_ppw(ppw);
   if (current_mapping() == 0) {  // lanes = particles, ppw particles per wavefront
-    const uint32_t chunk = (uint32_t)clamp_chunk(current_chunk());
+    const uint32_t chunk = (uint32_t)clamp_chunk(fs.arr ? current_chunk() : single_chunk());
     // the clouds' z ranges for the kernels' segment loads (a launch of a
     // wider index kind that allows them)
     if (index_kind(g) != kIdxBuf && g.seg_bits && (fs.arr || fs.one.n > 0))
@@ -1466,14 +1450,18 @@ void launch_weight(const GridDev& g, const Filters& fs, const WorkItem* d_items,
         cloud_zrange_kernel<<<dim3(kZrParts, std::min(fs.count - base, 65535u)), kZrThreads, 0, s>>>(fs, base);
     if (!fs.arr) {
       if (fs.one.n == 0) return;
-      if (launch_split(g, fs.one, nullptr, s)) return;
-      if (ppw == 64) lanes_single_q<1>(g, fs.one, chunk, s);
-      else if (ppw == 32) lanes_single_q<2>(g, fs.one, chunk, s);
-      else lanes_single_q<4>(g, fs.one, chunk, s);
+      // the particles below first by whole-cloud wavefronts, the others split
+      const uint32_t first = split_first(fs.one.n, fs.one.m, (uint32_t)(ppw * kBlockWaves));
+      FilterDev f = fs.one;
+      f.n = first;
+      if (first && ppw == 64) lanes_single_q<1>(g, f, chunk, s);
+      else if (first && ppw == 32) lanes_single_q<2>(g, f, chunk, s);
+      else if (first) lanes_single_q<4>(g, f, chunk, s);
+      launch_split(g, fs.one, first, nullptr, s);
       return;
     }
     if (nitems == 0) return;
-    launch_lanes_fleet(g, fs.arr, d_items, nitems, d_counter, ppw, persistent, chunk, s);
+    launch_lanes_fleet(g, fs.arr, fs.own_grids != 0, d_items, nitems, d_counter, ppw, persistent, chunk, s);
     return;
   }
   if (!fs.arr) {
@@ -1514,12 +1502,15 @@ void launch_weight_poses(const GridDev& g, const float* cx, const float* cy, con
     f.order = o.order;
   }
   if (current_mapping() == 0) {
-    const uint32_t chunk = (uint32_t)clamp_chunk(current_chunk());
+    const uint32_t chunk = (uint32_t)clamp_chunk(single_chunk());
     if (index_kind(g) != kIdxBuf && g.seg_bits) cloud_zrange_kernel<<<dim3(kZrParts, 1), kZrThreads, 0, s>>>(single(f), 0u);
-    if (launch_split(g, f, out, s)) return;
-    if (ppw == 64) lanes_poses_q<1>(g, f, out, chunk, s);
-    else if (ppw == 32) lanes_poses_q<2>(g, f, out, chunk, s);
-    else lanes_poses_q<4>(g, f, out, chunk, s);
+    const uint32_t first = split_first(n, m, (uint32_t)(ppw * kBlockWaves));
+    FilterDev whole = f;
+    whole.n = first;
+    if (first && ppw == 64) lanes_poses_q<1>(g, whole, out, chunk, s);
+    else if (first && ppw == 32) lanes_poses_q<2>(g, whole, out, chunk, s);
+    else if (first) lanes_poses_q<4>(g, whole, out, chunk, s);
+    launch_split(g, f, first, out, s);
     return;
   }
   if (ppw == 16) launch_poses_pb<16>(g, f, out, s);
@@ -1536,19 +1527,19 @@ void launch_zero_u32(uint32_t* p, uint32_t n, hipStream_t s) {
 // The grids wider than a buffer share the 64-bit kernel (it reads every grid,
 // and takes segment loads like the 32-bit kind).
 template <int P, int W, bool KFILTER>
-void split_pw(const GridDev& g, const FilterDev& f, float* out, hipStream_t s) {
-  const dim3 b((f.n + P - 1) / P), t(Split<P, W>::kThreads);
+void split_pw(const GridDev& g, const FilterDev& f, uint32_t first, float* out, hipStream_t s) {
+  const dim3 b((f.n - first + P - 1) / P), t(Split<P, W>::kThreads);
   if (index_kind(g) == kIdxBuf) {
     switch (grid_mode(g)) {
-      case kFixedGrid: lanes_split_kernel<P, W, kIdxBuf, KFILTER, kFixedGrid><<<b, t, 0, s>>>(g, f, out); break;
-      case kCleanGrid: lanes_split_kernel<P, W, kIdxBuf, KFILTER, kCleanGrid><<<b, t, 0, s>>>(g, f, out); break;
-      default: lanes_split_kernel<P, W, kIdxBuf, KFILTER, kAnyGrid><<<b, t, 0, s>>>(g, f, out); break;
+      case kFixedGrid: lanes_split_kernel<P, W, kIdxBuf, KFILTER, kFixedGrid><<<b, t, 0, s>>>(g, f, first, out); break;
+      case kCleanGrid: lanes_split_kernel<P, W, kIdxBuf, KFILTER, kCleanGrid><<<b, t, 0, s>>>(g, f, first, out); break;
+      default: lanes_split_kernel<P, W, kIdxBuf, KFILTER, kAnyGrid><<<b, t, 0, s>>>(g, f, first, out); break;
     }
   } else {
     switch (grid_mode(g)) {
-      case kFixedGrid: lanes_split_kernel<P, W, kIdx64, KFILTER, kFixedGrid><<<b, t, 0, s>>>(g, f, out); break;
-      case kCleanGrid: lanes_split_kernel<P, W, kIdx64, KFILTER, kCleanGrid><<<b, t, 0, s>>>(g, f, out); break;
-      default: lanes_split_kernel<P, W, kIdx64, KFILTER, kAnyGrid><<<b, t, 0, s>>>(g, f, out); break;
+      case kFixedGrid: lanes_split_kernel<P, W, kIdx64, KFILTER, kFixedGrid><<<b, t, 0, s>>>(g, f, first, out); break;
+      case kCleanGrid: lanes_split_kernel<P, W, kIdx64, KFILTER, kCleanGrid><<<b, t, 0, s>>>(g, f, first, out); break;
+      default: lanes_split_kernel<P, W, kIdx64, KFILTER, kAnyGrid><<<b, t, 0, s>>>(g, f, first, out); break;
     }
   }
 }
@@ -1570,10 +1561,11 @@ void split_pw(const GridDev& g, const FilterDev& f, float* out, hipStream_t s) {
 constexpr uint32_t kSplit4Max = 2048, kSplit8Max = 5632, kSplitMax = 20480;
 
 template <bool KFILTER>
-void split_kf(const GridDev& g, const FilterDev& f, float* out, hipStream_t s) {
-  if (f.n <= kSplit4Max) split_pw<4, 4, KFILTER>(g, f, out, s);
-  else if (f.n <= kSplit8Max) split_pw<8, 4, KFILTER>(g, f, out, s);
-  else split_pw<16, 4, KFILTER>(g, f, out, s);
+void split_kf(const GridDev& g, const FilterDev& f, uint32_t first, float* out, hipStream_t s) {
+  const uint32_t n = f.n - first;
+  if (n <= kSplit4Max) split_pw<4, 4, KFILTER>(g, f, first, out, s);
+  else if (n <= kSplit8Max) split_pw<8, 4, KFILTER>(g, f, first, out, s);
+  else split_pw<16, 4, KFILTER>(g, f, first, out, s);
 }
 
 #undef A3D_LANES_VARIANT
@@ -1581,22 +1573,34 @@ void split_kf(const GridDev& g, const FilterDev& f, float* out, hipStream_t s) {
 
 bool order_pays(uint32_t n) { return current_mapping() != 0 || n > kSplit4Max; }
 
-// A single filter's launch, or (out) explicit poses; false: too many for the
-// split form.
-bool launch_split(const GridDev& g, const FilterDev& f, float* out, hipStream_t s) {
-  if (f.n > kSplitMax) return false;
-  if (out) split_kf<false>(g, f, out, s);
-  else split_kf<true>(g, f, nullptr, s);
-  return true;
+// Whole-cloud workgroups of per_block particles last as long as the cloud: one
+// more of them per CU than fits evenly (256 CUs) costs the launch a whole turn
+// (98,304 particles x 20,000 points take 1,313 us, 100,000 took 1,529). So up to
+// kSplit4Max particles past a whole number of turns go to the split form (92 us
+// for these 1,696), for clouds of kTurnPoints points or more.
+constexpr uint32_t kCus = 256, kTurnPoints = 2048;
+
+uint32_t split_first(uint32_t n, uint32_t m, uint32_t per_block) {
+  if (n <= kSplitMax) return 0;
+  const uint32_t rest = n % (kCus * per_block);
+  return rest <= kSplit4Max && m >= kTurnPoints ? n - rest : n;
+}
+
+// The particles from first on of a single filter's launch, or (out) of explicit
+// poses.
+void launch_split(const GridDev& g, const FilterDev& f, uint32_t first, float* out, hipStream_t s) {
+  if (first >= f.n) return;
+  if (out) split_kf<false>(g, f, first, out, s);
+  else split_kf<true>(g, f, first, nullptr, s);
 }
 
 #else
-template <int Q>
+template <int Q, bool OWN>
 int fleet_blocks_per_cu(int v) {
   int per_cu = 1;
 #define A3D_OCCUPANCY(ik, gm)                                                                                          \
   case 3 * ik + gm:                                                                                                    \
-    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lanes_fleet_kernel<Q, ik, gm>, kBlockThreads, 0);      \
+    (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lanes_fleet_kernel<Q, ik, gm, OWN>, kBlockThreads, 0); \
     break;
   switch (v) {
     A3D_OCCUPANCY(kIdxBuf, kAnyGrid)
@@ -1615,7 +1619,7 @@ int fleet_blocks_per_cu(int v) {
 
 // g.clean and g.fixed must hold for every grid the filters name (the caller
 // clears them otherwise), and g's index kind must be at least as wide as each grid's.
-template <int Q>
+template <int Q, bool OWN>
 void lanes_fleet_q(const GridDev& g, const FilterDev* fs, const WorkItem* items, uint32_t nitems, uint32_t* counter,
                    int persistent, uint32_t chunk, hipStream_t s) {
   const int v = lanes_variant(g);
@@ -1626,7 +1630,7 @@ void lanes_fleet_q(const GridDev& g, const FilterDev* fs, const WorkItem* items,
       int dev = 0;
       (void)hipGetDevice(&dev);
       (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-      for (int k = 0; k < kVariants; ++k) per_cu[k] = fleet_blocks_per_cu<Q>(k);
+      for (int k = 0; k < kVariants; ++k) per_cu[k] = fleet_blocks_per_cu<Q, OWN>(k);
       if (cus < 1) cus = 256;
     }
     blocks = (uint32_t)(cus * std::max(1, per_cu[v]));
@@ -1639,19 +1643,41 @@ void lanes_fleet_q(const GridDev& g, const FilterDev* fs, const WorkItem* items,
   if (blocks == 0) return;
   const dim3 b(blocks), t(kBlockThreads);
   const uint32_t deal = (uint32_t)current_deal();
-#define A3D_LAUNCH b, t, 0, s
-  A3D_LANES_VARIANT(v, lanes_fleet_kernel, Q, A3D_LAUNCH, g, fs, items, nitems, counter, persistent, chunk, deal)
+#define A3D_LAUNCH(ik, gm)                                                                                         \
+  case 3 * ik + gm:                                                                                                \
+    lanes_fleet_kernel<Q, ik, gm, OWN><<<b, t, 0, s>>>(g, fs, items, nitems, counter, persistent, chunk, deal);    \
+    break;
+  switch (v) {
+    A3D_LAUNCH(kIdxBuf, kAnyGrid)
+    A3D_LAUNCH(kIdxBuf, kCleanGrid)
+    A3D_LAUNCH(kIdxBuf, kFixedGrid)
+    A3D_LAUNCH(kIdx32, kAnyGrid)
+    A3D_LAUNCH(kIdx32, kCleanGrid)
+    A3D_LAUNCH(kIdx32, kFixedGrid)
+    A3D_LAUNCH(kIdx64, kAnyGrid)
+    A3D_LAUNCH(kIdx64, kCleanGrid)
+    A3D_LAUNCH(kIdx64, kFixedGrid)
+  }
 #undef A3D_LAUNCH
+}
+
+template <bool OWN>
+void lanes_fleet_own(const GridDev& g, const FilterDev* fs, const WorkItem* items, uint32_t nitems, uint32_t* counter,
+                     int ppw, int persistent, uint32_t chunk, hipStream_t s) {
+  if (ppw == 64) lanes_fleet_q<1, OWN>(g, fs, items, nitems, counter, persistent, chunk, s);
+  else if (ppw == 32) lanes_fleet_q<2, OWN>(g, fs, items, nitems, counter, persistent, chunk, s);
+  else lanes_fleet_q<4, OWN>(g, fs, items, nitems, counter, persistent, chunk, s);
 }
 
 #undef A3D_LANES_VARIANT
 }  // namespace
 
-void launch_lanes_fleet(const GridDev& g, const FilterDev* fs, const WorkItem* items, uint32_t nitems,
+void launch_lanes_fleet(const GridDev& g, const FilterDev* fs, bool own_grids, const WorkItem* items, uint32_t nitems,
                         uint32_t* counter, int ppw, int persistent, uint32_t chunk, hipStream_t s) {
-  if (ppw == 64) lanes_fleet_q<1>(g, fs, items, nitems, counter, persistent, chunk, s);
-  else if (ppw == 32) lanes_fleet_q<2>(g, fs, items, nitems, counter, persistent, chunk, s);
-  else lanes_fleet_q<4>(g, fs, items, nitems, counter, persistent, chunk, s);
+  if (own_grids)
+    lanes_fleet_own<true>(g, fs, items, nitems, counter, ppw, persistent, chunk, s);
+  else
+    lanes_fleet_own<false>(g, fs, items, nitems, counter, ppw, persistent, chunk, s);
 }
 
 #endif

@@ -66,3 +66,33 @@ def test_poses_at_tile_edges(gpu, room, env, n, monkeypatch):
         w = g.cloud_weights(cloud, t[:, 0], t[:, 1], t[:, 2], t[:, 3])
         ow = oracle.cloud_weight_batch(room["ogrid"], cloud, t[:, 0], t[:, 1], t[:, 2], t[:, 3])
         assert np.array_equal(w.view(np.int32), ow.view(np.int32)), (n, m)
+
+
+# whole turns of 16,384 by whole-cloud wavefronts and the rest split: no rest, the
+# smallest, the largest split one, one more; clouds around the rule's 2,048 points
+@pytest.mark.parametrize("n,m", [(32768, 2050), (32769, 2050), (34816, 2050), (34817, 2050), (32900, 2047), (32900, 2048)])
+def test_rest_of_a_turn(gpu, room, n, m):
+    g, t = _open(gpu, room), _poses(room, n)
+    cloud = np.resize(room["step"].cloud, (m, 3)).astype(np.float32)
+    w = g.cloud_weights(cloud, t[:, 0], t[:, 1], t[:, 2], t[:, 3])
+    ow = oracle.cloud_weight_batch(room["ogrid"], cloud, t[:, 0], t[:, 1], t[:, 2], t[:, 3])
+    assert np.array_equal(w.view(np.int32), ow.view(np.int32))
+
+
+# whole-cloud wavefronts: the last tile's rest, at every tile and wavefront shape
+@pytest.mark.parametrize("ppw", [16, 32, 64])
+@pytest.mark.parametrize("tile", [32, 256])
+def test_last_tile_of_whole_cloud_wavefronts(gpu, room, ppw, tile):
+    g, t = _open(gpu, room), _poses(room, 21000)
+    saved = gpu.get_tile(), gpu.get_cloud_tile()
+    try:
+        gpu.set_tile(ppw)
+        gpu.set_cloud_tile(tile)
+        for m in (0, 1, 7, 8, 9, 15, 16, 17, 31, 32, 33, 255, 256, 257, 300):
+            cloud = np.ascontiguousarray(room["step"].cloud[:m])
+            w = g.cloud_weights(cloud, t[:, 0], t[:, 1], t[:, 2], t[:, 3])
+            ow = oracle.cloud_weight_batch(room["ogrid"], cloud, t[:, 0], t[:, 1], t[:, 2], t[:, 3])
+            assert np.array_equal(w.view(np.int32), ow.view(np.int32)), m
+    finally:
+        gpu.set_tile(saved[0])
+        gpu.set_cloud_tile(saved[1])
