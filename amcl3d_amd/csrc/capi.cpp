@@ -467,11 +467,6 @@ static int grid_alloc(const double mn[3], const double mx[3], double res, double
     delete G;
     return fail(A3D_ERR_NOMEM, "grid: cannot allocate " + std::to_string(bytes) + " bytes of prob");
   }
-  if (hipMemset(G->prob + G->g.cells, 0, sizeof(float)) != hipSuccess) {
-    (void)hipFree(G->prob);
-    delete G;
-    return fail(A3D_ERR_HIP, "grid: cannot clear the zero cell");
-  }
   if (keep_dist && hipMalloc(&G->dist, bytes) != hipSuccess) {
     (void)hipFree(G->prob);
     delete G;
@@ -482,6 +477,14 @@ static int grid_alloc(const double mn[3], const double mx[3], double res, double
     (void)hipFree(G->dist);
     delete G;
     return fail(A3D_ERR_HIP, "grid: cannot create a stream");
+  }
+  launch_zero_u32(reinterpret_cast<uint32_t*>(G->prob + G->g.cells), 1, G->stream);
+  if (hipGetLastError() != hipSuccess || hipStreamSynchronize(G->stream) != hipSuccess) {
+    (void)hipFree(G->prob);
+    (void)hipFree(G->dist);
+    (void)hipStreamDestroy(G->stream);
+    delete G;
+    return fail(A3D_ERR_HIP, "grid: cannot clear the zero cell");
   }
   G->g.prob = G->prob;
   G->g.dist = G->dist;
@@ -495,21 +498,19 @@ int a3d_grid_create_from_points(const float* xyz, size_t n, const double min[3],
   a3d_grid* G = nullptr;
   int rc = grid_alloc(min, max, res, sensor_dev, keep_dist != 0, &G);
   if (rc) return rc;
-  float* d_xyz = nullptr;
+  Pooled xyz_buf;
   if (n) {
-    if (hipMalloc(&d_xyz, n * 3 * sizeof(float)) != hipSuccess) {
+    if (!xyz_buf.take(false, n * 3 * sizeof(float))) {
       a3d_grid_destroy(G);
       return fail(A3D_ERR_NOMEM, "a3d_grid_create_from_points: cannot stage points");
     }
-    if (!hip_ok(hipMemcpy(d_xyz, xyz, n * 3 * sizeof(float), hipMemcpyHostToDevice), "upload points")) {
-      (void)hipFree(d_xyz);
+    if (!hip_ok(hipMemcpy(xyz_buf.p, xyz, n * 3 * sizeof(float), hipMemcpyHostToDevice), "upload points")) {
       a3d_grid_destroy(G);
       return A3D_ERR_HIP;
     }
   }
-  rc = build_grid_device(d_xyz, n, G->g, G->prob, G->dist, sensor_dev, G->stream);
-  if (rc == A3D_OK && !hip_ok(hipStreamSynchronize(G->stream), "computeGrid")) rc = A3D_ERR_HIP;
-  (void)hipFree(d_xyz);
+  rc = build_grid_device(xyz_buf.f(), n, G->g, G->prob, G->dist, sensor_dev, G->stream);
+  if (!hip_ok(hipStreamSynchronize(G->stream), "computeGrid") && rc == A3D_OK) rc = A3D_ERR_HIP;
   if (rc) {
     a3d_grid_destroy(G);
     return rc;

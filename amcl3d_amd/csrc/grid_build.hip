@@ -133,8 +133,8 @@ __global__ __launch_bounds__(kGThreads) void grid_tile_kernel(GridDev g, BucketD
   __shared__ float4 pts[kBatch];
   __shared__ uint32_t blist[kGThreads];
   __shared__ uint32_t bpre[kGThreads + 1];
-  __shared__ uint32_t nlist;
-  __shared__ uint32_t notdone;
+  __shared__ uint32_t nlist, first_wave;
+  __shared__ uint32_t farthest;
   const int tid = threadIdx.x;
   const uint64_t tile = tile0 + blockIdx.x;
   const uint32_t tx = (uint32_t)(tile % ntx);
@@ -183,25 +183,24 @@ __global__ __launch_bounds__(kGThreads) void grid_tile_kernel(GridDev g, BucketD
       bhi[a] = bucket_axis((double)hi[a] + r, b.org[a], b.h, b.nb[a]);
     }
     const uint32_t wx = bhi[0] - blo[0] + 1, wy = bhi[1] - blo[1] + 1, wz = bhi[2] - blo[2] + 1;
-    const uint64_t total = (uint64_t)wx * wy * wz;
+    const uint32_t total = wx * wy * wz;  // at most the number of buckets, below 2^32
     for (uint64_t base = 0; base < total; base += kGThreads) {
       if (tid == 0) nlist = 0;
       __syncthreads();
-      const uint64_t e = base + tid;
-      if (e < total) {
-        uint32_t bi[3];
-        bi[0] = blo[0] + (uint32_t)(e % wx);
-        bi[1] = blo[1] + (uint32_t)((e / wx) % wy);
-        bi[2] = blo[2] + (uint32_t)(e / ((uint64_t)wx * wy));
+      const uint32_t e = (uint32_t)base + tid;
+      if (base + tid < total) {
+        const uint32_t row = e / wx, layer = row / wy;
+        const uint32_t bi[3] = {blo[0] + (e - row * wx), blo[1] + (row - layer * wy), blo[2] + layer};
         const uint32_t id = bi[0] + b.nb[0] * (bi[1] + b.nb[1] * bi[2]);
-        const uint32_t cnt = b.start[id + 1] - b.start[id];
+        const uint32_t at = b.start[id], cnt = b.start[id + 1] - at;
         if (cnt) {
           const double gap = box_gap(b, lo, hi, bi);
           const bool in_prev = bi[0] >= plo[0] && bi[0] <= phi[0] && bi[1] >= plo[1] && bi[1] <= phi[1] &&
                                bi[2] >= plo[2] && bi[2] <= phi[2] && gap <= r_prev;
           if (gap <= r && !in_prev) {
             const uint32_t slot = atomicAdd(&nlist, 1u);
-            blist[slot] = id;
+            blist[slot] = at;
+            bpre[slot] = cnt;
           }
         }
       }
@@ -211,16 +210,23 @@ __global__ __launch_bounds__(kGThreads) void grid_tile_kernel(GridDev g, BucketD
         __syncthreads();  // nlist is reset at the top of the next chunk
         continue;
       }
-      if (tid == 0) {
-        uint32_t acc = 0;
-        for (uint32_t k = 0; k < nl; ++k) {
-          bpre[k] = acc;
-          acc += b.start[blist[k] + 1] - b.start[blist[k]];
-        }
-        bpre[nl] = acc;
+      // exclusive sums of the buckets' counts (a thread per bucket; thread 0
+      // adding them up, two global reads a bucket, held each tile for tens of
+      // microseconds)
+      const uint32_t cnt = (uint32_t)tid < nl ? bpre[tid] : 0u;
+      uint32_t inc = cnt;
+      for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t v = __shfl_up(inc, d);
+        if ((tid & 63) >= d) inc += v;
       }
+      if (tid == 63) first_wave = inc;
       __syncthreads();
-      const uint32_t tp = bpre[nl];
+      static_assert(kGThreads == 128, "two wavefronts");
+      if (tid >= 64) inc += first_wave;
+      bpre[tid] = inc - cnt;
+      if (tid == kGThreads - 1) bpre[kGThreads] = inc;
+      __syncthreads();
+      const uint32_t tp = bpre[kGThreads];
       for (uint32_t pb = 0; pb < tp; pb += kBatch) {
         const uint32_t len = min((uint32_t)kBatch, tp - pb);
         for (uint32_t k = tid; k < len; k += kGThreads) {
@@ -231,7 +237,7 @@ __global__ __launch_bounds__(kGThreads) void grid_tile_kernel(GridDev g, BucketD
             if (bpre[mid] <= q) l = mid;
             else h = mid;
           }
-          const uint32_t gi = b.start[blist[l]] + (q - bpre[l]);
+          const uint32_t gi = blist[l] + (q - bpre[l]);
           pts[k] = make_float4(b.px[gi], b.py[gi], b.pz[gi], 0.f);
         }
         __syncthreads();
@@ -252,29 +258,33 @@ __global__ __launch_bounds__(kGThreads) void grid_tile_kernel(GridDev g, BucketD
         __syncthreads();
       }
     }
-    bool ok = true;
+    // the tile's largest best distance (bit patterns of non-negative floats
+    // are ordered like their values), through one LDS word
     const double lim = r * r * (1.0 - 1e-6);
     const bool past_cut = lim >= cut;  // unseen points give prob 0, as does best
+    float worst = 0.0f;
 #pragma unroll
     for (int c = 0; c < 4; ++c)
-      if (cv[c] && !((double)best[c] <= lim) && !past_cut) ok = false;
-    // workgroup AND of ok through one LDS word (every thread passes each barrier)
-    if (tid == 0) notdone = 0u;
+      if (cv[c]) worst = fmaxf(worst, best[c]);
+    for (int d = 32; d >= 1; d >>= 1) worst = fmaxf(worst, __shfl_xor(worst, d));
+    if (tid == 0) farthest = 0u;
     __syncthreads();
-    if (!ok) notdone = 1u;
+    if ((tid & 63) == 0) atomicMax(&farthest, __float_as_uint(worst));
     __syncthreads();
-    const bool finished = (notdone == 0u) || r >= rmax;
+    worst = __uint_as_float(farthest);
     __syncthreads();
-    if (finished) break;
+    if (past_cut || (double)worst <= lim || r >= rmax) break;  // uniform over the workgroup
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
       plo[a] = blo[a];
       phi[a] = bhi[a];
     }
     r_prev = r;
-    // the radius at which the prob cut applies, if that comes before 2r
-    const double rc = sqrt(cut / (1.0 - 1e-6)) * (1.0 + 1e-9);
-    r = (rc > r && rc < 2.0 * r) ? rc : 2.0 * r;
+    // the radius that settles every cell (no point is nearer to a cell than its
+    // best) or at which the prob cut applies, if that comes before 2r: a round
+    // no wider than needed streams fewer points
+    const double need = sqrt(fmin((double)worst, cut) / (1.0 - 1e-6)) * (1.0 + 1e-9);
+    r = (need > r && need < 2.0 * r) ? need : 2.0 * r;
   }
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
@@ -308,37 +318,29 @@ int build_grid_device(const float* d_xyz, size_t n, const GridDev& g, float* d_p
   }
   if (nbk >= 0xfffffff0ull || n >= 0xfffffff0ull)
     return fail(A3D_ERR_ARG, "computeGrid: too many buckets or points for one build");
-  uint32_t *cnt = nullptr, *start = nullptr, *key = nullptr;
-  float *px = nullptr, *py = nullptr, *pz = nullptr, *cut = nullptr;
-  void* tmp = nullptr;
   size_t tmp_bytes = 0;
-  int rc = A3D_OK;
-  auto cleanup = [&]() {
-    (void)hipFree(cnt);
-    (void)hipFree(start);
-    (void)hipFree(key);
-    (void)hipFree(px);
-    (void)hipFree(py);
-    (void)hipFree(pz);
-    (void)hipFree(cut);
-    (void)hipFree(tmp);
-  };
-#define A3D_TRY(call)              \
-  if (!hip_ok((call), #call)) {    \
-    cleanup();                     \
-    return A3D_ERR_HIP;            \
+  // Working memory from the pool; every return leaves the stream idle.
+#define A3D_TRY(call)               \
+  if (!hip_ok((call), #call)) {     \
+    (void)hipStreamSynchronize(s);  \
+    return A3D_ERR_HIP;             \
   }
-  A3D_TRY(hipMalloc(&cnt, (nbk + 1) * sizeof(uint32_t)));
-  A3D_TRY(hipMalloc(&start, (nbk + 1) * sizeof(uint32_t)));
-  A3D_TRY(hipMalloc(&key, n * sizeof(uint32_t)));
-  A3D_TRY(hipMalloc(&px, n * sizeof(float)));
-  A3D_TRY(hipMalloc(&py, n * sizeof(float)));
-  A3D_TRY(hipMalloc(&pz, n * sizeof(float)));
+  Pooled work, scan, cut_buf;
+  const uint64_t nb4 = (nbk + 1 + 63) & ~63ull, n4 = ((uint64_t)n + 63) & ~63ull;  // words, 256-byte aligned
+  A3D_TRY(work.take(false, (2 * nb4 + 4 * n4) * 4) ? hipSuccess : hipErrorOutOfMemory);
+  uint32_t* const cnt = static_cast<uint32_t*>(work.p);
+  uint32_t* const start = cnt + nb4;
+  uint32_t* const key = start + nb4;
+  float* const px = reinterpret_cast<float*>(key + n4);
+  float* const py = px + n4;
+  float* const pz = py + n4;
+  float* cut = nullptr;
   launch_zero_u32(cnt, (uint32_t)(nbk + 1), s);
   bucket_count_kernel<<<(uint32_t)((n + 255) / 256), 256, 0, s>>>(d_xyz, (uint32_t)n, b, cnt, key);
   A3D_TRY(hipGetLastError());
   A3D_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp_bytes, cnt, start, (int)(nbk + 1), s));
-  A3D_TRY(hipMalloc(&tmp, tmp_bytes));
+  A3D_TRY(scan.take(false, tmp_bytes) ? hipSuccess : hipErrorOutOfMemory);
+  void* const tmp = scan.p;
   A3D_TRY(hipcub::DeviceScan::ExclusiveSum(tmp, tmp_bytes, cnt, start, (int)(nbk + 1), s));
   // reuse cnt as the fill cursor
   A3D_TRY(hipMemcpyAsync(cnt, start, nbk * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
@@ -354,7 +356,8 @@ int build_grid_device(const float* d_xyz, size_t n, const GridDev& g, float* d_p
   for (int a = 0; a < 3; ++a) rmax += (b.nb[a] * b.h + 1.0) * (b.nb[a] * b.h + 1.0);
   rmax = std::sqrt(rmax) * 2.0;
   if (!d_dist) {  // prob only: the search may stop where prob reaches 0
-    A3D_TRY(hipMalloc(&cut, sizeof(float)));
+    A3D_TRY(cut_buf.take(false, sizeof(float)) ? hipSuccess : hipErrorOutOfMemory);
+    cut = cut_buf.f();
     prob_cut_kernel<<<1, 64, 0, s>>>(c1, c2, cut);
     A3D_TRY(hipGetLastError());
   }
@@ -366,8 +369,7 @@ int build_grid_device(const float* d_xyz, size_t n, const GridDev& g, float* d_p
   }
   A3D_TRY(hipStreamSynchronize(s));
 #undef A3D_TRY
-  cleanup();
-  return rc;
+  return A3D_OK;
 }
 
 }  // namespace a3d
