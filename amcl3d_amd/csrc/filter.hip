@@ -1101,15 +1101,49 @@ __device__ float chunk_walk(float s, uint32_t nq, int k, float* prefix, const Ld
   return s;
 }
 
+// A sum of up to kSerialSubs sub-tiles is added term by term: it crosses a
+// binade every few sub-tiles, 64 adds take no longer than a scan of their maps,
+// and no maps are needed (updates of 600, 1,000 and 1,500 particles 34, 36 and
+// 44 us with maps, 25, 30 and 40 us without).
+constexpr uint32_t kSerialSubs = 32;
+__device__ __forceinline__ float chunk_serial(float s, uint32_t nq, const float* terms, float* prefix) {
+  const float4* const x = reinterpret_cast<const float4*>(terms);
+  float4 a[8], b[8];  // half a sub-tile is read while the other is added
+  auto rd = [&](uint32_t h, float4 (&v)[8]) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] = x[h * 8 + c];
+  };
+  auto add = [&](const float4 (&v)[8]) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      s += v[c].x;
+      s += v[c].y;
+      s += v[c].z;
+      s += v[c].w;
+    }
+  };
+  rd(0, a);
+  for (uint32_t q = 0; q < nq; ++q) {
+    rd(2 * q + 1, b);
+    add(a);
+    if (q + 1 < nq) rd(2 * q + 2, a);
+    add(b);
+    if (prefix && lane_id() == 0) prefix[q] = s;
+  }
+  return s;
+}
+
 // s[k] + the chunk's len terms of sum k in order, for every k, in every thread.
 // xv[k][u]: this thread's term u * kChainThreads + tid of sum k (0 past len).
-// prefix (or null): the checkpoints of sum NS - 1 from the chunk's first on.
+// prefix (or null): the checkpoints of sum NS - 1 from the chunk's first on;
+// first: nothing has been added yet.
 template <int NS, int K>
-__device__ __forceinline__ void chunk_sums(float (&s)[NS], const float (&xv)[NS][K], uint32_t len, float* prefix,
-                                           ChunkLds<NS, K>& L) {
+__device__ __forceinline__ void chunk_sums(float (&s)[NS], const float (&xv)[NS][K], uint32_t len, bool first,
+                                           float* prefix, ChunkLds<NS, K>& L) {
   const uint32_t tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
   constexpr uint32_t kW = kChainThreads / 64, kSubs = ChunkLds<NS, K>::kSubs;
   const uint32_t nq = (len + 63) / 64;
+  const bool serial = first && nq <= kSerialSubs;  // uniform
 #pragma unroll
   for (int k = 0; k < NS; ++k) {
 #pragma unroll
@@ -1117,11 +1151,13 @@ __device__ __forceinline__ void chunk_sums(float (&s)[NS], const float (&xv)[NS]
       const uint32_t q = u * kW + wave;
       if (q >= nq) continue;  // uniform over the wavefront
       L.x[k][u * kChainThreads + tid] = xv[k][u];
+      if (serial) continue;
       const float w = wave_sum(xv[k][u]);
       if (lane == 0) L.part[k][q] = w;
     }
   }
   __syncthreads();
+  if (!serial) {
 #pragma unroll
   for (int k = 0; k < NS; ++k) {
     // the guesses: s plus the float sums of the sub-tiles before this one
@@ -1161,11 +1197,13 @@ __device__ __forceinline__ void chunk_sums(float (&s)[NS], const float (&xv)[NS]
       }
     }
   }
-  __syncthreads();
+    __syncthreads();
+  }
 #pragma unroll
   for (int k = 0; k < NS; ++k) {
     if (wave == (uint32_t)k) {
-      const float v = chunk_walk(s[k], nq, k, k == NS - 1 ? prefix : nullptr, L);
+      float* const pre = k == NS - 1 ? prefix : nullptr;
+      const float v = serial ? (nq ? chunk_serial(s[k], nq, L.x[k], pre) : s[k]) : chunk_walk(s[k], nq, k, pre, L);
       if (lane == 0) L.s[k] = v;
     }
   }
@@ -1189,7 +1227,7 @@ __device__ __forceinline__ float exact_sum(uint32_t n, const float* __restrict__
       xv[0][u] = i < len ? x[base + i] : 0.0f;
     }
     if (base) __syncthreads();  // every thread has read the previous chunk's sum
-    chunk_sums<1, kChunkPer>(s, xv, len, prefix ? prefix + base / kGroup : nullptr, L);
+    chunk_sums<1, kChunkPer>(s, xv, len, base == 0, prefix ? prefix + base / kGroup : nullptr, L);
   }
   return s[0];
 }
@@ -1419,7 +1457,7 @@ __global__ __launch_bounds__(kChainThreads) void tail_c_tiled_kernel(Filters fs)
 // The whole tail by one workgroup per filter, for filters of at most
 // kChainThreads * K particles: a particle's fields and weights stay in its
 // thread's registers between the sums, so the six launches and their passes
-// over memory become one (600 particles: 41 -> 34 us for the whole update).
+// over memory become one (600 particles: 41 -> 25 us for the whole update).
 template <int K>
 __global__ __launch_bounds__(kChainThreads) void tail_one_kernel(GridDev g, Filters fs) {
   __shared__ __align__(16) unsigned char lds[sizeof(ChunkLds<5, K>)];
@@ -1444,7 +1482,7 @@ __global__ __launch_bounds__(kChainThreads) void tail_one_kernel(GridDev g, Filt
     t2[1][u] = in[u] ? wr[u] : 0.f;
   }
   float s2[2] = {0.f, 0.f};
-  chunk_sums<2, K>(s2, t2, n, nullptr, *reinterpret_cast<ChunkLds<2, K>*>(lds));
+  chunk_sums<2, K>(s2, t2, n, true, nullptr, *reinterpret_cast<ChunkLds<2, K>*>(lds));
   const float wtp = s2[0], wtr = s2[1];
   float t1[1][K];
 #pragma unroll
@@ -1461,7 +1499,7 @@ __global__ __launch_bounds__(kChainThreads) void tail_one_kernel(GridDev g, Filt
   }
   __syncthreads();  // the sums have been read
   float s1[1] = {0.f};
-  chunk_sums<1, K>(s1, t1, n, nullptr, *reinterpret_cast<ChunkLds<1, K>*>(lds));
+  chunk_sums<1, K>(s1, t1, n, true, nullptr, *reinterpret_cast<ChunkLds<1, K>*>(lds));
   const float wt = s1[0];
   float t5[5][K];
   int irregular = 0;
@@ -1478,7 +1516,7 @@ __global__ __launch_bounds__(kChainThreads) void tail_one_kernel(GridDev g, Filt
   }
   irregular = __syncthreads_or(irregular);
   float s5[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
-  chunk_sums<5, K>(s5, t5, n, f.scratch + sc_c32(n), *reinterpret_cast<ChunkLds<5, K>*>(lds));
+  chunk_sums<5, K>(s5, t5, n, true, f.scratch + sc_c32(n), *reinterpret_cast<ChunkLds<5, K>*>(lds));
   if (tid == 0) {
     float* const sums = sums_of(f);
     sums[0] = wtp;
