@@ -302,18 +302,18 @@ __global__ void voxel_place_kernel(const uint32_t* voxel, uint32_t n, const uint
 // The centroids.  Half a wavefront takes a voxel of up to 32 points: it orders
 // them by index (a lane's rank is the number of smaller ones) and sums them in
 // that order.  A voxel of more points is taken by the whole wavefront, which
-// ranks them the same way (c^2 / 64 steps), or, past kRankMax points or where
-// that is shorter, searches all the cloud's points for them (n / 64 steps).
-constexpr uint32_t kRankMax = 1024;
+// sorts their indices, or, past kSortMax points, searches all the cloud's points
+// for them.
+constexpr uint32_t kSortMax = 1024;
 __global__ __launch_bounds__(256) void voxel_average_kernel(const uint8_t* pts, uint32_t n, size_t stride,
                                                             const uint32_t* voxel, const uint32_t* count,
                                                             const uint32_t* start, const uint32_t* list,
                                                             const uint32_t* total, float* ox, float* oy, float* oz) {
   constexpr uint32_t kWaves = 4;
-  __shared__ float xyz[kWaves][3][kRankMax];
+  __shared__ float xyz[kWaves][3][kSortMax];
   const int lane = lane_id(), l = lane & 31, half = lane >> 5;
   const uint32_t wave = threadIdx.x >> 6, nv = *total;
-  float(&xs)[3][kRankMax] = xyz[wave];
+  float(&xs)[3][kSortMax] = xyz[wave];
   auto put = [&](uint32_t at, uint32_t i) {
     const float* p = point_at(pts, stride, i);
     xs[0][at] = p[0];
@@ -346,42 +346,69 @@ __global__ __launch_bounds__(256) void voxel_average_kernel(const uint8_t* pts, 
       crowded &= crowded - 1;
       const uint32_t v = (uint32_t)__builtin_amdgcn_readlane((int)o, src);
       const uint32_t cv = (uint32_t)__builtin_amdgcn_readlane((int)c, src);
-      if (cv <= kRankMax && (uint64_t)cv * cv <= 2 * (uint64_t)n) {
+      if (cv <= kSortMax) {  // bitonic sort of the listed points' indices in LDS
         const uint32_t* const lv = list + start[v];
+        uint32_t* const si = reinterpret_cast<uint32_t*>(xs[0]);
+        uint32_t np = 64;
+        while (np < cv) np <<= 1;
         wave_lds_sync();
-        for (uint32_t j0 = 0; j0 < cv; j0 += 64) {
-          const uint32_t mine = j0 + lane < cv ? lv[j0 + lane] : 0xffffffffu;
-          uint32_t r = 0;
-          for (uint32_t j1 = 0; j1 < cv; j1 += 64) {
-            const uint32_t other = j1 + lane < cv ? lv[j1 + lane] : 0xffffffffu;
 #pragma unroll
-            for (int j = 0; j < 64; ++j) r += (uint32_t)__builtin_amdgcn_readlane((int)other, j) < mine ? 1u : 0u;
-          }
-          if (j0 + lane < cv) put(r, mine);
+        for (uint32_t k = 0; k < kSortMax / 64; ++k) {
+          const uint32_t j = k * 64 + lane;
+          if (k * 64 < np) si[j] = j < cv ? lv[j] : 0xffffffffu;
         }
+        for (uint32_t k = 2; k <= np; k <<= 1) {
+          for (uint32_t d = k >> 1; d > 0; d >>= 1) {
+            wave_lds_sync();
+            for (uint32_t t = lane; t < np / 2; t += 64) {
+              const uint32_t p = 2 * t - (t & (d - 1)), q = p + d;
+              const uint32_t x = si[p], y = si[q];
+              if ((x > y) == ((p & k) == 0)) {
+                si[p] = y;
+                si[q] = x;
+              }
+            }
+          }
+        }
+        wave_lds_sync();
+        uint32_t at[kSortMax / 64];
+#pragma unroll
+        for (uint32_t k = 0; k < kSortMax / 64; ++k) at[k] = k * 64 + lane < cv ? si[k * 64 + lane] : 0u;
+        wave_lds_sync();  // the indices have been read: the points go over them
+#pragma unroll
+        for (uint32_t k = 0; k < kSortMax / 64; ++k)
+          if (k * 64 + lane < cv) put(k * 64 + lane, at[k]);
         wave_lds_sync();
         if (lane < 3) sum(lane, 0, cv, v);
         continue;
       }
+      constexpr uint32_t kAhead = 16;  // loads in flight
       float sx = 0.f, sy = 0.f, sz = 0.f;
-      for (uint32_t j0 = 0; j0 < n; j0 += 64) {
-        const uint32_t j = j0 + lane;
-        const bool in = j < n && voxel[j] == v;
-        uint64_t m = __ballot(in);
-        if (!m) continue;
-        float x = 0.f, y = 0.f, z = 0.f;
-        if (in) {
-          const float* p = point_at(pts, stride, j);
-          x = p[0];
-          y = p[1];
-          z = p[2];
+      for (uint32_t j0 = 0; j0 < n; j0 += 64 * kAhead) {
+        uint32_t vx[kAhead];
+#pragma unroll
+        for (uint32_t k = 0; k < kAhead; ++k) {
+          const uint32_t j = j0 + k * 64 + lane;
+          vx[k] = j < n ? voxel[j] : kNoVoxel;
         }
-        while (m) {
-          const int q = (int)__builtin_ctzll(m);
-          m &= m - 1;
-          sx += readlane_f(x, q);
-          sy += readlane_f(y, q);
-          sz += readlane_f(z, q);
+#pragma unroll
+        for (uint32_t k = 0; k < kAhead; ++k) {
+          uint64_t m = __ballot(vx[k] == v);
+          if (!m) continue;
+          float x = 0.f, y = 0.f, z = 0.f;
+          if (vx[k] == v) {
+            const float* p = point_at(pts, stride, j0 + k * 64 + lane);
+            x = p[0];
+            y = p[1];
+            z = p[2];
+          }
+          while (m) {
+            const int q = (int)__builtin_ctzll(m);
+            m &= m - 1;
+            sx += readlane_f(x, q);
+            sy += readlane_f(y, q);
+            sz += readlane_f(z, q);
+          }
         }
       }
       if (lane == 0) {
