@@ -224,8 +224,9 @@ enum { A3D_MAP_PARTICLE_LANES = 0, A3D_MAP_POINT_LANES = 1 };
 int a3d_set_tile(int particles_per_wave);
 int a3d_get_tile(int* particles_per_wave);
 /* Points of the cloud staged per LDS tile by the A3D_MAP_PARTICLE_LANES
- * kernels (32, 64, 128 or 256; default 64): the workgroup's wavefronts walk
- * the cloud one tile at a time, one barrier per tile.  Point-lane kernels
+ * kernels (32, 64, 128 or 256; default 64, and 256 in single-filter and pose
+ * launches until it is set): the workgroup's wavefronts walk the cloud one
+ * tile at a time, one barrier per tile.  Point-lane kernels
  * always stage 64 (one point per lane). */
 int a3d_set_cloud_tile(int points);
 int a3d_get_cloud_tile(int* points);
