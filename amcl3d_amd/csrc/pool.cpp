@@ -82,10 +82,13 @@ void pool_give(PoolBuf& b) {
   {
     std::lock_guard<std::mutex> lock(P.mu);
     if (P.bytes[b.host] + b.bytes <= kIdleMax[b.host]) {
-      P.idle.push_back(b);
-      P.bytes[b.host] += b.bytes;
-      b.p = nullptr;
-      return;
+      try {  // destructors come here: no exception leaves
+        P.idle.push_back(b);
+        P.bytes[b.host] += b.bytes;
+        b.p = nullptr;
+        return;
+      } catch (...) {
+      }
     }
   }
   release(b);
