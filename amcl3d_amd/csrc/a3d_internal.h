@@ -86,6 +86,16 @@ struct GridDev {
   uint32_t fx_near;
 };
 
+// A pose's offset o along an axis in the fixed-point form.  Below 2^20 cells the
+// product is a multiple of 2^-1074 within half of that; farther out its rounding
+// would grow with it (2^-20 of a cell at 2^33 cells), so there the offset is a
+// NaN, whose low word of 0 sends every point to the exact form.  Only poses given
+// explicitly lie so far out.
+__host__ __device__ inline double fixed_offset(const GridDev& g, double o) {
+  const double t = o * g.fx_scale;
+  return __builtin_fabs(t) < 0x1p-1022 ? t + g.fx_shift : __builtin_nan("");
+}
+
 // One filter and the parameters of the call being made on it.  Arrays are
 // device pointers.
 struct FilterDev {

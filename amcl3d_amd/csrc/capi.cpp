@@ -66,33 +66,39 @@ static bool axis_clean(double res, double inv_res, uint32_t size) {
   return true;
 }
 
-// The fixed-point cells of the cloud weight, on a clean grid.  For a point at s of a pose at
-// offset o the reference's cell is floor(q / res) with q the float nearest to
-// s + o: its argument differs from (s + o) / res by at most half a float
-// spacing of q over res, at most half that of the axis' largest q.  The fixed
-// form has the same value within 2^-33 for each of its two roundings and q *
-// 2^-33 for the rounding of fx_scale, a subnormal (2^-1074 is its last bit).
-// delta is the sum of these bounds, so the two give the same cell unless the
-// fixed form is within delta of a cell's face.  The bound of the map (lim)
-// must be a face too, within delta's slack, on every axis.  fixed is set while
-// few groups of 256 evaluations hold a point that close (6 delta each: 28% at
-// the limit, 12% on 2,000 cells, 1.5% on 200).
+// The fixed-point cells of the cloud weight, on a clean grid.  For a point at s
+// of a pose at offset o the reference's cell is floor(q / res) with q the float
+// nearest to s + o.  delta bounds, in cells and over every axis, how far the
+// fixed form of s + o can lie from it:
+//   half a float spacing of the axis' largest q, for the rounding of q;
+//   the error of fx_scale times the largest q: a subnormal's last bit is
+//   2^-1074, so the scale is 1 / res within 2^-33 of a cell per unit (exact
+//   where 1 / res has few bits);
+//   2^-33 for each rounding of the form itself (the offset's product, fx_shift,
+//   the multiply-add) and 2^-34 for those of 1 / res and q / res: 2^-30 is over
+//   twice their sum;
+//   the distance of the map's bound (lim, a float) from the nearest face.
+// The two then give the same cell unless the fixed form is within delta of a
+// face, where the kernels redo the lane.  fixed is set while few groups of 256
+// evaluations hold a point that close (6 delta each: 28% at the limit, 12% on
+// 2,000 cells, 1.5% on 200); past it, and on maps whose last cell is cut, the
+// clean form stands.
 static void fixed_meta(GridDev& g) {
   g.fixed = 0u;
-  if (!g.clean) return;
-  const double slack = 0x1p-20;
-  double half = 0.0;
+  if (!g.clean || !(g.inv_res < 0x1p20) || !(g.inv_res > 0x1p-20)) return;
+  g.fx_scale = std::ldexp(g.inv_res, -1042);
+  const double scale_err = std::fabs(std::ldexp(g.fx_scale, 1042) - g.inv_res);
+  double delta = 0.0;
   for (int a = 0; a < 3; ++a) {
     float b;
     std::memcpy(&b, &g.lim[a], 4);
     const double t = (double)b * g.inv_res, n = std::nearbyint(t);
-    if (!(n >= 1.0 && n < 0x1p19 && std::fabs(t - n) <= slack / 2)) return;
+    if (!(n >= 1.0 && n < 0x1p19)) return;
     g.fx_size[a] = (uint32_t)n;
-    half = std::max(half, std::ldexp(1.0, std::ilogb(b) - 24));
+    const double half = std::ldexp(1.0, std::ilogb(b) - 24);
+    delta = std::max(delta, (half * g.inv_res + (double)b * scale_err) * 1.0001 + std::fabs(t - n) + 0x1p-30);
   }
-  const double delta = half * g.inv_res * 1.0001 + slack;
-  if (!(delta <= 0x1p-12) || !(g.inv_res < 0x1p20) || !(g.inv_res > 0x1p-20)) return;
-  g.fx_scale = std::ldexp(g.inv_res, -1042);
+  if (!(delta <= 0x1p-12)) return;
   g.fx_shift = std::ldexp(delta, -1042);
   g.fx_near = (uint32_t)std::ceil(std::ldexp(2.0 * delta, 32)) + 2u;
   g.fixed = 1u;

@@ -333,9 +333,9 @@ struct LanePose {
 
 __device__ __forceinline__ void set_fixed(const GridDev& g, LanePose& lp, bool act, float tx, float ty, float tz) {
   const double out = __hiloint2double(0x3ff00000, (int)0x80000000u);
-  lp.fx = act ? ((double)tx - g.min[0]) * g.fx_scale + g.fx_shift : out;
-  lp.fy = act ? ((double)ty - g.min[1]) * g.fx_scale + g.fx_shift : out;
-  lp.fz = act ? ((double)tz - g.min[2]) * g.fx_scale + g.fx_shift : out;
+  lp.fx = act ? fixed_offset(g, (double)tx - g.min[0]) : out;
+  lp.fy = act ? fixed_offset(g, (double)ty - g.min[1]) : out;
+  lp.fz = act ? fixed_offset(g, (double)tz - g.min[2]) : out;
   lp.tx = act ? tx : __builtin_nanf("");
   lp.ty = ty;
   lp.tz = tz;
