@@ -96,6 +96,12 @@ __host__ __device__ inline double fixed_offset(const GridDev& g, double o) {
   return __builtin_fabs(t) < 0x1p-1022 ? t + g.fx_shift : __builtin_nan("");
 }
 
+// Every coordinate of a point that is in no map: a NaN with its payload's bits
+// set.  The rotation and the fixed-point form keep the payload, so the low word
+// is never near a face and the lane is not redone; the high word of any NaN is
+// past every map, whatever its payload.
+constexpr float kOutside = __builtin_nanf("0x3fffff");
+
 // One filter and the parameters of the call being made on it.  Arrays are
 // device pointers.
 struct FilterDev {

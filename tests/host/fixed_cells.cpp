@@ -4,7 +4,9 @@
 // uniform ones, under offsets of many poses.  Reads lines of
 //   nx ny nz  res  minx miny minz  cut  draws  seed
 // (max lies `cut` cells below the last face) and prints for each
-//   fixed  near-fraction-bound  judged  wrong  (judged: evaluations away from the faces)
+//   fixed  near-fraction-bound  judged  wrong  outside-near
+// (judged: evaluations away from the faces; outside-near: lanes that would be
+// redone for the point that stands for padding and non-finite points)
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -78,7 +80,17 @@ int main() {
       ++judged;
       wrong += f.in != r.in || (r.in && f.i != r.i);
     }
-    std::printf("%u %.9g %ld %ld\n", g.fixed, std::ldexp((double)g.fx_near, -32), judged, wrong);
+    long outside = 0;
+    for (int d = 0; g.fixed && d < 20000; ++d) {  // rotated by any yaw, as the kernel does
+      const float yaw = (float)(6.4 * u01(rng) - 3.2), c = std::cos(yaw), n = std::sin(yaw), p = a3d::kOutside;
+      const float s[3] = {p * c + p * -n, p * n + p * c, p};
+      for (int a = 0; a < 3; ++a) {
+        Cell f{};
+        const double o = (double)(float)(m[a] + g.ext[a] * u01(rng)) - m[a];
+        outside += !fixed(g, a, s[a], o, f) || f.in;
+      }
+    }
+    std::printf("%u %.9g %ld %ld %ld\n", g.fixed, std::ldexp((double)g.fx_near, -32), judged, wrong, outside);
   }
   return 0;
 }

@@ -25,7 +25,7 @@ def checker(tmp_path_factory):
         out = subprocess.run([exe], input=text, capture_output=True, text=True, check=True, timeout=300).stdout
         rows = [line.split() for line in out.splitlines()]
         assert len(rows) == len(grids)
-        return [(int(f), float(near), int(j), int(w)) for f, near, j, w in rows]
+        return [(int(f), float(near), int(j), int(w), int(o)) for f, near, j, w, o in rows]
 
     return check
 
@@ -45,7 +45,7 @@ CELLS = [(0.05, (900, 40, 70), (-17.35, 3.1, -0.4)), (0.05, (2000, 2000, 600), (
 @pytest.mark.parametrize("part", range(3))
 def test_cells_match_the_reference(checker, part):
     grids = [n + (res,) + mn + (0.0, 3_000_000, 11 + part) for res, n, mn in CELLS[part::3]]
-    for g, (fixed, near, judged, wrong) in zip(grids, checker(grids)):
+    for g, (fixed, near, judged, wrong, _) in zip(grids, checker(grids)):
         assert wrong == 0, (g, near, judged, wrong)
         if fixed:
             assert judged > 300_000, (g, judged)  # a third of the draws are away from the faces
@@ -61,7 +61,7 @@ def test_random_extents(checker):
         n = tuple(int(v) for v in rng.integers(20, 1200, 3))
         mn = tuple(float(v) for v in np.round(rng.uniform(-50, 50, 3), 2))
         grids.append(n + (res,) + mn + (0.0, 100_000, k))
-    for g, (fixed, near, judged, wrong) in zip(grids, checker(grids)):
+    for g, (fixed, near, judged, wrong, _) in zip(grids, checker(grids)):
         assert wrong == 0, (g, near, judged, wrong)
 
 
@@ -78,3 +78,13 @@ def test_which_grids_are_fixed(checker):
     grids = [n + (res,) + mn + (cut, 1000, 1) for n, res, mn, cut in want]
     got = [r[0] for r in checker(grids)]
     assert dict(zip(want, got)) == want
+
+
+def test_outside_points_are_not_redone(checker):
+    """The point staged for padding and for non-finite points: out of the map
+    and away from every face under any pose, so that no lane repeats it."""
+    grids = [n + (res,) + mn + (0.0, 1000, 2) for res, n, mn in CELLS]
+    rows = checker(grids)
+    assert sum(r[0] for r in rows) > len(rows) // 2
+    for g, (fixed, near, judged, wrong, outside) in zip(grids, rows):
+        assert outside == 0, (g, outside)

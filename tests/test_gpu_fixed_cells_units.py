@@ -48,3 +48,25 @@ def test_points_near_cell_faces(gpu, name, poses):
         w = g.cloud_weights(cloud, t[:, 0], t[:, 1], t[:, 2], t[:, 3], roll, pitch)
         ow = oracle.cloud_weight_batch(og, cloud, t[:, 0], t[:, 1], t[:, 2], t[:, 3], roll, pitch)
         assert np.array_equal(w.view(np.int32), ow.view(np.int32)), (name, roll)
+
+
+@pytest.mark.parametrize("poses", [40, 2500, 7000, 29000])
+def test_many_points_and_rotations_that_are_not_finite(gpu, poses):
+    n, res, mn = GRIDS["19.9 m"]
+    n, mn = np.array(n), np.array(mn)
+    mx = mn + n * res
+    prob = np.random.default_rng(7).uniform(0.0, 4.0, (n[2], n[1], n[0])).astype(F32)
+    g, og = gpu.Grid3d().from_cells(prob, mn, mx, res, 0.1), oracle.GridMeta(mn, mx, res, prob)
+    rng = np.random.default_rng(poses)
+    cloud = rng.uniform(-5, 5, (300, 3)).astype(F32)
+    bad = rng.random(300) < 0.4
+    cloud[bad, rng.integers(0, 3, bad.sum())] = rng.choice([np.nan, np.inf, -np.inf], bad.sum())
+    t = np.empty((poses, 4), F32)
+    t[:, :3] = rng.uniform(mn, mx, (poses, 3))
+    t[:, 3] = rng.uniform(-3.2, 3.2, poses)
+    t[::2, :3] = np.round(t[::2, :3], 1)  # offsets on faces
+    t[3::50, 3] = rng.choice([np.nan, np.inf], len(t[3::50]))
+    for roll, pitch in ((0.0, 0.0), (0.03, -0.07), (np.nan, 0.0)):
+        w = g.cloud_weights(cloud, t[:, 0], t[:, 1], t[:, 2], t[:, 3], roll, pitch)
+        ow = oracle.cloud_weight_batch(og, cloud, t[:, 0], t[:, 1], t[:, 2], t[:, 3], roll, pitch)
+        assert np.array_equal(w.view(np.int32), ow.view(np.int32)), roll
