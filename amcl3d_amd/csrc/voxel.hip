@@ -197,20 +197,46 @@ __global__ void voxel_clear_kernel(uint4* p, uint32_t n) {
   if (i < n) p[i] = make_uint4(0u, 0u, 0u, 0u);
 }
 
-// Every finite point's voxel, and its bit.  Bound by the atomics (21 us for
-// 100,000 points; testing the bit before setting it measured the same).
-__global__ void voxel_mark_kernel(const uint8_t* pts, uint32_t n, size_t stride, const VoxelMeta* meta, uint32_t* key,
-                                  uint32_t* bits) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const VoxelMeta m = *meta;
-  const float* p = point_at(pts, stride, i);
-  uint32_t k = kNoVoxel;
-  if (finite3(p)) {
-    k = voxel_key(m, p);
-    atomicOr(&bits[k >> 5], 1u << (k & 31));
+// Every finite point's voxel, and its bit.  Atomics of many points on a few words
+// queue up (1.8 ns each: 1,000,000 points in 900 voxels took 1,830 us), so a
+// workgroup first joins its points' bits word by word in a hash table in LDS and
+// sets each word once (1,085 us for that whole call, where 2,650 went before and
+// 2,380 with the sort; a scan of 100,000 points 169 instead of 189 us).
+// Workgroups of 256 and 512 points join less (1,252 and 1,236 us).
+constexpr uint32_t kMarkThreads = 1024;
+__global__ __launch_bounds__(kMarkThreads) void voxel_mark_kernel(const uint8_t* pts, uint32_t n, size_t stride,
+                                                                  const VoxelMeta* meta, uint32_t* key,
+                                                                  uint32_t* bits) {
+  constexpr uint32_t kSlots = 2 * kMarkThreads, kFree = 0xffffffffu;  // half empty: every word finds a slot
+  __shared__ uint32_t word[kSlots], mask[kSlots];
+  const uint32_t tid = threadIdx.x, i = blockIdx.x * kMarkThreads + tid;
+#pragma unroll
+  for (uint32_t h = tid; h < kSlots; h += kMarkThreads) {
+    word[h] = kFree;
+    mask[h] = 0u;
   }
-  key[i] = k;
+  uint32_t k = kNoVoxel;
+  if (i < n) {
+    const VoxelMeta m = *meta;
+    const float* p = point_at(pts, stride, i);
+    if (finite3(p)) k = voxel_key(m, p);
+    key[i] = k;
+  }
+  __syncthreads();
+  if (k != kNoVoxel) {
+    const uint32_t w = k >> 5;
+    uint32_t h = (w * 2654435769u) >> (32 - __builtin_ctz(kSlots));
+    for (;;) {
+      const uint32_t was = atomicCAS(&word[h], kFree, w);
+      if (was == kFree || was == w) break;
+      h = (h + 1) & (kSlots - 1);
+    }
+    atomicOr(&mask[h], 1u << (k & 31));
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t h = tid; h < kSlots; h += kMarkThreads)
+    if (word[h] != kFree) atomicOr(&bits[word[h]], mask[h]);
 }
 
 __device__ inline uint32_t block_sum_u(uint32_t v, uint32_t* red) {
@@ -267,10 +293,15 @@ __global__ void voxel_tally_kernel(uint32_t* key, uint32_t n, const uint32_t* bi
   slot[i] = atomicAdd(&count[o], 1u);
 }
 
+// Voxels of up to kSortMax points are summed by half a wavefront or one, larger
+// ones by a workgroup each.
+constexpr uint32_t kSortMax = 1024;
+
 // Where each voxel's list starts: a workgroup takes one range for its voxels
-// (the lists' order does not matter).
+// (the lists' order does not matter).  The voxels of more than kSortMax points
+// are listed in crowd (used[0]: list words taken, used[1]: such voxels).
 __global__ __launch_bounds__(kVT) void voxel_alloc_kernel(const uint32_t* count, const uint32_t* total, uint32_t* start,
-                                                          uint32_t* used) {
+                                                          uint32_t* used, uint32_t* crowd) {
   __shared__ uint32_t red[kVT / 64];
   __shared__ uint32_t base;
   const uint32_t tid = threadIdx.x, o = blockIdx.x * kVT + tid, nv = *total;
@@ -289,6 +320,7 @@ __global__ __launch_bounds__(kVT) void voxel_alloc_kernel(const uint32_t* count,
   if (tid == kVT - 1) base = atomicAdd(used, r + c);
   __syncthreads();
   if (o < nv) start[o] = base + r;
+  if (c > kSortMax) crowd[atomicAdd(used + 1, 1u)] = o;
 }
 
 __global__ void voxel_place_kernel(const uint32_t* voxel, uint32_t n, const uint32_t* start, const uint32_t* slot,
@@ -299,21 +331,20 @@ __global__ void voxel_place_kernel(const uint32_t* voxel, uint32_t n, const uint
   if (o != kNoVoxel) list[start[o] + slot[i]] = i;  // < n: a voxel's slots cover exactly its count
 }
 
-// The centroids.  Half a wavefront takes a voxel of up to 32 points: it orders
-// them by index (a lane's rank is the number of smaller ones) and sums them in
-// that order.  A voxel of more points is taken by the whole wavefront, which
-// sorts their indices, or, past kSortMax points, searches all the cloud's points
-// for them.
-constexpr uint32_t kSortMax = 1024;
-__global__ __launch_bounds__(256) void voxel_average_kernel(const uint8_t* pts, uint32_t n, size_t stride,
-                                                            const uint32_t* voxel, const uint32_t* count,
+// The centroids of voxels of up to kSortMax points.  Half a wavefront takes a
+// voxel of up to 32: it orders them by index (a lane's rank is the number of
+// smaller ones) and sums them in that order.  A voxel of more points is taken by
+// the whole wavefront, which sorts their indices.
+__global__ __launch_bounds__(256) void voxel_average_kernel(const uint8_t* pts, size_t stride, const uint32_t* count,
                                                             const uint32_t* start, const uint32_t* list,
-                                                            const uint32_t* total, float* ox, float* oy, float* oz) {
+                                                            const uint32_t* total, const uint32_t* used, float* ox,
+                                                            float* oy, float* oz, uint32_t* host_crowd) {
   constexpr uint32_t kWaves = 4;
   __shared__ float xyz[kWaves][3][kSortMax];
   const int lane = lane_id(), l = lane & 31, half = lane >> 5;
   const uint32_t wave = threadIdx.x >> 6, nv = *total;
   float(&xs)[3][kSortMax] = xyz[wave];
+  if (blockIdx.x == 0 && threadIdx.x == 0) *host_crowd = used[1];
   auto put = [&](uint32_t at, uint32_t i) {
     const float* p = point_at(pts, stride, i);
     xs[0][at] = p[0];
@@ -346,78 +377,122 @@ __global__ __launch_bounds__(256) void voxel_average_kernel(const uint8_t* pts, 
       crowded &= crowded - 1;
       const uint32_t v = (uint32_t)__builtin_amdgcn_readlane((int)o, src);
       const uint32_t cv = (uint32_t)__builtin_amdgcn_readlane((int)c, src);
-      if (cv <= kSortMax) {  // bitonic sort of the listed points' indices in LDS
-        const uint32_t* const lv = list + start[v];
-        uint32_t* const si = reinterpret_cast<uint32_t*>(xs[0]);
-        uint32_t np = 64;
-        while (np < cv) np <<= 1;
-        wave_lds_sync();
+      if (cv > kSortMax) continue;
+      // bitonic sort of the listed points' indices in LDS
+      const uint32_t* const lv = list + start[v];
+      uint32_t* const si = reinterpret_cast<uint32_t*>(xs[0]);
+      uint32_t np = 64;
+      while (np < cv) np <<= 1;
+      wave_lds_sync();
 #pragma unroll
-        for (uint32_t k = 0; k < kSortMax / 64; ++k) {
-          const uint32_t j = k * 64 + lane;
-          if (k * 64 < np) si[j] = j < cv ? lv[j] : 0xffffffffu;
-        }
-        for (uint32_t k = 2; k <= np; k <<= 1) {
-          for (uint32_t d = k >> 1; d > 0; d >>= 1) {
-            wave_lds_sync();
-            for (uint32_t t = lane; t < np / 2; t += 64) {
-              const uint32_t p = 2 * t - (t & (d - 1)), q = p + d;
-              const uint32_t x = si[p], y = si[q];
-              if ((x > y) == ((p & k) == 0)) {
-                si[p] = y;
-                si[q] = x;
-              }
+      for (uint32_t k = 0; k < kSortMax / 64; ++k) {
+        const uint32_t j = k * 64 + lane;
+        if (k * 64 < np) si[j] = j < cv ? lv[j] : 0xffffffffu;
+      }
+      for (uint32_t k = 2; k <= np; k <<= 1) {
+        for (uint32_t d = k >> 1; d > 0; d >>= 1) {
+          wave_lds_sync();
+          for (uint32_t t = lane; t < np / 2; t += 64) {
+            const uint32_t p = 2 * t - (t & (d - 1)), q = p + d;
+            const uint32_t x = si[p], y = si[q];
+            if ((x > y) == ((p & k) == 0)) {
+              si[p] = y;
+              si[q] = x;
             }
           }
         }
-        wave_lds_sync();
-        uint32_t at[kSortMax / 64];
-#pragma unroll
-        for (uint32_t k = 0; k < kSortMax / 64; ++k) at[k] = k * 64 + lane < cv ? si[k * 64 + lane] : 0u;
-        wave_lds_sync();  // the indices have been read: the points go over them
-#pragma unroll
-        for (uint32_t k = 0; k < kSortMax / 64; ++k)
-          if (k * 64 + lane < cv) put(k * 64 + lane, at[k]);
-        wave_lds_sync();
-        if (lane < 3) sum(lane, 0, cv, v);
-        continue;
       }
-      constexpr uint32_t kAhead = 16;  // loads in flight
-      float sx = 0.f, sy = 0.f, sz = 0.f;
-      for (uint32_t j0 = 0; j0 < n; j0 += 64 * kAhead) {
-        uint32_t vx[kAhead];
+      wave_lds_sync();
+      uint32_t at[kSortMax / 64];
 #pragma unroll
-        for (uint32_t k = 0; k < kAhead; ++k) {
-          const uint32_t j = j0 + k * 64 + lane;
-          vx[k] = j < n ? voxel[j] : kNoVoxel;
-        }
+      for (uint32_t k = 0; k < kSortMax / 64; ++k) at[k] = k * 64 + lane < cv ? si[k * 64 + lane] : 0u;
+      wave_lds_sync();  // the indices have been read: the points go over them
 #pragma unroll
-        for (uint32_t k = 0; k < kAhead; ++k) {
-          uint64_t m = __ballot(vx[k] == v);
-          if (!m) continue;
-          float x = 0.f, y = 0.f, z = 0.f;
-          if (vx[k] == v) {
-            const float* p = point_at(pts, stride, j0 + k * 64 + lane);
-            x = p[0];
-            y = p[1];
-            z = p[2];
-          }
-          while (m) {
-            const int q = (int)__builtin_ctzll(m);
-            m &= m - 1;
-            sx += readlane_f(x, q);
-            sy += readlane_f(y, q);
-            sz += readlane_f(z, q);
-          }
-        }
-      }
-      if (lane == 0) {
-        ox[v] = sx / (float)cv;
-        oy[v] = sy / (float)cv;
-        oz[v] = sz / (float)cv;
-      }
+      for (uint32_t k = 0; k < kSortMax / 64; ++k)
+        if (k * 64 + lane < cv) put(k * 64 + lane, at[k]);
+      wave_lds_sync();
+      if (lane < 3) sum(lane, 0, cv, v);
     }
   }
+}
+
+// The centroids of the voxels in crowd, a workgroup each.  A voxel's points are
+// marked in a bitmap over the cloud's indices, kWindow of them at a time; its set
+// bits in order are the points in index order, gathered to LDS kVT at a time and
+// summed in that order.  Bound by the adds (three lanes, one dependent add per
+// point).  A wavefront that searched all the cloud's points for each such voxel
+// took 2.2 ms (900 voxels of 1,100 in 1,000,000 points); this takes 90 us.
+constexpr uint32_t kWindow = 1u << 18;
+__global__ __launch_bounds__(kVT) void voxel_crowded_kernel(const uint8_t* pts, uint32_t n, size_t stride,
+                                                            const uint32_t* count, const uint32_t* start,
+                                                            const uint32_t* list, const uint32_t* crowd, float* ox,
+                                                            float* oy, float* oz) {
+  constexpr uint32_t kPer = kWindow / 32 / kVT;  // bitmap words per thread
+  __shared__ uint32_t bits[kWindow / 32];
+  __shared__ uint32_t idx[kVT];
+  __shared__ float xyz[3][kVT];
+  __shared__ uint32_t red[kVT / 64];
+  const uint32_t tid = threadIdx.x, v = crowd[blockIdx.x], c = count[v];
+  const int lane = lane_id(), wave = tid >> 6;
+  const uint32_t* const lv = list + start[v];
+  float s = 0.f;  // threads 0, 1, 2: x, y, z
+  for (uint32_t w0 = 0; w0 < n; w0 += kWindow) {  // n <= kMaxBitmapPoints: no overflow
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) bits[k * kVT + tid] = 0u;
+    __syncthreads();
+    for (uint32_t j = tid; j < c; j += kVT) {
+      const uint32_t i = lv[j] - w0;  // wraps below the window
+      if (i < kWindow) atomicOr(&bits[i >> 5], 1u << (i & 31));
+    }
+    __syncthreads();
+    uint32_t w[kPer], own = 0;  // consecutive words
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) {
+      w[k] = bits[tid * kPer + k];
+      own += (uint32_t)__popc(w[k]);
+    }
+    uint32_t inc = own;
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t t = __shfl_up(inc, d);
+      if (lane >= d) inc += t;
+    }
+    if (lane == 63) red[wave] = inc;
+    __syncthreads();
+    uint32_t first = inc - own, cw = 0;  // this thread's first point's position, points in the window
+    for (uint32_t k = 0; k < kVT / 64; ++k) {
+      if (k < (uint32_t)wave) first += red[k];
+      cw += red[k];
+    }
+    for (uint32_t t0 = 0; t0 < cw; t0 += kVT) {  // uniform
+      uint32_t q = first;
+#pragma unroll
+      for (uint32_t k = 0; k < kPer; ++k) {
+        uint32_t m = w[k];
+        const uint32_t after = q + (uint32_t)__popc(m);
+        if (after > t0 && q < t0 + kVT) {
+          for (; m; m &= m - 1, ++q)
+            if (q - t0 < kVT) idx[q - t0] = w0 + (tid * kPer + k) * 32 + (uint32_t)__builtin_ctz(m);
+        }
+        q = after;
+      }
+      __syncthreads();
+      const uint32_t len = min((uint32_t)kVT, cw - t0);
+      if (tid < len) {
+        const float* p = point_at(pts, stride, idx[tid]);
+        xyz[0][tid] = p[0];
+        xyz[1][tid] = p[1];
+        xyz[2][tid] = p[2];
+      }
+      __syncthreads();
+      if (tid < 3) {
+#pragma unroll 8
+        for (uint32_t j = 0; j < len; ++j) s += xyz[tid][j];
+      }
+      // idx is written next, xyz only after another barrier
+    }
+    __syncthreads();  // red and bits have been read
+  }
+  if (tid < 3) (tid == 0 ? ox : tid == 1 ? oy : oz)[v] = s / (float)c;
 }
 
 }  // namespace
@@ -464,7 +539,7 @@ int voxel_grid_device(const void* d_pts, size_t n, size_t stride, float leaf, fl
   };
   struct Host {
     VoxelMeta meta;
-    uint32_t total;
+    uint32_t total, crowd;
   };
   constexpr size_t kPartAt = (sizeof(VoxelMeta) + 63) & ~(size_t)63;
   constexpr size_t kTotalAt = kPartAt + kBoundsBlocks * sizeof(VoxelBounds);
@@ -498,7 +573,7 @@ int voxel_grid_device(const void* d_pts, size_t n, size_t stride, float leaf, fl
   if (bitmap) {
     const uint32_t words = (uint32_t)(((uint64_t)lattice + 31) / 32), wp = (words + 3) & ~3u, np = (nn + 3) & ~3u;
     const uint32_t rank_blocks = (words + kRankWords - 1) / kRankWords;
-    A3D_TRY(grow(w.buf, false, (2 * (size_t)wp + 5 * (size_t)np + 4 + rank_blocks) * 4));
+    A3D_TRY(grow(w.buf, false, (2 * (size_t)wp + 5 * (size_t)np + 4 + rank_blocks + nn / kSortMax) * 4));
     uint32_t* const bits = static_cast<uint32_t*>(w.buf.p);  // cleared together with used and count
     uint32_t* const used = bits + wp;
     uint32_t* const count = used + 4;
@@ -508,18 +583,24 @@ int voxel_grid_device(const void* d_pts, size_t n, size_t stride, float leaf, fl
     uint32_t* const start = slot + np;
     uint32_t* const list = start + np;
     uint32_t* const sums = list + np;
+    uint32_t* const crowd = sums + rank_blocks;  // fewer than nn / kSortMax voxels hold more than kSortMax
     const uint32_t clear = (wp + 4 + np) / 4;
     voxel_clear_kernel<<<(clear + 255) / 256, 256, 0, s>>>(reinterpret_cast<uint4*>(bits), clear);
-    voxel_mark_kernel<<<blocks, 256, 0, s>>>(pts, nn, stride, meta, voxel, bits);
+    voxel_mark_kernel<<<(nn + kMarkThreads - 1) / kMarkThreads, kMarkThreads, 0, s>>>(pts, nn, stride, meta, voxel, bits);
     voxel_count_kernel<<<rank_blocks, kRankWords, 0, s>>>(bits, words, sums);
     voxel_rank_kernel<<<rank_blocks, kRankWords, 0, s>>>(bits, words, sums, before, total, &host->total);
     voxel_tally_kernel<<<blocks, 256, 0, s>>>(voxel, nn, bits, before, count, slot);
-    voxel_alloc_kernel<<<(nn + kVT - 1) / kVT, kVT, 0, s>>>(count, total, start, used);
+    voxel_alloc_kernel<<<(nn + kVT - 1) / kVT, kVT, 0, s>>>(count, total, start, used, crowd);
     voxel_place_kernel<<<blocks, 256, 0, s>>>(voxel, nn, start, slot, list);
-    voxel_average_kernel<<<std::min(1024u, (nn + 7) / 8), 256, 0, s>>>(pts, nn, stride, voxel, count, start, list,
-                                                                       total, d_x, d_y, d_z);
+    voxel_average_kernel<<<std::min(1024u, (nn + 7) / 8), 256, 0, s>>>(pts, stride, count, start, list, total, used,
+                                                                       d_x, d_y, d_z, &host->crowd);
     A3D_TRY(hipGetLastError());
     A3D_TRY(hipStreamSynchronize(s));
+    if (host->crowd) {
+      voxel_crowded_kernel<<<host->crowd, kVT, 0, s>>>(pts, nn, stride, count, start, list, crowd, d_x, d_y, d_z);
+      A3D_TRY(hipGetLastError());
+      A3D_TRY(hipStreamSynchronize(s));
+    }
     *out_n = host->total;
     return A3D_OK;
   }
