@@ -1565,20 +1565,27 @@ void split_pw(const GridDev& g, const FilterDev& f, uint32_t first, float* out, 
   }
 }
 
-// Launches of up to kSplitMax particles take the split form.  Weight kernel
-// alone, whole-cloud wavefronts of 16 against the split form at P = 4, 8, 16
-// (us, fixed-point cells; particles x points, map, spread):
+// Launches of up to kSplitMax particles take the split form, but for those that
+// fill a turn of whole-cloud workgroups (split_first).  Weight kernel alone,
+// whole-cloud wavefronts of 16 against the split form at P = 4, 8, 16 (us,
+// fixed-point cells; particles x points, map, spread):
 //   1,000 x 4,000 floor, tilted, 0.1 m      157    26   38   61
 //   2,000 x 4,000 floor, tilted, 0.5 m      192    47   45   73
 //   5,000 x 6,000 floor, tilted, 0.1 m      205    98   77   82
 //   5,000 x 6,000 floor, tilted, 1 m        268   130  133  154
 //   6,500 x 6,000 floor, tilted, 0.5 m      214   152  151  115
-//   12,000 x 6,000 floor, tilted, 0.1 m     208   231  153  132
-//   20,011 x 7,993 floor, tilted, 0.5 m     343   490  390  323
-//   28,000 x 5,000 floor, level, 0.1 m      177   413  262  249
+// and, with the rest of a turn split where the rule says so, at P = 16 only:
+//   12,288 x 6,000 floor, tilted, 0.1 / 1 m  -            130 / 260
+//   12,400 x 6,000 floor, tilted, 0.1 / 1 m 187 / 218     173 / 279
+//   14,000 x 6,000 floor, tilted, 0.1 / 1 m 186 / 213     199 / 346
+//   16,900 x 6,000 floor, tilted, 0.1 / 1 m 217 / 244     202 / 350
+//   20,480 x 6,000 floor, tilted, 0.1 / 1 m 229 / 369     203 / 393
+//   24,000 x 6,000 floor, tilted, 0.1 / 1 m 231 / 358       -
+//   28,000 x 5,000 floor, level, 0.1 m      177           249
 // Small P is bound by the adding wavefront (one dependent add per point, 4.6
-// ns), larger P by the gathers; from 20,000 particles on there are enough
-// whole-cloud wavefronts, which share more lines per workgroup (64 particles).
+// ns), larger P by the gathers and by its own turns (256 CUs x 3 x 16 = 12,288);
+// from 20,000 particles on there are enough whole-cloud wavefronts, which share
+// more lines per workgroup (64 particles).
 constexpr uint32_t kSplit4Max = 2048, kSplit8Max = 5632, kSplitMax = 20480;
 
 template <bool KFILTER>
@@ -1599,11 +1606,16 @@ bool order_pays(uint32_t n) { return current_mapping() != 0 || n > kSplit4Max; }
 // (98,304 particles x 20,000 points take 1,313 us, 100,000 took 1,529). So up to
 // kSplit4Max particles past a whole number of turns go to the split form (92 us
 // for these 1,696), for clouds of kTurnPoints points or more.
+// From three quarters of the first turn on, and a little past it, whole-cloud
+// workgroups are the better form: with the split form 14,000 x 6,000 over 1 m took
+// 346 us, 213 by them, and a sliver past the turn costs them little (16,385 x
+// 1,500 over 1 m 129 and 90 us).
 constexpr uint32_t kCus = 256, kTurnPoints = 2048;
 
 uint32_t split_first(uint32_t n, uint32_t m, uint32_t per_block) {
-  if (n <= kSplitMax) return 0;
-  const uint32_t rest = n % (kCus * per_block);
+  const uint32_t turn = kCus * per_block;
+  if (n <= kSplitMax && (n <= turn / 4 * 3 || n > turn + turn / 64)) return 0;
+  const uint32_t rest = n % turn;
   return rest <= kSplit4Max && m >= kTurnPoints ? n - rest : n;
 }
 
