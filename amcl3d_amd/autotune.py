@@ -15,6 +15,10 @@ LDS cloud tile):
   * persistent launches (fleets, served batches) add a fifth element, how the
     work list is dealt to the XCDs: 0 contiguous ranges, k runs of k blocks
     round-robin.
+Single filters and poses that do not fill the chip (up to 20,480 particles, but
+for 12,289 to 16,640 at ppw 16) have a shape of their own in mapping 0: ppw, tile
+and, up to 2,048 particles, order have no effect there, so one candidate of
+mapping 0 is enough for them.
 Every shape gives bit-identical results, so the choice is purely a timing
 one: run the caller's workload once per candidate (after one untimed warm-up)
 and keep the fastest.

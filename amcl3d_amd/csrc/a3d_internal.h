@@ -261,9 +261,10 @@ int current_ppw();
 // Points per LDS cloud tile of the particle-lane kernels (32, 64, 128, 256).
 int clamp_chunk(int points);
 int current_chunk();
-// The same for a single filter or explicit poses: 256 unless the caller has set
-// a tile (100,000 x 20,000: 1,446 us against 1,530 at 64; no other shape
-// measured slower with it).
+// The same for a single filter or explicit poses: 256 at the default setting
+// (100,000 x 20,000: 1,446 us against 1,530 at 64; no other shape measured slower
+// with it), any other setting as it is.  The default is a value of the setting,
+// not a state beside it, so a caller that saves and restores it changes nothing.
 int single_chunk();
 // Work-list dealing of persistent (fleet, served) launches: 0 contiguous
 // ranges per XCD, k > 0 runs of k items dealt round-robin.

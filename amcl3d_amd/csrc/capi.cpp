@@ -18,8 +18,8 @@ namespace a3d {
 
 static thread_local std::string g_err;
 static int g_ppw = 16;
-static int g_chunk = 64;  // points per LDS cloud tile (particle-lane kernels)
-static bool g_chunk_set = false;  // by the caller
+constexpr int kDefaultChunk = 64;
+static int g_chunk = kDefaultChunk;  // points per LDS cloud tile (particle-lane kernels)
 static int g_deal = 0;    // work-list dealing of persistent launches
 static int g_mapping = A3D_MAP_PARTICLE_LANES;
 static int g_order = A3D_ORDER_SPATIAL;
@@ -33,7 +33,7 @@ int fail(int code, const std::string& msg) {
 
 int current_ppw() { return g_ppw; }
 int current_chunk() { return g_chunk; }
-int single_chunk() { return g_chunk_set ? g_chunk : 256; }
+int single_chunk() { return g_chunk == kDefaultChunk ? 256 : g_chunk; }
 int current_deal() { return g_deal; }
 int current_mapping() { return g_mapping; }
 int current_order() { return g_order; }
@@ -404,7 +404,6 @@ int a3d_set_cloud_tile(int points) {
   if (points != 32 && points != 64 && points != 128 && points != 256)
     return fail(A3D_ERR_ARG, "a3d_set_cloud_tile: points per tile must be 32, 64, 128 or 256");
   g_chunk = points;
-  g_chunk_set = true;
   return A3D_OK;
 }
 

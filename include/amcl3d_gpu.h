@@ -219,15 +219,21 @@ int a3d_pf_timing(a3d_pf* pf, int reset, double* weight_ms_avg, uint64_t* launch
  * particles (64, 32 or 16), each lane one particle and 64/particles_per_wave
  * consecutive points per step.  A3D_MAP_POINT_LANES: lanes are 64
  * consecutive points, a wavefront walks the cloud for `particles_per_wave`
- * particles through an LDS tile. */
+ * particles through an LDS tile.
+ * Single filters and poses that do not fill the chip (up to 20,480 particles,
+ * but for those from three quarters of a turn of whole-cloud workgroups to 1/64
+ * past it, 12,289 to 16,640 at 16 per wavefront, and the rest of a turn of larger
+ * ones) have a shape of their own in the particle-lane mapping: tile and cloud
+ * tile have no effect on it, and up to 2,048 particles are visited in index
+ * order whatever the order set. */
 enum { A3D_MAP_PARTICLE_LANES = 0, A3D_MAP_POINT_LANES = 1 };
 int a3d_set_tile(int particles_per_wave);
 int a3d_get_tile(int* particles_per_wave);
 /* Points of the cloud staged per LDS tile by the A3D_MAP_PARTICLE_LANES
- * kernels (32, 64, 128 or 256; default 64, and 256 in single-filter and pose
- * launches until it is set): the workgroup's wavefronts walk the cloud one
- * tile at a time, one barrier per tile.  Point-lane kernels
- * always stage 64 (one point per lane). */
+ * kernels (32, 64, 128 or 256): the workgroup's wavefronts walk the cloud one
+ * tile at a time, one barrier per tile.  At 64, the default, single-filter and
+ * pose launches stage 256 points; the other values hold for every launch.
+ * Point-lane kernels always stage 64 (one point per lane). */
 int a3d_set_cloud_tile(int points);
 int a3d_get_cloud_tile(int* points);
 /* How persistent launches (fleets, served batches) deal their work list of
@@ -242,9 +248,10 @@ int a3d_set_mapping(int mapping);
 int a3d_get_mapping(int* mapping);
 /* Order in which the cloud-weight kernel visits a filter's particles (the
  * particles themselves stay in index order; results are identical):
- * A3D_ORDER_INDEX, or A3D_ORDER_SPATIAL, a counting sort by a Morton code of
- * (x, y, z, yaw) over the particles' bounding box, computed on the device
- * before each single-filter update. */
+ * A3D_ORDER_INDEX, or A3D_ORDER_SPATIAL, a counting sort by the leading bits of
+ * x, y, z and yaw around the particles' mean, computed on the device before each
+ * update (in the particle-lane mapping, of single filters of more than 2,048
+ * particles). */
 enum { A3D_ORDER_INDEX = 0, A3D_ORDER_SPATIAL = 1 };
 int a3d_set_order(int order);
 int a3d_get_order(int* order);
