@@ -238,8 +238,8 @@ struct a3d_pf {
   float* x = nullptr;  // one allocation: x y z a w wp wr
   float* scratch = nullptr;
   uint8_t* inmap = nullptr;
-  float* mean = nullptr;  // 4 floats of pinned host memory, written by the update's last kernel
-  PoolBuf mean_buf;
+  float* mean = nullptr;  // mean_buf's 4 floats, written by the update's last kernel; null before the first particles
+  PoolBuf mean_buf;       // pinned host memory, device memory where there is none
   uint32_t* idx = nullptr;
   void* ord = nullptr;     // particle visiting order buffers (order_view)
   float* stage = nullptr;  // host-input staging
@@ -604,10 +604,10 @@ int a3d_grid_cloud_weight(const a3d_grid* g, const float* x, const float* y, con
   const size_t in = 3 * m + 4 * n;
   const bool ordered = g_order == A3D_ORDER_SPATIAL && order_pays((uint32_t)n) && (double)n * (double)m >= kPoseOrderMin;
   const size_t dev_floats = (in + n + 64 + 63) & ~(size_t)63;  // 2 * kZrParts of the spare ones for the z ranges
-  const bool pinned = (in + n) * 4 <= kPinnedMax;
   Pooled d, h;
-  if (!d.take(false, dev_floats * 4 + (ordered ? order_bytes((uint32_t)n) : 0)) || (pinned && !h.take(true, (in + n) * 4)))
+  if (!d.take(false, dev_floats * 4 + (ordered ? order_bytes((uint32_t)n) : 0)))
     return fail(A3D_ERR_NOMEM, "a3d_grid_cloud_weight: staging");
+  const bool pinned = (in + n) * 4 <= kPinnedMax && h.take(true, (in + n) * 4);
   const float* const src[7] = {x, y, z, tx, ty, tz, yaw};
   hipStream_t s = g->stream;
   float* at = pinned ? h.f() : d.f();
@@ -725,7 +725,7 @@ int a3d_pf_create(a3d_pf** out) {
     delete p;
     return fail(A3D_ERR_HIP, "a3d_pf_create: cannot create a stream");
   }
-  if (!pool_take(p->mean_buf, true, 16)) {
+  if (!pool_take(p->mean_buf, true, 16) && !pool_take(p->mean_buf, false, 16)) {
     (void)hipStreamDestroy(p->stream);
     delete p;
     return fail(A3D_ERR_NOMEM, "a3d_pf_create: cannot allocate the mean");
@@ -759,6 +759,19 @@ int a3d_pf_destroy(a3d_pf* p) {
   return A3D_OK;
 }
 
+// A mean of zeros; the stream is idle.
+static int pf_clear_mean(a3d_pf* p) {
+  p->mean = static_cast<float*>(p->mean_buf.p);
+  if (p->mean_buf.host) {
+    std::fill(p->mean, p->mean + 4, 0.0f);
+    return A3D_OK;
+  }
+  launch_zero_u32(reinterpret_cast<uint32_t*>(p->mean), 4, p->stream);
+  A3D_HIP(hipGetLastError());
+  A3D_HIP(hipStreamSynchronize(p->stream));
+  return A3D_OK;
+}
+
 // Resizes the particle set like std::vector::resize: surviving particles keep
 // their values, new ones are zero (Particle() constructor).
 static int pf_resize(a3d_pf* p, uint32_t n) {
@@ -787,12 +800,10 @@ static int pf_resize(a3d_pf* p, uint32_t n) {
   p->x = x;
   p->scratch = sc;
   p->inmap = in;
-  p->mean = static_cast<float*>(p->mean_buf.p);  // the stream is idle
-  std::fill(p->mean, p->mean + 4, 0.0f);
   p->idx = idx;
   p->ord = ord;
   p->n = n;
-  return A3D_OK;
+  return pf_clear_mean(p);
 }
 
 static int pf_stage(a3d_pf* p, size_t floats) { return ensure_stage(p->stage, p->stage_cap, floats); }
@@ -940,8 +951,7 @@ int a3d_pf_update(a3d_pf* p, const a3d_grid* g, const float* x, const float* y, 
     }
     rc = a3d_pf_set_particles(p, pp.data(), p->n);
     if (rc) return rc;
-    std::fill(p->mean, p->mean + 4, 0.0f);  // set_particles left the stream idle
-    return A3D_OK;
+    return pf_clear_mean(p);  // set_particles left the stream idle
   }
   int rc = pf_stage(p, 3 * m + 4 * nb + 16);
   if (rc) return rc;
@@ -1039,8 +1049,9 @@ int a3d_pf_get_mean(const a3d_pf* p, float mean[4]) {
     std::fill(mean, mean + 4, 0.f);
     return A3D_OK;
   }
+  if (!p->mean_buf.host) A3D_HIP(hipMemcpyAsync(mean, p->mean, 16, hipMemcpyDeviceToHost, p->stream));
   A3D_HIP(hipStreamSynchronize(p->stream));
-  std::copy(p->mean, p->mean + 4, mean);
+  if (p->mean_buf.host) std::copy(p->mean, p->mean + 4, mean);
   return A3D_OK;
 }
 

@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstdlib>
 #include <mutex>
 #include <vector>
 
@@ -36,11 +37,21 @@ void release(const PoolBuf& b) {
     (void)hipFree(b.p);
 }
 
+// Test knob: A3D_NO_PINNED=1, read once, refuses pinned memory.
+bool no_pinned() {
+  static const bool no = [] {
+    const char* v = std::getenv("A3D_NO_PINNED");
+    return v && v[0] == '1';
+  }();
+  return no;
+}
+
 hipError_t fresh(PoolBuf& b) { return b.host ? hipHostMalloc(&b.p, b.bytes, hipHostMallocDefault) : hipMalloc(&b.p, b.bytes); }
 
 }  // namespace
 
 bool pool_take(PoolBuf& out, bool host, size_t bytes) {
+  if (host && no_pinned()) return false;
   PoolBuf b{};
   b.host = host;
   b.bytes = kSmallest;  // powers of two, then whole steps of kStep
@@ -70,7 +81,10 @@ bool pool_take(PoolBuf& out, bool host, size_t bytes) {
     }
     for (const PoolBuf& c : drop) release(c);
     b.p = nullptr;
-    if (fresh(b) != hipSuccess) return false;
+    if (fresh(b) != hipSuccess) {
+      (void)hipGetLastError();  // the caller may go on without: no later check reports this
+      return false;
+    }
   }
   out = b;
   return true;

@@ -543,16 +543,27 @@ int voxel_grid_device(const void* d_pts, size_t n, size_t stride, float leaf, fl
   };
   constexpr size_t kPartAt = (sizeof(VoxelMeta) + 63) & ~(size_t)63;
   constexpr size_t kTotalAt = kPartAt + kBoundsBlocks * sizeof(VoxelBounds);
-  A3D_TRY(grow(w.meta, false, kTotalAt + 64));
-  A3D_TRY(grow(w.host, true, sizeof(Host)));
-  VoxelMeta* const meta = static_cast<VoxelMeta*>(w.meta.p);
-  VoxelBounds* const part = reinterpret_cast<VoxelBounds*>(static_cast<uint8_t*>(w.meta.p) + kPartAt);
-  uint32_t* const total = reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(w.meta.p) + kTotalAt);
-  Host* const host = static_cast<Host*>(w.host.p);
+  constexpr size_t kHostAt = kTotalAt + 64;
+  A3D_TRY(grow(w.meta, false, kHostAt + sizeof(Host)));
+  uint8_t* const rec = static_cast<uint8_t*>(w.meta.p);
+  VoxelMeta* const meta = reinterpret_cast<VoxelMeta*>(rec);
+  VoxelBounds* const part = reinterpret_cast<VoxelBounds*>(rec + kPartAt);
+  uint32_t* const total = reinterpret_cast<uint32_t*>(rec + kTotalAt);
+  // the kernels write the host's record to pinned memory, or, where there is
+  // none, beside the rest, and it is copied
+  const bool pinned = grow(w.host, true, sizeof(Host)) == hipSuccess;
+  Host copy{};
+  Host* const out = pinned ? static_cast<Host*>(w.host.p) : reinterpret_cast<Host*>(rec + kHostAt);
+  const Host* const host = pinned ? out : &copy;
+  auto wait = [&]() {
+    const hipError_t e = pinned ? hipSuccess : hipMemcpyAsync(&copy, out, sizeof(Host), hipMemcpyDeviceToHost, s);
+    const hipError_t done = hipStreamSynchronize(s);
+    return e != hipSuccess ? e : done;
+  };
   voxel_bounds_kernel<<<kBoundsBlocks, kVT, 0, s>>>(pts, nn, stride, part);
-  voxel_meta_kernel<<<1, 64, 0, s>>>(part, leaf, meta, &host->meta);
+  voxel_meta_kernel<<<1, 64, 0, s>>>(part, leaf, meta, &out->meta);
   A3D_TRY(hipGetLastError());
-  A3D_TRY(hipStreamSynchronize(s));
+  A3D_TRY(wait());
   const VoxelMeta hm = host->meta;
   if (hm.nfin == 0) return A3D_OK;
   if (hm.overflow) {  // PCL: integer indices would overflow, output = input
@@ -588,14 +599,14 @@ int voxel_grid_device(const void* d_pts, size_t n, size_t stride, float leaf, fl
     voxel_clear_kernel<<<(clear + 255) / 256, 256, 0, s>>>(reinterpret_cast<uint4*>(bits), clear);
     voxel_mark_kernel<<<(nn + kMarkThreads - 1) / kMarkThreads, kMarkThreads, 0, s>>>(pts, nn, stride, meta, voxel, bits);
     voxel_count_kernel<<<rank_blocks, kRankWords, 0, s>>>(bits, words, sums);
-    voxel_rank_kernel<<<rank_blocks, kRankWords, 0, s>>>(bits, words, sums, before, total, &host->total);
+    voxel_rank_kernel<<<rank_blocks, kRankWords, 0, s>>>(bits, words, sums, before, total, &out->total);
     voxel_tally_kernel<<<blocks, 256, 0, s>>>(voxel, nn, bits, before, count, slot);
     voxel_alloc_kernel<<<(nn + kVT - 1) / kVT, kVT, 0, s>>>(count, total, start, used, crowd);
     voxel_place_kernel<<<blocks, 256, 0, s>>>(voxel, nn, start, slot, list);
     voxel_average_kernel<<<std::min(1024u, (nn + 7) / 8), 256, 0, s>>>(pts, stride, count, start, list, total, used,
-                                                                       d_x, d_y, d_z, &host->crowd);
+                                                                       d_x, d_y, d_z, &out->crowd);
     A3D_TRY(hipGetLastError());
-    A3D_TRY(hipStreamSynchronize(s));
+    A3D_TRY(wait());
     if (host->crowd) {
       voxel_crowded_kernel<<<host->crowd, kVT, 0, s>>>(pts, nn, stride, count, start, list, crowd, d_x, d_y, d_z);
       A3D_TRY(hipGetLastError());
