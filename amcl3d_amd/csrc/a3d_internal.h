@@ -309,6 +309,16 @@ struct PoolBuf {
 };
 bool pool_take(PoolBuf& out, bool host, size_t bytes);
 void pool_give(PoolBuf& b);
+// hipMalloc; where device memory runs out the pool's idle buffers are freed first.
+// No error is left for a later check to report.
+hipError_t dev_malloc_bytes(void** p, size_t bytes);
+template <class T>
+hipError_t dev_malloc(T** p, size_t bytes) {
+  void* v = nullptr;
+  const hipError_t e = dev_malloc_bytes(&v, bytes);
+  *p = static_cast<T*>(v);
+  return e;
+}
 struct Pooled : PoolBuf {  // given back at the end of its scope
   Pooled() = default;
   Pooled(const Pooled&) = delete;

@@ -275,7 +275,7 @@ static int ensure_stage(float*& buf, size_t& cap, size_t floats) {
   buf = nullptr;
   cap = 0;
   const size_t want = std::max(floats, (size_t)1 << 16);
-  A3D_HIP(hipMalloc(&buf, want * sizeof(float)));
+  A3D_HIP(dev_malloc(&buf, want * sizeof(float)));
   cap = want;
   return A3D_OK;
 }
@@ -314,7 +314,7 @@ int a3d_device_synchronize(void) {
 int a3d_buffer_alloc(size_t bytes, void** dptr) {
   if (!dptr || bytes == 0) return fail(A3D_ERR_ARG, "a3d_buffer_alloc: null output or zero size");
   *dptr = nullptr;
-  if (hipMalloc(dptr, bytes) != hipSuccess) return fail(A3D_ERR_NOMEM, "a3d_buffer_alloc: hipMalloc failed");
+  if (dev_malloc(dptr, bytes) != hipSuccess) return fail(A3D_ERR_NOMEM, "a3d_buffer_alloc: hipMalloc failed");
   return A3D_OK;
 }
 
@@ -468,11 +468,11 @@ static int grid_alloc(const double mn[3], const double mx[3], double res, double
   G->sensor_dev = sensor_dev;
   const size_t bytes = G->g.cells * sizeof(float);
   // one more float, 0, after the last cell: the cell that rejected points read
-  if (hipMalloc(&G->prob, prob_alloc_bytes(G->g)) != hipSuccess) {
+  if (dev_malloc(&G->prob, prob_alloc_bytes(G->g)) != hipSuccess) {
     delete G;
     return fail(A3D_ERR_NOMEM, "grid: cannot allocate " + std::to_string(bytes) + " bytes of prob");
   }
-  if (keep_dist && hipMalloc(&G->dist, bytes) != hipSuccess) {
+  if (keep_dist && dev_malloc(&G->dist, bytes) != hipSuccess) {
     (void)hipFree(G->prob);
     delete G;
     return fail(A3D_ERR_NOMEM, "grid: cannot allocate the distance field");
@@ -781,8 +781,8 @@ static int pf_resize(a3d_pf* p, uint32_t n) {
   uint8_t* in = nullptr;
   uint32_t* idx = nullptr;
   void* ord = nullptr;
-  if (hipMalloc(&x, 7 * (size_t)n * 4) != hipSuccess || hipMalloc(&sc, scratch_floats(n) * 4) != hipSuccess ||
-      hipMalloc(&in, n) != hipSuccess || hipMalloc(&idx, (size_t)n * 4) != hipSuccess || hipMalloc(&ord, order_bytes(n)) != hipSuccess) {
+  if (dev_malloc(&x, 7 * (size_t)n * 4) != hipSuccess || dev_malloc(&sc, scratch_floats(n) * 4) != hipSuccess ||
+      dev_malloc(&in, n) != hipSuccess || dev_malloc(&idx, (size_t)n * 4) != hipSuccess || dev_malloc(&ord, order_bytes(n)) != hipSuccess) {
     (void)hipFree(x);
     (void)hipFree(sc);
     (void)hipFree(in);

@@ -97,7 +97,7 @@ static int grow(float*& buf, size_t& cap, size_t floats, hipStream_t s) {
   buf = nullptr;
   cap = 0;
   const size_t want = std::max(floats, (size_t)1 << 16);
-  if (hipMalloc(&buf, want * sizeof(float)) != hipSuccess) return fail(A3D_ERR_NOMEM, "fleet: staging allocation");
+  if (dev_malloc(&buf, want * sizeof(float)) != hipSuccess) return fail(A3D_ERR_NOMEM, "fleet: staging allocation");
   cap = want;
   return A3D_OK;
 }
@@ -128,7 +128,7 @@ static int build_items(a3d_fleet* fl, const uint32_t* m) {
     (void)hipFree(fl->d_items);
     fl->d_items = nullptr;
     fl->items_cap = 0;
-    if (hipMalloc(&fl->d_items, items.size() * sizeof(WorkItem)) != hipSuccess)
+    if (dev_malloc(&fl->d_items, items.size() * sizeof(WorkItem)) != hipSuccess)
       return fail(A3D_ERR_NOMEM, "fleet: work list allocation");
     fl->items_cap = items.size();
   }
@@ -210,16 +210,16 @@ int a3d_fleet_create(size_t nfilters, const uint32_t* num_particles, a3d_fleet**
     return fail(A3D_ERR_ARG, "a3d_fleet_create: more than 2^32 particles");
   }
   bool ok = hipStreamCreateWithFlags(&fl->stream, hipStreamNonBlocking) == hipSuccess &&
-            hipMalloc(&fl->state, 7 * fl->total * 4) == hipSuccess &&
-            hipMalloc(&fl->scratch, fl->soff[nfilters] * 4) == hipSuccess &&
-            hipMalloc(&fl->inmap, fl->total) == hipSuccess && hipMalloc(&fl->mean, 16 * nfilters) == hipSuccess &&
-            hipMalloc(&fl->d_filters, sizeof(FilterDev) * nfilters) == hipSuccess &&
-            hipMalloc(&fl->d_counter, 64) == hipSuccess;
+            dev_malloc(&fl->state, 7 * fl->total * 4) == hipSuccess &&
+            dev_malloc(&fl->scratch, fl->soff[nfilters] * 4) == hipSuccess &&
+            dev_malloc(&fl->inmap, fl->total) == hipSuccess && dev_malloc(&fl->mean, 16 * nfilters) == hipSuccess &&
+            dev_malloc(&fl->d_filters, sizeof(FilterDev) * nfilters) == hipSuccess &&
+            dev_malloc(&fl->d_counter, 64) == hipSuccess;
   fl->ooff.assign(nfilters + 1, 0);
   for (size_t f = 0; f < nfilters; ++f) fl->ooff[f + 1] = fl->ooff[f] + order_stride(fl->n[f]);
   if (ok)
-    ok = hipMalloc(&fl->ord, fl->ooff[nfilters]) == hipSuccess &&
-         hipMalloc(&fl->d_ord, sizeof(OrderDev) * nfilters) == hipSuccess;
+    ok = dev_malloc(&fl->ord, fl->ooff[nfilters]) == hipSuccess &&
+         dev_malloc(&fl->d_ord, sizeof(OrderDev) * nfilters) == hipSuccess;
   if (ok) {
     fl->h_ord.resize(nfilters);
     for (size_t f = 0; f < nfilters; ++f) fl->h_ord[f] = order_view(fl->ord + fl->ooff[f], fl->n[f]);
@@ -504,7 +504,7 @@ int a3d_fleet_set_layout(a3d_fleet* fl, const uint32_t* m, const uint32_t* nb) {
   }
   fl->layout = false;
   fl->staged = false;
-  if (!fl->d_lay && hipMalloc(&fl->d_lay, lay.size() * sizeof(uint64_t)) != hipSuccess) {
+  if (!fl->d_lay && dev_malloc(&fl->d_lay, lay.size() * sizeof(uint64_t)) != hipSuccess) {
     fl->d_lay = nullptr;
     return fail(A3D_ERR_NOMEM, "a3d_fleet_set_layout: device allocation failed");
   }

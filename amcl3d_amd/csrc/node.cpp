@@ -244,8 +244,8 @@ int a3d_node_create(const a3d_node_params* params, const a3d_grid* grid, uint64_
     delete nd;
     return rc;
   }
-  if (hipMalloc(&nd->d_z4, 16 * (size_t)params->num_particles) != hipSuccess ||
-      hipMalloc(&nd->d_u01, 4) != hipSuccess || hipMalloc(&nd->d_key, 16) != hipSuccess ||
+  if (dev_malloc(&nd->d_z4, 16 * (size_t)params->num_particles) != hipSuccess ||
+      dev_malloc(&nd->d_u01, 4) != hipSuccess || dev_malloc(&nd->d_key, 16) != hipSuccess ||
       !(nd->vws = voxel_workspace_new())) {
     a3d_node_destroy(nd);
     return fail(A3D_ERR_NOMEM, "a3d_node_create: cannot allocate the draw buffers");
@@ -363,14 +363,14 @@ int a3d_node_point_cloud(a3d_node* nd, int64_t now_ns, const void* points, size_
       (void)hipFree(nd->d_raw);
       nd->d_raw = nullptr;
       nd->raw_cap = 0;
-      if (hipMalloc(&nd->d_raw, n * stride) != hipSuccess) return fail(A3D_ERR_NOMEM, "a3d_node_point_cloud: scan");
+      if (dev_malloc(&nd->d_raw, n * stride) != hipSuccess) return fail(A3D_ERR_NOMEM, "a3d_node_point_cloud: scan");
       nd->raw_cap = n * stride;
     }
     if (n > nd->v_cap) {
       (void)hipFree(nd->d_v);
       nd->d_v = nullptr;
       nd->v_cap = 0;
-      if (hipMalloc(&nd->d_v, 3 * n * sizeof(float)) != hipSuccess)
+      if (dev_malloc(&nd->d_v, 3 * n * sizeof(float)) != hipSuccess)
         return fail(A3D_ERR_NOMEM, "a3d_node_point_cloud: voxels");
       nd->v_cap = n;
     }
@@ -378,7 +378,7 @@ int a3d_node_point_cloud(a3d_node* nd, int64_t now_ns, const void* points, size_
       (void)hipFree(nd->d_rng);
       nd->d_rng = nullptr;
       nd->rng_cap = 0;
-      if (hipMalloc(&nd->d_rng, nr * sizeof(float)) != hipSuccess)
+      if (dev_malloc(&nd->d_rng, nr * sizeof(float)) != hipSuccess)
         return fail(A3D_ERR_NOMEM, "a3d_node_point_cloud: ranges");
       nd->rng_cap = nr;
     }

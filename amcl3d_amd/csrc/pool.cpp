@@ -1,8 +1,11 @@
 // Buffers for the length of one call: device memory and pinned host memory that
 // kernels read and write directly.  hipMalloc, hipFree and pinning cost tens of
 // microseconds each, as much as the smallest calls' kernels, so a returned
-// buffer is kept for the next call of any thread, as long as the idle buffers of
-// its kind fit kIdleMax; a buffer is given back only once no stream uses it.
+// buffer is kept for the next call of any thread; a buffer is given back only
+// once no stream uses it.  The idle buffers of a kind take at most kIdleMax: one
+// more frees those given back longest ago, so a large call's buffers don't keep
+// the sizes in use out.  They are all freed when device memory runs out, also
+// for what does not come from here (dev_malloc).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -48,6 +51,19 @@ bool no_pinned() {
 
 hipError_t fresh(PoolBuf& b) { return b.host ? hipHostMalloc(&b.p, b.bytes, hipHostMallocDefault) : hipMalloc(&b.p, b.bytes); }
 
+// Gives the idle buffers back, after an allocation that failed.
+void drain() {
+  (void)hipGetLastError();
+  std::vector<PoolBuf> drop;
+  Pool& P = pool();
+  {
+    std::lock_guard<std::mutex> lock(P.mu);
+    drop.swap(P.idle);
+    P.bytes[0] = P.bytes[1] = 0;
+  }
+  for (const PoolBuf& c : drop) release(c);
+}
+
 }  // namespace
 
 bool pool_take(PoolBuf& out, bool host, size_t bytes) {
@@ -71,15 +87,8 @@ bool pool_take(PoolBuf& out, bool host, size_t bytes) {
       }
     }
   }
-  if (fresh(b) != hipSuccess) {  // give the idle ones back and try again
-    (void)hipGetLastError();
-    std::vector<PoolBuf> drop;
-    {
-      std::lock_guard<std::mutex> lock(P.mu);
-      drop.swap(P.idle);
-      P.bytes[0] = P.bytes[1] = 0;
-    }
-    for (const PoolBuf& c : drop) release(c);
+  if (fresh(b) != hipSuccess) {
+    drain();
     b.p = nullptr;
     if (fresh(b) != hipSuccess) {
       (void)hipGetLastError();  // the caller may go on without: no later check reports this
@@ -93,20 +102,39 @@ bool pool_take(PoolBuf& out, bool host, size_t bytes) {
 void pool_give(PoolBuf& b) {
   if (!b.p) return;
   Pool& P = pool();
-  {
+  std::vector<PoolBuf> drop;
+  try {  // destructors come here: no exception leaves
     std::lock_guard<std::mutex> lock(P.mu);
-    if (P.bytes[b.host] + b.bytes <= kIdleMax[b.host]) {
-      try {  // destructors come here: no exception leaves
-        P.idle.push_back(b);
-        P.bytes[b.host] += b.bytes;
-        b.p = nullptr;
-        return;
-      } catch (...) {
+    if (b.bytes <= kIdleMax[b.host]) {
+      P.idle.push_back(b);
+      P.bytes[b.host] += b.bytes;
+      b.p = nullptr;
+      for (size_t i = 0; P.bytes[b.host] > kIdleMax[b.host];) {  // ends before the one just added
+        if (P.idle[i].host != b.host) {
+          ++i;
+          continue;
+        }
+        drop.push_back(P.idle[i]);
+        P.bytes[b.host] -= P.idle[i].bytes;
+        P.idle.erase(P.idle.begin() + (ptrdiff_t)i);
       }
     }
+  } catch (...) {  // no room for the lists: the bound is kept by the next call
   }
-  release(b);
+  if (b.p) release(b);
   b.p = nullptr;
+  for (const PoolBuf& c : drop) release(c);
+}
+
+hipError_t dev_malloc_bytes(void** p, size_t bytes) {
+  *p = nullptr;
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipSuccess) return e;
+  drain();
+  *p = nullptr;
+  e = hipMalloc(p, bytes);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
 }
 
 }  // namespace a3d

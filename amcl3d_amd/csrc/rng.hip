@@ -96,8 +96,8 @@ extern "C" int a3d_session_draws(uint64_t seed, uint64_t step, int num_particles
   uint64_t* dp = nullptr;
   float* du = nullptr;
   int rc = A3D_OK;
-  if (hipMalloc(&dz, 4 * (size_t)n * 4) != hipSuccess || hipMalloc(&dp, 16) != hipSuccess ||
-      hipMalloc(&du, 4) != hipSuccess) {
+  if (dev_malloc(&dz, 4 * (size_t)n * 4) != hipSuccess || dev_malloc(&dp, 16) != hipSuccess ||
+      dev_malloc(&du, 4) != hipSuccess) {
     rc = fail(A3D_ERR_NOMEM, "a3d_session_draws: allocation");
   } else {
     const uint64_t h[2] = {seed, step};

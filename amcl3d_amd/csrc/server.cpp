@@ -144,7 +144,7 @@ bool grow_dev(T*& p, size_t& cap, size_t count) {
   p = nullptr;
   cap = 0;
   const size_t want = std::max(count, (size_t)1024) * 3 / 2;
-  if (hipMalloc(&p, want * sizeof(T)) != hipSuccess) return false;
+  if (dev_malloc(&p, want * sizeof(T)) != hipSuccess) return false;
   cap = want;
   return true;
 }
@@ -198,9 +198,9 @@ static int alloc_session(a3d_server* S, Session& se) {
   se.bytes = 7 * n * 4 + scratch_floats((uint32_t)n) * 4 + n + 64 + order_stride((uint32_t)n);
   if (S->hbm_used + se.bytes > S->cfg.hbm_budget_bytes)
     return fail(A3D_ERR_NOMEM, "serving: session does not fit in the HBM budget");
-  if (hipMalloc(&se.state, 7 * n * 4) != hipSuccess || hipMalloc(&se.scratch, scratch_floats((uint32_t)n) * 4) != hipSuccess ||
-      hipMalloc(&se.inmap, n) != hipSuccess || hipMalloc(&se.mean, 64) != hipSuccess ||
-      hipMalloc(&se.ord, order_stride((uint32_t)n)) != hipSuccess) {
+  if (dev_malloc(&se.state, 7 * n * 4) != hipSuccess || dev_malloc(&se.scratch, scratch_floats((uint32_t)n) * 4) != hipSuccess ||
+      dev_malloc(&se.inmap, n) != hipSuccess || dev_malloc(&se.mean, 64) != hipSuccess ||
+      dev_malloc(&se.ord, order_stride((uint32_t)n)) != hipSuccess) {
     (void)hipFree(se.state);
     (void)hipFree(se.scratch);
     (void)hipFree(se.inmap);
@@ -474,7 +474,7 @@ int a3d_server_create(const a3d_server_config* cfg, a3d_server** out) {
   for (auto& s : S->slots) {
     ok = ok && hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking) == hipSuccess &&
          hipEventCreateWithFlags(&s.done, hipEventDisableTiming) == hipSuccess &&
-         hipMalloc(&s.d_counter, 64) == hipSuccess && hipMalloc(&s.d_u01, 4 * 4096) == hipSuccess;
+         dev_malloc(&s.d_counter, 64) == hipSuccess && dev_malloc(&s.d_u01, 4 * 4096) == hipSuccess;
   }
   if (!ok) {
     a3d_server_destroy(S);
@@ -521,7 +521,7 @@ int a3d_server_add_map(a3d_server* S, const a3d_grid* g, int* map_id) {
   if (!S || !g || !map_id) return fail(A3D_ERR_ARG, "a3d_server_add_map: null argument");
   std::lock_guard<std::mutex> lk(S->mu);
   GridDev* d = nullptr;
-  if (hipMalloc(&d, sizeof(GridDev)) != hipSuccess) return fail(A3D_ERR_NOMEM, "a3d_server_add_map: allocation");
+  if (dev_malloc(&d, sizeof(GridDev)) != hipSuccess) return fail(A3D_ERR_NOMEM, "a3d_server_add_map: allocation");
   if (hipMemcpy(d, &g->g, sizeof(GridDev), hipMemcpyHostToDevice) != hipSuccess) {
     (void)hipFree(d);
     return fail(A3D_ERR_HIP, "a3d_server_add_map: copy");
@@ -547,7 +547,7 @@ int a3d_server_open_session(a3d_server* S, int map_id, int num_particles, const 
   // ParticleFilter::init with the session's step-0 draws
   float* z4 = nullptr;
   uint64_t* ss = nullptr;
-  if (hipMalloc(&z4, 4 * (size_t)se.n * 4) != hipSuccess || hipMalloc(&ss, 16) != hipSuccess) {
+  if (dev_malloc(&z4, 4 * (size_t)se.n * 4) != hipSuccess || dev_malloc(&ss, 16) != hipSuccess) {
     (void)hipFree(z4);
     free_session(S, se);
     return fail(A3D_ERR_NOMEM, "a3d_server_open_session: init staging");
