@@ -274,8 +274,8 @@ __global__ __launch_bounds__(kKT) void order_scatter_kernel(OrderJob j) {
 // particles: the
 // fields stay in registers between the passes, the histogram in LDS, and a
 // particle's rank inside its key comes from the LDS add that counts it.  The
-// moments are float sums of the differences to particle 0 (they only place the
-// levels).  Bound by the latency of its dependent phases: 7 us for 1,000
+// moments are sums in 64 bits, as in the four kernels, of the differences to
+// particle 0.  Bound by the latency of its dependent phases: 7 us for 1,000
 // particles and 16 us for 5,000, where the four kernels take 20 and 22 us and
 // three more launches.  Batches keep the four: a workgroup of 16 wavefronts
 // waits for a whole free CU beside the other batches' weight kernels (48
@@ -284,7 +284,7 @@ template <int K>
 __global__ __launch_bounds__(kBT) void order_one_kernel(FilterDev f, OrderDev o) {
   constexpr int kWaves = kBT / 64, kPer = kOrderKeys / kBT;
   __shared__ uint32_t h[kOrderKeys];
-  __shared__ float red[8][kWaves];
+  __shared__ double red[8][kWaves];
   __shared__ OrderLevels lv;
   __shared__ uint32_t tot[kWaves];
   const uint32_t tid = threadIdx.x, n = f.n;
@@ -303,29 +303,43 @@ __global__ __launch_bounds__(kBT) void order_one_kernel(FilterDev f, OrderDev o)
   for (int k = 0; k < 4; ++k) origin[k] = arr[k][0];
 #pragma unroll
   for (int k = 0; k < kPer; ++k) h[k * kBT + tid] = 0u;
-  float s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  double s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
   for (int u = 0; u < K; ++u) {
     if (tid + (uint32_t)u * kBT >= n) break;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const float d0 = v[u][k] - origin[k], d = isfinite(d0) ? d0 : 0.0f;
+      const float d0 = v[u][k] - origin[k];
+      const double d = isfinite(d0) ? (double)d0 : 0.0;
       s[k] += d;
       s[4 + k] += d * d;
     }
   }
+  // lanes 8 k .. 8 k + 7 end with the wavefront's sum k: each step halves the sums
+  // a lane carries (10 exchanges instead of 48)
+  double t;
+  {
+    double a[4], b[2];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    s[k] = wave_sum(s[k]);
-    if (lane == 0) red[k][wave] = s[k];
+    for (int k = 0; k < 4; ++k)
+      a[k] = ((lane & 32) ? s[4 + k] : s[k]) + __shfl_xor((lane & 32) ? s[k] : s[4 + k], 32);
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      b[k] = ((lane & 16) ? a[2 + k] : a[k]) + __shfl_xor((lane & 16) ? a[k] : a[2 + k], 16);
+    t = ((lane & 8) ? b[1] : b[0]) + __shfl_xor((lane & 8) ? b[0] : b[1], 8);
+    for (int d = 4; d >= 1; d >>= 1) t += __shfl_xor(t, d);
   }
+  if ((lane & 7) == 0) red[lane >> 3][wave] = t;
   __syncthreads();
   if (wave == 0) {
+    static_assert(kWaves == 16, "two wavefronts' sums per lane");
+    t = red[lane >> 3][lane & 7] + red[lane >> 3][8 + (lane & 7)];
+    for (int d = 4; d >= 1; d >>= 1) t += __shfl_xor(t, d);
     double s1[4], s2[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      s1[k] = (double)wave_sum(lane < kWaves ? red[k][lane] : 0.0f);
-      s2[k] = (double)wave_sum(lane < kWaves ? red[4 + k][lane] : 0.0f);
+      s1[k] = readlane_d(t, 8 * k);
+      s2[k] = readlane_d(t, 8 * (k + 4));
     }
     order_levels(s1, s2, n, &lv);
   }
