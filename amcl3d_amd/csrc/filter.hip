@@ -1046,66 +1046,8 @@ __device__ __forceinline__ void subtile_map(float r, uint32_t& d0, uint32_t& d1,
   pp = (uint32_t)__builtin_amdgcn_readlane((int)(f.p0 | (f.p1 << 1)), 63);
 }
 
-// One wavefront adds the nq sub-tiles of a chunk to s in order; the running
-// sum after each goes to prefix[0 .. nq) (when given).
-template <class Lds>
-__device__ float chunk_walk(float s, uint32_t nq, int k, float* prefix, const Lds& L) {
-  const uint32_t lane = lane_id();
-  for (uint32_t q = 0; q < nq;) {
-    const uint32_t Q = q + lane;
-    const bool have = Q < nq;
-    const uint32_t fe = have ? L.fe[k][Q] : 0u, fl = fe & 0xffu;
-    if (s == 0.0f) {  // +0 plus sub-tiles of zeros stays +0
-      const uint32_t Z = first_false(have && !(fl & (kPos | kNeg | kIrregularTerm)));
-      if (prefix && lane < Z) prefix[Q] = 0.0f;
-      q += Z;
-      if (q == nq) break;
-    } else if (normal_finite(s)) {
-      const int E = float_exponent(fabsf(s)), e = (int)(fe >> 12) - 256;
-      const bool use_a = e == E && !(fl & kNoMapA), use_b = e + 1 == E && !(fl & kNoMapB);
-      const bool sign_ok = (s > 0.0f) ? !(fl & kNeg) : !(fl & kPos);
-      const uint32_t d0 = have ? (use_a ? L.d0a[k][Q] : L.d0b[k][Q]) : 0u;
-      const uint32_t d1 = have ? (use_a ? L.d1a[k][Q] : L.d1b[k][Q]) : 0u;
-      const uint32_t pp = use_a ? fe >> 8 : fe >> 10;
-      const bool valid = have && (use_a || use_b) && sign_ok && d0 < (1u << 24) && d1 < (1u << 24);
-      if (__ballot(valid) & 1ull) {
-        uint32_t kb, ka;
-        const uint32_t C = run_maps(s, E, ParityFn{d0, d1, pp & 1u, (pp >> 1) & 1u}, valid, kb, ka);
-        if (C > 0) {
-          const bool neg = s < 0.0f;
-          if (prefix && lane < C) prefix[Q] = from_k(ka, E, neg);
-          s = from_k((uint32_t)__builtin_amdgcn_readlane((int)ka, C - 1), E, neg);
-          q += C;
-          if (q == nq) break;
-          if (C == 64) continue;
-        }
-      }
-    }
-    // sub-tile q, which no map covers, by the reference's float adds: every
-    // lane reads the same terms (broadcasts); the zeros past the end leave
-    // the sum, never -0.0, unchanged
-    const float4* x = reinterpret_cast<const float4*>(L.x[k] + q * 64);
-    float4 v[16];
-#pragma unroll
-    for (int c = 0; c < 16; ++c) v[c] = x[c];
-#pragma unroll
-    for (int c = 0; c < 16; ++c) {
-      s += v[c].x;
-      s += v[c].y;
-      s += v[c].z;
-      s += v[c].w;
-    }
-    if (prefix && lane == 0) prefix[q] = s;
-    ++q;
-  }
-  return s;
-}
-
-// A sum of up to kSerialSubs sub-tiles is added term by term: it crosses a
-// binade every few sub-tiles, 64 adds take no longer than a scan of their maps,
-// and no maps are needed (updates of 600, 1,000 and 1,500 particles 34, 36 and
-// 44 us with maps, 25, 30 and 40 us without).
-constexpr uint32_t kSerialSubs = 32;
+// s + nq sub-tiles of terms in order, the running sum after each in prefix (when
+// given); every lane reads the same terms (broadcasts).
 __device__ __forceinline__ float chunk_serial(float s, uint32_t nq, const float* terms, float* prefix) {
   const float4* const x = reinterpret_cast<const float4*>(terms);
   float4 a[8], b[8];  // half a sub-tile is read while the other is added
@@ -1132,6 +1074,76 @@ __device__ __forceinline__ float chunk_serial(float s, uint32_t nq, const float*
   }
   return s;
 }
+
+// One wavefront adds the nq sub-tiles of a chunk to s in order; the running
+// sum after each goes to prefix[0 .. nq) (when given).
+template <class Lds>
+__device__ float chunk_walk(float s, uint32_t nq, int k, float* prefix, const Lds& L) {
+  const uint32_t lane = lane_id();
+  for (uint32_t q = 0; q < nq;) {
+    const uint32_t Q = q + lane;
+    const bool have = Q < nq;
+    const uint32_t fe = have ? L.fe[k][Q] : 0u, fl = fe & 0xffu, q0 = q;
+    if (s == 0.0f) {  // +0 plus sub-tiles of zeros stays +0
+      const uint32_t Z = first_false(have && !(fl & (kPos | kNeg | kIrregularTerm)));
+      if (prefix && lane < Z) prefix[Q] = 0.0f;
+      q += Z;
+      if (q == nq) break;
+    } else if (normal_finite(s)) {
+      const int E = float_exponent(fabsf(s)), e = (int)(fe >> 12) - 256;
+      const bool use_a = e == E && !(fl & kNoMapA), use_b = e + 1 == E && !(fl & kNoMapB);
+      const bool sign_ok = (s > 0.0f) ? !(fl & kNeg) : !(fl & kPos);
+      const uint32_t d0 = have ? (use_a ? L.d0a[k][Q] : L.d0b[k][Q]) : 0u;
+      const uint32_t d1 = have ? (use_a ? L.d1a[k][Q] : L.d1b[k][Q]) : 0u;
+      const uint32_t pp = use_a ? fe >> 8 : fe >> 10;
+      const bool valid = have && (use_a || use_b) && sign_ok && d0 < (1u << 24) && d1 < (1u << 24);
+      if (__ballot(valid) & 1ull) {
+        uint32_t kb, ka;
+        const uint32_t C = run_maps(s, E, ParityFn{d0, d1, pp & 1u, (pp >> 1) & 1u}, valid, kb, ka);
+        if (C > 0) {
+          const bool neg = s < 0.0f;
+          if (prefix && lane < C) prefix[Q] = from_k(ka, E, neg);
+          s = from_k((uint32_t)__builtin_amdgcn_readlane((int)ka, C - 1), E, neg);
+          q += C;
+          if (q == nq) break;
+          if (C == 64) continue;
+        }
+      }
+    }
+    // sub-tile q, which no map covers, and those after it with terms of both signs,
+    // which none can, by the reference's float adds; the zeros past the end leave
+    // the sum, never -0.0, unchanged
+    // (trying their maps one sub-tile at a time 20,000 terms took 163 us, now 104)
+    const uint64_t mixed = __ballot((fl & (kPos | kNeg)) == (kPos | kNeg));
+    const uint32_t done = q - q0;
+    const uint32_t run = done < 64 ? 1u + (uint32_t)__builtin_ctzll(~(mixed >> done >> 1)) : 1u;
+    if (run > 1) {
+      s = chunk_serial(s, run, L.x[k] + q * 64, prefix ? prefix + q : nullptr);
+      q += run;
+      continue;
+    }
+    const float4* x = reinterpret_cast<const float4*>(L.x[k] + q * 64);
+    float4 v[16];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) v[c] = x[c];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+      s += v[c].x;
+      s += v[c].y;
+      s += v[c].z;
+      s += v[c].w;
+    }
+    if (prefix && lane == 0) prefix[q] = s;
+    ++q;
+  }
+  return s;
+}
+
+// A sum of up to kSerialSubs sub-tiles is added term by term: it crosses a
+// binade every few sub-tiles, 64 adds take no longer than a scan of their maps,
+// and no maps are needed (updates of 600, 1,000 and 1,500 particles 34, 36 and
+// 44 us with maps, 25, 30 and 40 us without).
+constexpr uint32_t kSerialSubs = 32;
 
 // s[k] + the chunk's len terms of sum k in order, for every k, in every thread.
 // xv[k][u]: this thread's term u * kChainThreads + tid of sum k (0 past len).
