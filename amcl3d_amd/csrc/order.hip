@@ -17,10 +17,11 @@
 // poses apart in x rarely are, and a yaw apart moves a point by its range.
 // Each bit goes to the coordinate with the largest remaining deviation in
 // weights kSep.  Against one bit each in turn (x, y, z, yaw), the weight
-// kernel measured (1000 x 1000 x 200 map, 20,011 particles within 0.5 m and
-// 0.15 rad, 7,993 points, tilted) 350 instead of 435 us, 120 instead of 140 us
-// (8,000 within 1 m, 4,001 points); on the 2000 x 2000 x 600 map 520 instead
-// of 640 us (20,000 within 1 m, 10,000 points) and 1,918 instead of 1,940 us
+// kernel of cells in floating point measured (1000 x 1000 x 200 map, 20,011
+// particles within 0.5 m and 0.15 rad, 7,993 points, tilted) 350 instead of 435
+// us, 120 instead of 140 us (8,000 within 1 m, 4,001 points); on the 2000 x 2000 x
+// 600 map 520 instead of 640 us (20,000 within 1 m, 10,000 points) and 1,918
+// instead of 1,940 us
 // (100,000 within 0.1 m, 20,000 points).  Weights of half or twice kSep are
 // within 3% of it.  A set spread over several metres (global localisation) has
 // no two particles on one line; its key orders by region alone (z, y, x in

@@ -490,11 +490,11 @@ __device__ __forceinline__ double fma3(double a, double s, double c) {
 }
 
 // kFixed: the cell's index (any where the point is outside the map), vm, and
-// near, the least fraction of the three axes
-// (below fx_near: cell_redo decides).  24 vector instructions per 64
-// evaluations, its share of the rotation, the sum and the loop included, where
-// kClean takes 34: per axis the offset add, two conversions, the product and
-// the truncation become one multiply-add.
+// near, the least fraction of the three axes (below fx_near: cell_redo decides).
+// Per axis the offset add, two conversions, the product and the truncation
+// become one multiply-add: 25.9 vector instructions per 64 evaluations, with the
+// rotation, the sum, the loop and the redone lanes (24 without those), where
+// kClean takes 34.7.
 template <bool RP0, int IK>
 __device__ __forceinline__ typename ProbSrc<IK>::Idx cell_fixed(const GridDev& g, const LanePose& lp, const float4& p,
                                                                    uint64_t& vm, uint32_t& near) {
@@ -519,11 +519,12 @@ __device__ __forceinline__ typename ProbSrc<IK>::Idx keep_in_map(const ProbSrc<I
 }
 
 // A group of kFixed cells: where every lane of every step is in the map (most
-// groups of a tracking filter inside a building) the selects and the counts, an
-// eighth of the loop, are left out and the group is counted once in full
-// (100,000 x 8,000 on the 1000 x 1000 x 200 map: 640 -> 612 us; in the split
-// form, 4 wavefronts per SIMD, the branch cost more than it left out: 256 ->
-// 369 us for 20,011 x 7,993).
+// groups of a tracking filter inside a building) the selects and the counts are
+// left out and the group is counted once in full.  It gains where issue bounds
+// the kernel (100,000 x 20,000 on the 2000 x 2000 x 600 map: update 1,563 -> 1,555
+// us), not where gathers do (100,000 x 8,000 on the 1000 x 1000 x 200 map: 544 ->
+// 563 us).  In the split form, 4 wavefronts per SIMD, the branch costs more than
+// it leaves out (20,011 x 7,993: 327 -> 471 us), and it is not used there.
 template <int U, int IK>
 __device__ __forceinline__ void group_in_map(const ProbSrc<IK>& src, const uint64_t (&vm)[U],
                                              typename ProbSrc<IK>::Idx (&idx)[U], int& cnt, int& full) {
