@@ -1006,6 +1006,7 @@ struct ChunkLds {
   // a sub-tile's maps (SubRec's fields; fe = flags | pp << 8 | (e + 256) << 12)
   uint32_t d0a[NS][kSubs], d1a[NS][kSubs], d0b[NS][kSubs], d1b[NS][kSubs], fe[NS][kSubs];
   float s[NS];
+  uint32_t mixed[NS];  // some sub-tile of the chunk has terms of both signs
 };
 
 // The map of one sub-tile (a wavefront's terms) from the scaled magnitudes r =
@@ -1076,14 +1077,16 @@ __device__ __forceinline__ float chunk_serial(float s, uint32_t nq, const float*
 }
 
 // One wavefront adds the nq sub-tiles of a chunk to s in order; the running
-// sum after each goes to prefix[0 .. nq) (when given).
-template <class Lds>
+// sum after each goes to prefix[0 .. nq) (when given).  MIXED: some sub-tile has
+// terms of both signs.  (Its code in every sum's walk cost the others 4%.)
+template <bool MIXED, class Lds>
 __device__ float chunk_walk(float s, uint32_t nq, int k, float* prefix, const Lds& L) {
   const uint32_t lane = lane_id();
   for (uint32_t q = 0; q < nq;) {
     const uint32_t Q = q + lane;
     const bool have = Q < nq;
-    const uint32_t fe = have ? L.fe[k][Q] : 0u, fl = fe & 0xffu, q0 = q;
+    const uint32_t fe = have ? L.fe[k][Q] : 0u, fl = fe & 0xffu;
+    [[maybe_unused]] const uint32_t q0 = q;
     if (s == 0.0f) {  // +0 plus sub-tiles of zeros stays +0
       const uint32_t Z = first_false(have && !(fl & (kPos | kNeg | kIrregularTerm)));
       if (prefix && lane < Z) prefix[Q] = 0.0f;
@@ -1110,31 +1113,30 @@ __device__ float chunk_walk(float s, uint32_t nq, int k, float* prefix, const Ld
         }
       }
     }
-    // sub-tile q, which no map covers, and those after it with terms of both signs,
-    // which none can, by the reference's float adds; the zeros past the end leave
-    // the sum, never -0.0, unchanged
-    // (trying their maps one sub-tile at a time 20,000 terms took 163 us, now 104)
-    const uint64_t mixed = __ballot((fl & (kPos | kNeg)) == (kPos | kNeg));
-    const uint32_t done = q - q0;
-    const uint32_t run = done < 64 ? 1u + (uint32_t)__builtin_ctzll(~(mixed >> done >> 1)) : 1u;
-    if (run > 1) {
-      s = chunk_serial(s, run, L.x[k] + q * 64, prefix ? prefix + q : nullptr);
-      q += run;
-      continue;
+    // sub-tile q, which no map covers, by the reference's float adds: every
+    // lane reads the same terms (broadcasts); the zeros past the end leave
+    // the sum, never -0.0, unchanged.  With it those after it that have terms of
+    // both signs, and so no map (a scan for each: 20,000 such terms 163 us, now 89)
+    uint32_t run = 1;
+    if constexpr (MIXED) {
+      const uint64_t mixed = __ballot((fl & (kPos | kNeg)) == (kPos | kNeg));
+      if (q - q0 < 64) run += (uint32_t)__builtin_ctzll(~(mixed >> (q - q0) >> 1));
     }
-    const float4* x = reinterpret_cast<const float4*>(L.x[k] + q * 64);
-    float4 v[16];
+    do {
+      const float4* x = reinterpret_cast<const float4*>(L.x[k] + q * 64);
+      float4 v[16];
 #pragma unroll
-    for (int c = 0; c < 16; ++c) v[c] = x[c];
+      for (int c = 0; c < 16; ++c) v[c] = x[c];
 #pragma unroll
-    for (int c = 0; c < 16; ++c) {
-      s += v[c].x;
-      s += v[c].y;
-      s += v[c].z;
-      s += v[c].w;
-    }
-    if (prefix && lane == 0) prefix[q] = s;
-    ++q;
+      for (int c = 0; c < 16; ++c) {
+        s += v[c].x;
+        s += v[c].y;
+        s += v[c].z;
+        s += v[c].w;
+      }
+      if (prefix && lane == 0) prefix[q] = s;
+      ++q;
+    } while (MIXED && --run);
   }
   return s;
 }
@@ -1168,6 +1170,7 @@ __device__ __forceinline__ void chunk_sums(float (&s)[NS], const float (&xv)[NS]
       if (lane == 0) L.part[k][q] = w;
     }
   }
+  if (!serial && tid < (uint32_t)NS) L.mixed[tid] = 0u;
   __syncthreads();
   if (!serial) {
 #pragma unroll
@@ -1206,6 +1209,7 @@ __device__ __forceinline__ void chunk_sums(float (&s)[NS], const float (&xv)[NS]
         L.d0b[k][q] = d0b;
         L.d1b[k][q] = d1b;
         L.fe[k][q] = fl | (ppa << 8) | (ppb << 10) | ((uint32_t)(e + 256) << 12);
+        if ((fl & (kPos | kNeg)) == (kPos | kNeg)) L.mixed[k] = 1u;
       }
     }
   }
@@ -1215,7 +1219,13 @@ __device__ __forceinline__ void chunk_sums(float (&s)[NS], const float (&xv)[NS]
   for (int k = 0; k < NS; ++k) {
     if (wave == (uint32_t)k) {
       float* const pre = k == NS - 1 ? prefix : nullptr;
-      const float v = serial ? (nq ? chunk_serial(s[k], nq, L.x[k], pre) : s[k]) : chunk_walk(s[k], nq, k, pre, L);
+      float v = s[k];
+      if (serial) {
+        if (nq) v = chunk_serial(s[k], nq, L.x[k], pre);
+      } else {
+        const bool mixed = __builtin_amdgcn_readfirstlane((int)L.mixed[k]) != 0;
+        v = mixed ? chunk_walk<true>(s[k], nq, k, pre, L) : chunk_walk<false>(s[k], nq, k, pre, L);
+      }
       if (lane == 0) L.s[k] = v;
     }
   }
