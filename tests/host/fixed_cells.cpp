@@ -4,8 +4,8 @@
 // uniform ones, under offsets of many poses.  Reads lines of
 //   nx ny nz  res  minx miny minz  cut  draws  seed
 // (max lies `cut` cells below the last face) and prints for each
-//   fixed  near-fraction-bound  judged  wrong  outside-near
-// (judged: evaluations away from the faces; outside-near: lanes that would be
+//   fixed  near-fraction-bound  compared  wrong  outside-near
+// (compared: evaluations away from the faces; outside-near: lanes that would be
 // redone for the point that stands for padding and non-finite points)
 #include <cmath>
 #include <cstdio>
@@ -55,7 +55,7 @@ int main() {
     for (int a = 0; a < 3; ++a) mx[a] = m[a] + ((double)size[a] - cut) * res;
     a3d::GridDev g{};
     a3d::grid_meta(m, mx, res, g);
-    long judged = 0, wrong = 0;
+    long compared = 0, wrong = 0;
     std::mt19937_64 rng(seed);
     std::uniform_real_distribution<double> u01(0.0, 1.0);
     for (long d = 0; g.fixed && d < draws; ++d) {
@@ -77,7 +77,7 @@ int main() {
       }
       Cell f{}, r = reference(g, a, s, o);
       if (!fixed(g, a, s, o, f)) continue;
-      ++judged;
+      ++compared;
       wrong += f.in != r.in || (r.in && f.i != r.i);
     }
     long outside = 0;
@@ -90,7 +90,7 @@ int main() {
         outside += !fixed(g, a, s[a], o, f) || f.in;
       }
     }
-    std::printf("%u %.9g %ld %ld %ld\n", g.fixed, std::ldexp((double)g.fx_near, -32), judged, wrong, outside);
+    std::printf("%u %.9g %ld %ld %ld\n", g.fixed, std::ldexp((double)g.fx_near, -32), compared, wrong, outside);
   }
   return 0;
 }

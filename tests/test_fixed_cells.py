@@ -13,21 +13,21 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 @pytest.fixture(scope="session")
-def checker(tmp_path_factory):
+def compare(tmp_path_factory):
     lib = os.path.dirname(os.path.abspath(_lib.LIB_PATH))
     exe = str(tmp_path_factory.mktemp("host") / "fixed_cells")
     subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
                     "-o", exe, os.path.join(ROOT, "tests", "host", "fixed_cells.cpp"), "-L" + lib, "-lamcl3d_gpu",
                     "-Wl,-rpath," + lib, "-L/opt/rocm/lib", "-Wl,-rpath-link,/opt/rocm/lib"], check=True)
 
-    def check(grids):
+    def run(grids):
         text = "".join("%d %d %d %.17g %.17g %.17g %.17g %.17g %d %d\n" % g for g in grids)
         out = subprocess.run([exe], input=text, capture_output=True, text=True, check=True, timeout=300).stdout
         rows = [line.split() for line in out.splitlines()]
         assert len(rows) == len(grids)
         return [(int(f), float(near), int(j), int(w), int(o)) for f, near, j, w, o in rows]
 
-    return check
+    return run
 
 
 # units per cell, cells per axis, min
@@ -43,16 +43,16 @@ CELLS = [(0.05, (900, 40, 70), (-17.35, 3.1, -0.4)), (0.05, (2000, 2000, 600), (
 
 
 @pytest.mark.parametrize("part", range(3))
-def test_cells_match_the_reference(checker, part):
+def test_cells_match_the_reference(compare, part):
     grids = [n + (res,) + mn + (0.0, 3_000_000, 11 + part) for res, n, mn in CELLS[part::3]]
-    for g, (fixed, near, judged, wrong, _) in zip(grids, checker(grids)):
-        assert wrong == 0, (g, near, judged, wrong)
+    for g, (fixed, near, compared, wrong, _) in zip(grids, compare(grids)):
+        assert wrong == 0, (g, near, compared, wrong)
         if fixed:
-            assert judged > 300_000, (g, judged)  # a third of the draws are away from the faces
+            assert compared > 300_000, (g, compared)  # a third of the draws are away from the faces
             assert near <= 2.0 ** -11 * 1.01
 
 
-def test_random_extents(checker):
+def test_random_extents(compare):
     """Whole-cell maps of any extent: the bound of the map, a float, is a face only to within its rounding."""
     rng = np.random.default_rng(5)
     grids = []
@@ -61,11 +61,11 @@ def test_random_extents(checker):
         n = tuple(int(v) for v in rng.integers(20, 1200, 3))
         mn = tuple(float(v) for v in np.round(rng.uniform(-50, 50, 3), 2))
         grids.append(n + (res,) + mn + (0.0, 100_000, k))
-    for g, (fixed, near, judged, wrong, _) in zip(grids, checker(grids)):
-        assert wrong == 0, (g, near, judged, wrong)
+    for g, (fixed, near, compared, wrong, _) in zip(grids, compare(grids)):
+        assert wrong == 0, (g, near, compared, wrong)
 
 
-def test_which_grids_are_fixed(checker):
+def test_which_grids_are_fixed(compare):
     """The mode of the grids the GPU tests weight on: a rule that turned the
     form off everywhere, or on for a grid outside it, would show here."""
     want = {((200, 180, 60), 0.1, (0.0, 0.0, 0.0), 0.0): 1, ((900, 40, 70), 0.05, (-17.35, 3.1, -0.4), 0.0): 1,
@@ -76,15 +76,15 @@ def test_which_grids_are_fixed(checker):
             ((9000, 8, 9), 0.05, (-100.0, 0.0, 0.0), 0.0): 0, ((4000, 9, 8), 1000.0, (0.0, 0.0, 0.0), 0.0): 0,
             ((120, 80, 30), 0.1, (0.0, 0.0, 0.0), 0.5): 0, ((150, 90, 40), 0.07, (0.0, -2.0, 0.0), 0.0): 0}
     grids = [n + (res,) + mn + (cut, 1000, 1) for n, res, mn, cut in want]
-    got = [r[0] for r in checker(grids)]
+    got = [r[0] for r in compare(grids)]
     assert dict(zip(want, got)) == want
 
 
-def test_outside_points_are_not_redone(checker):
+def test_outside_points_are_not_redone(compare):
     """The point staged for padding and for non-finite points: out of the map
     and away from every face under any pose, so that no lane repeats it."""
     grids = [n + (res,) + mn + (0.0, 1000, 2) for res, n, mn in CELLS]
-    rows = checker(grids)
+    rows = compare(grids)
     assert sum(r[0] for r in rows) > len(rows) // 2
-    for g, (fixed, near, judged, wrong, outside) in zip(grids, rows):
+    for g, (fixed, near, compared, wrong, outside) in zip(grids, rows):
         assert outside == 0, (g, outside)
